@@ -1280,14 +1280,15 @@ extern "C" NCTensor *nc_relpos_attention_step(NCTensor *q, NCTensor *kv_cache, N
 // ---- LSTM layer (nc_ext.h; kernels and the reasons for their split in k_lstm.hip) --------------
 // Saved for the backward pass: the normalised gate sums (rows, N), 1/rms (n_gate, N), the states c_0 .. c_T
 // (C, N + B) and h_0 .. h_T, the packed biases and gains, and u.
+constexpr int LSTM_MAX_GATES = 4;
 extern "C" NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCTensor **b, int n_gate, int type,
                                    float eps, NCTensor *h, NCTensor *c)
 {
     NCContext *m = nc_ctx(pre);
-    if (!pre->dev->is_hip || m->matmul_bf16 || m->matmul_invariant || (n_gate != 3 && n_gate != 4) || h->n_dims != 2) return nullptr;
+    if (!pre->dev->is_hip || m->matmul_bf16 || m->matmul_invariant || (n_gate != 3 && n_gate != LSTM_MAX_GATES) || h->n_dims != 2) return nullptr;
     const size_t C = h->dims[0], B = h->dims[1], rows = C * n_gate;
     if (C < 1 || B < 1 || C > K_LSTM_MAX_UNITS || h->node || c->node) return nullptr;
-    NCTensor *all[11] = { pre, u, h, c };
+    NCTensor *all[4 + 2 * LSTM_MAX_GATES] = { pre, u, h, c }; // then each gate's bias and gain
     int count = 4;
     for (int j = 0; j < n_gate; j++) {
         all[count++] = b[j];
@@ -1304,7 +1305,7 @@ extern "C" NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCT
     const size_t zd[2] = { rows, N }, rd[2] = { (size_t)n_gate, N }, sd[2] = { C, N + B }, gd[1] = { rows + n_gate };
     NCTensor *z = new_f32(pre, 2, zd), *rstd = new_f32(pre, 2, rd), *hs = new_f32(pre, 2, sd), *cs = new_f32(pre, 2, sd), *gb = new_f32(pre, 1, gd);
     KLstmParams pp;
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < LSTM_MAX_GATES; j++) {
         pp.b[j] = j < n_gate ? nc_f32(b[j]) : nullptr;
         pp.g[j] = j < n_gate && g ? nc_f32(g[j]) : nullptr;
     }
@@ -1330,7 +1331,7 @@ extern "C" NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCT
         k_lstm_cell(m->stream, &a, n_gate, (int)B, 1);
     }
     m->launches += 1 + 2 * (int64_t)T;
-    NCTensor *args[10] = { pre, u };
+    NCTensor *args[2 + 2 * LSTM_MAX_GATES] = { pre, u };
     const int n_args = 2 + (g ? 2 : 1) * n_gate;
     for (int j = 0; j < n_gate; j++) {
         args[2 + j] = b[j];
@@ -1381,7 +1382,7 @@ static void lstm_layer_bw(NCNode *nd, NCTensor *g, NCTensor **ga)
     }
     KLstmGrads pg;
     const size_t one[1] = { C };
-    for (int j = 0; j < 4; j++) {
+    for (int j = 0; j < LSTM_MAX_GATES; j++) {
         pg.db[j] = pg.dg[j] = nullptr;
         if (j >= n_gate) continue;
         ga[2 + j] = new_f32(g, 1, one);

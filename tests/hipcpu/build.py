@@ -18,7 +18,9 @@ SOURCES = ["k_gemm.hip", "k_elementwise.hip", "k_norm.hip", "k_lstm.hip", "k_att
            "nc_core.cpp", "nc_autodiff.cpp", "nc_ops.cpp", "nc_params_io.cpp"]
 NO_CONTRACT = {"k_cdf.hip", "nc_ops.cpp"}
 FLAGS = ["-x", "c++", "-std=c++17", "-O1", "-g", "-fPIC", "-fno-strict-aliasing", "-Wno-unknown-attributes",
-         "-Wno-unused-function", "-Wno-unused-value", "-Wno-array-bounds", "-I", HERE, "-iquote", CSRC]
+         "-Wno-unused-function", "-Wno-unused-value", "-Wno-array-bounds", "-I", HERE, "-iquote", CSRC,
+         # host stack arrays have no guard page: an index outside one ends the process here
+         "-fsanitize=array-bounds", "-fsanitize-trap=array-bounds"]
 # the dynamic LDS array of a kernel becomes a pointer to the launch's guarded buffer
 DYN_LDS = re.compile(r"extern\s+__shared__\s+__attribute__\(\(aligned\(16\)\)\)\s+(\w+)\s+(\w+)\[\];")
 # occupancy hints mean nothing to the host compiler (and it rejects them on plain functions)

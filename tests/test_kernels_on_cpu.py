@@ -2,7 +2,8 @@
 against a stand-in HIP runtime: work-items are fibers, wavefront shuffles and
 the three MFMA instructions follow their documented lane layouts, and device
 memory and dynamic LDS end at guard pages, so an out-of-range access is a
-SIGSEGV at the faulting statement.  The GPU parity tests are then re-run
+SIGSEGV at the faulting statement; an index outside an array ends the process too
+(-fsanitize=array-bounds, trapping).  The GPU parity tests are then re-run
 against that build: same kernel sources, same checks, on the CPU.  (The
 float results of libm's tanhf / expf differ in the last bit from the GPU's,
 which is why one tolerance-marginal model case is left to the GPU run.)"""
@@ -52,8 +53,9 @@ def test_gpu_parity_tests_pass_on_the_cpu_build(emulated):
     256 keys, integer CDF and lookup bit-exactness, optimiser, ...) and a
     model-level subset (training steps against the checker op by op and fused,
     whole-model gradient, cached per-timestep logits bit-identical, a profile
-    variant, the retrain pass, the LSTM model class and a file through the container), with
-    guard pages behind every device buffer."""
+    variant, the retrain pass, the LSTM model class and a file through the container), and
+    the kernels at the edges of their tiles and ranges, with guard pages behind every
+    device buffer and checked indices into the host's arrays."""
     ops = _pytest(emulated, ["-n", "4", "tests/test_gpu_ops.py", "-k", OPS_LEFT_TO_THE_GPU])
     model = _pytest(emulated, ["-n", "2", "tests/test_gpu_model.py", "-k",
                                "(test_training_steps_match_checker and TINY) or "
@@ -66,20 +68,23 @@ def test_gpu_parity_tests_pass_on_the_cpu_build(emulated):
                              "not (file_container and (reference or bf16)) and not full_size and "
                              "not (properties_small and bf16) and not 100_steps and not enwik8_profile and "
                              "not (memory_window and 0)"])
+    edges = _pytest(emulated, ["-n", "3", "tests/test_gpu_kernel_edges.py"])
     out_ops, out_model = ops.communicate(timeout=1500)[0], model.communicate(timeout=1500)[0]
-    out_new = new.communicate(timeout=1500)[0]
+    out_new, out_edges = new.communicate(timeout=1500)[0], edges.communicate(timeout=1500)[0]
     assert ops.returncode == 0, out_ops[-3000:]
     assert model.returncode == 0, out_model[-3000:]
     assert new.returncode == 0, out_new[-3000:]
+    assert edges.returncode == 0 and " passed" in out_edges, out_edges[-3000:]
     assert " passed" in out_ops and " passed" in out_model and " passed" in out_new and "skipped" not in out_new
 
 
 def test_results_do_not_depend_on_work_item_order(emulated):
-    """The op-level tests again with the work-items of every workgroup, and the workgroups of
+    """The op-level and edge tests again with the work-items of every workgroup, and the workgroups of
     every launch, run from the last to the first (HIPCPU_ORDER=reverse).  Between two
     barriers any order is one the hardware may pick, so a kernel that is missing a barrier
     (or whose workgroups rely on one another) gives different results here."""
-    p = _pytest(dict(emulated, HIPCPU_ORDER="reverse"), ["-n", "7", "tests/test_gpu_ops.py", "-k", OPS_LEFT_TO_THE_GPU])
+    p = _pytest(dict(emulated, HIPCPU_ORDER="reverse"), ["-n", "7", "tests/test_gpu_ops.py",
+                                                           "tests/test_gpu_kernel_edges.py", "-k", OPS_LEFT_TO_THE_GPU])
     out = p.communicate(timeout=1500)[0]
     assert p.returncode == 0 and " passed" in out, out[-3000:]
 
