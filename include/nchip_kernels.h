@@ -26,9 +26,6 @@ extern "C" {
    depend on m or n (64x64 tiles, two interleaved k chains, no split-K), so a
    column computed alone is bit-identical to the same column of a wide product */
 #define NCHIP_GEMM_WIDTH_INVARIANT 0x100
-/* precision flag: keep the small-product kernel out, so that with ksplit 1 every output element is
-   one chain over k whatever m and n are */
-#define NCHIP_GEMM_SEQUENTIAL 0x200
 
 /* C = act(alpha * op(A) * op(B) + beta * C + bias), batched.
    Replaces nc_matmul / nc_matmul_add (libnc.h:365-373, call sites
@@ -39,11 +36,13 @@ extern "C" {
    (nearest-even) on load, fp32 accumulation on the bf16 MFMA units.
    ksplit > 1 splits the reduction over that many workgroups whose partial
    tiles are summed in a fixed order by a second kernel; it needs
-   `workspace` of at least batch*ksplit*m*n floats.  Unless the product goes to
-   the small-product kernel (nchip_gemm_is_small, whose wavefronts split k), every
-   output element is a sequential MFMA accumulation chain over k = 0..K-1 that
-   does not depend on m, n or the tile shape; with NCHIP_GEMM_WIDTH_INVARIANT it
-   always is. */
+   `workspace` of at least batch*ksplit*m*n floats (NULL will do where
+   nchip_gemm_is_small and no rows are skipped: lda, ldb tight).  The tile class
+   is chosen from m, n, batch and ksplit;
+   inside a class every output element is a fixed sequence of MFMA
+   accumulations over k = 0..K-1 (the 64x64 class: two interleaved chains, added),
+   whatever m, n, the number of columns and the kernel that issues it.  With
+   NCHIP_GEMM_WIDTH_INVARIANT the class does not depend on the shape either. */
 int nchip_gemm(void *stream, int ta, int tb, int m, int n, int k, float alpha,
                const float *A, int64_t lda, int64_t stride_a,
                const float *B, int64_t ldb, int64_t stride_b,
@@ -232,8 +231,8 @@ void nchip_gemm_bf16_source(int mode);
 
 /* Chooses ksplit for nchip_gemm from the shape alone (never from data). */
 int nchip_gemm_pick_ksplit(int m, int n, int k, int batch);
-/* 1 when an unforced fp32 product of this shape (no activation gradient) is one launch of the
-   small-product kernel, whatever ksplit says */
+/* 1 when an fp32 product of this shape without an activation gradient, at the ksplit chosen
+   above, is one launch of the small-product kernel (the 64x64 class's sums) and takes no workspace */
 int nchip_gemm_is_small(int m, int n, int k, int batch);
 
 /* Relative-position causal attention, forward (nncp.c:722-800 fused).

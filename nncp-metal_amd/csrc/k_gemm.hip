@@ -10,7 +10,8 @@
 // Tile classes (chosen from the shape only): 128x128x32 with 8 wavefronts, 128x64x32 with 8
 // wavefronts, 64x64x32 with two k groups of 4 wavefronts (KW = 2: the groups split every
 // 32-deep slab, C = chain0 + chain1).  Inside a class a C element is a fixed sequence of MFMA
-// accumulations that does not depend on m, n or the number of columns.  The width-invariant
+// accumulations that does not depend on m, n or the number of columns; products with few tiles
+// of the 64x64 class go to gemm_small_kernel, which issues the same sums.  The width-invariant
 // class (NCHIP_GEMM_WIDTH_INVARIANT: 64x64x32, KW = 2, two accumulator sets per group = four
 // chains per element, no split-K) is used by encoder and decoder alike when a column computed
 // alone must equal the same column computed inside a larger matrix (bit-exact decode);
@@ -35,6 +36,7 @@
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4_u __attribute__((ext_vector_type(4), aligned(4)));
 typedef short shortx8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4))); // a first-class value, unlike the uint4 struct
 
@@ -1327,65 +1329,145 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
 #endif
 }
 
-// Small fp32 products: a 16 x 16 tile of C per workgroup and batch entry, its NW wavefronts
-// splitting the reduction in chunks of 16 k.  Each holds the operands of up to PF chunks in
-// registers, so one memory round trip covers K = 16 NW PF, and issues
-// v_mfma_f32_16x16x4_f32 straight from them (step s of a chunk takes k = 4 (lane / 16) + s on
-// both sides); the partial tiles meet in LDS and are summed in wavefront order.  No operand is
-// shared between tiles, which is what the tile kernel's LDS stages are for: when the output has
-// fewer 64 x 64 tiles than a chip fills, those stages are a serial chain of round trips instead:
-// 256 x 16 x 512 took 18.2 us through them and takes under 4.9 here.
-// (va / vb: the k-contiguous operand's columns may be read 16 bytes at a time)
-template <int NW, int PF, int TA, int TB>
-__global__ __launch_bounds__(64 * NW) void gemm_small_kernel(GemmArgs g, int va, int vb)
+// Small fp32 products: a 16 x 16 tile of C per workgroup and batch entry, with the bits of the
+// 64x64x32 class (KW = 2) that the shape would otherwise take.  That class gives every element
+// two chains per k chunk - chain 0 the first 16 k of each 32-deep slab, chain 1 the rest - and
+// with split-K adds the chunks' (chain 0 + chain 1) in order; a wavefront here is one such chain,
+// issued as v_mfma_f32_16x16x4_f32, which accumulates its four k in increasing order like the
+// 32x32x2 form its two.  No operand is shared between tiles, which is what the tile kernel's LDS
+// stages are for: when the output has fewer 64 x 64 tiles than a chip fills, those stages are a
+// serial chain of memory round trips; here a wavefront holds PF blocks of 16 k of both operands in
+// registers, so that one round trip covers K = 32 PF (per chunk, with SPLIT: 2 g.ksplit chains,
+// NW of them at a time).
+// VA / VB: the operand is contiguous along k (K at least 4), and a lane reads four k at once, at any
+// 4-byte alignment.  It then holds k = 4 (lane / 16) + s where the matrix instruction wants
+// k = 4 s + lane / 16: transpose_k4 exchanges the four 16-lane rows, four swaps for 16 k.
+__device__ __forceinline__ void transpose_k4(floatx4 &v)
 {
-    static_assert(NW >= 4, "a thread per element of the tile");
-    __shared__ float red[NW][256];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, il = lane & 15, kq = lane >> 4;
+    uint32_t r[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) r[s] = __float_as_uint(v[s]);
+#pragma unroll
+    for (int s = 0; s < 2; s++) { // upper 32 lanes of r[s] against lower 32 of r[s + 2]
+        const auto x = __builtin_amdgcn_permlane32_swap(r[s], r[s + 2], false, false);
+        r[s] = x[0]; r[s + 2] = x[1];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s += 2) { // odd 16-lane rows of r[s] against even ones of r[s + 1]
+        const auto x = __builtin_amdgcn_permlane16_swap(r[s], r[s + 1], false, false);
+        r[s] = x[0]; r[s + 1] = x[1];
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++) v[s] = __uint_as_float(r[s]);
+}
+
+constexpr int SMALL_KSPLIT = 16; // nchip_gemm_pick_ksplit's limit
+
+template <int NW, int PF, int VA, int VB, int SPLIT>
+__global__ __launch_bounds__(64 * NW) void gemm_small_kernel(GemmArgs g, int64_t am, int64_t ak, int64_t bn, int64_t bk)
+{
+    __shared__ float red[SPLIT ? 2 * SMALL_KSPLIT : 2][256];
+    // (w in a scalar register: the branches around the matrix instructions, which ignore the
+    // execution mask, have to be scalar ones)
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), il = lane & 15, kq = lane >> 4;
     const int m0 = blockIdx.x * 16, n0 = blockIdx.y * 16, bo = blockIdx.z / g.batch_in, bi = blockIdx.z % g.batch_in;
-    const int m = m0 + il < g.M ? m0 + il : g.M - 1, n = n0 + il < g.N ? n0 + il : g.N - 1;
-    const float NCHIP_GLOBAL *Am = as_global(g.A) + bo * g.sa + bi * g.sa_in + (TA ? (int64_t)m * g.lda : (int64_t)m);
-    const float NCHIP_GLOBAL *Bn = as_global(g.B) + bo * g.sb + bi * g.sb_in + (TB ? (int64_t)n : (int64_t)n * g.ldb);
-    const int K = g.K, nch = (K + 15) / 16;
-    floatx4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
-    for (int q0 = w; q0 < nch; q0 += NW * PF) {
-        floatx4 a[PF], b[PF];
-#pragma unroll
-        for (int p = 0; p < PF; p++) {
-            const int k = (q0 + p * NW) * 16 + 4 * kq;
-            if (!TB && vb && k < K) {
-                b[p] = *reinterpret_cast<const floatx4 NCHIP_GLOBAL *>(Bn + k);
+    // (am, ak / bn, bk: strides of A along m and k, of B along n and k; byte offsets from the tile's
+    // first row fit 32 bits, so an address is a scalar base and one register)
+    const char NCHIP_GLOBAL *A0 = (const char NCHIP_GLOBAL *)(as_global(g.A) + bo * g.sa + bi * g.sa_in + m0 * am);
+    const char NCHIP_GLOBAL *B0 = (const char NCHIP_GLOBAL *)(as_global(g.B) + bo * g.sb + bi * g.sb_in + n0 * bn);
+    const uint32_t ma = 4 * (uint32_t)(m0 + il < g.M ? il : g.M - 1 - m0) * (uint32_t)am, ka = 4 * (uint32_t)ak;
+    const uint32_t nb = 4 * (uint32_t)(n0 + il < g.N ? il : g.N - 1 - n0) * (uint32_t)bn, kb = 4 * (uint32_t)bk;
+    const int K = g.K, chains = SPLIT ? 2 * g.ksplit : 2;
+    // 16 k from k0 on.  A block that passes the end reads clamped addresses, so that every block
+    // issues the same loads; keep() clears what lies past it
+    const uint32_t aoff = ma + (VA ? 16 : ka) * kq, boff = nb + (VB ? 16 : kb) * kq; // this lane's first k of a block
+    auto fetch = [&](floatx4 &v, const char NCHIP_GLOBAL *p, uint32_t row, uint32_t off, uint32_t step, int k0, auto vec) {
+        constexpr bool V = decltype(vec)::value;
+        if (k0 + 16 <= K) { // uniform
+            const char NCHIP_GLOBAL *q = p + (V ? 4 : step) * (uint32_t)k0;
+            if constexpr (V) {
+                v = *reinterpret_cast<const floatx4_u NCHIP_GLOBAL *>(q + off);
             } else {
 #pragma unroll
-                for (int s = 0; s < 4; s++) b[p][s] = k + s < K ? (TB ? Bn[(int64_t)(k + s) * g.ldb] : Bn[k + s]) : 0.0f;
+                for (int s = 0; s < 4; s++) v[s] = *reinterpret_cast<const float NCHIP_GLOBAL *>(q + s * 4 * step + off);
             }
-            if (TA && va && k < K) {
-                a[p] = *reinterpret_cast<const floatx4 NCHIP_GLOBAL *>(Am + k);
-            } else {
+        } else if constexpr (V) {
+            const int k = k0 + 4 * kq;
+            v = *reinterpret_cast<const floatx4_u NCHIP_GLOBAL *>(p + (row + 4 * (uint32_t)(k < K - 4 ? k : K - 4)));
+        } else {
 #pragma unroll
-                for (int s = 0; s < 4; s++) a[p][s] = k + s < K ? (TA ? Am[k + s] : Am[(int64_t)(k + s) * g.lda]) : 0.0f;
+            for (int s = 0; s < 4; s++) {
+                const int k = k0 + 4 * s + kq;
+                v[s] = *reinterpret_cast<const float NCHIP_GLOBAL *>(p + (row + step * (uint32_t)(k < K ? k : K - 1)));
+            }
+        }
+    };
+    auto keep = [&](floatx4 &v, int k0, int kend, auto vec) {
+        if constexpr (decltype(vec)::value) {
+            if (k0 + 16 > kend) { // v was read from K - 4 where four k from k on pass the end: d of them are to go
+                const int k = k0 + 4 * kq, d = k < K - 4 ? 0 : k - (K - 4);
+                v = d & 1 ? floatx4{ v[1], v[2], v[3], 0.0f } : v;
+                v = d & 2 ? floatx4{ v[2], v[3], 0.0f, 0.0f } : v;
+                v = d > 3 ? floatx4{ 0.0f, 0.0f, 0.0f, 0.0f } : v;
+            }
+            transpose_k4(v);
+        } else if (k0 + 16 > kend) {
+#pragma unroll
+            for (int s = 0; s < 4; s++) v[s] = k0 + 4 * s + kq < kend ? v[s] : 0.0f;
+        }
+    };
+    // this thread's elements of the tile, and what the epilogue reads for them: fetched before the
+    // operands, it costs no round trip of its own at the end
+    constexpr int NE = NW >= 4 ? 1 : 4 / NW;
+    bool ok[NE];
+    int64_t off[NE];
+    float extra[NE], prev[NE], bv[NE];
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        const int e = threadIdx.x + i * 64 * NW, tm = m0 + (e & 15), tn = n0 + (e >> 4);
+        ok[i] = e < 256 && tm < g.M && tn < g.N;
+        off[i] = bo * g.sc + bi * g.sc_in + (int64_t)tn * g.ldc + tm;
+        extra[i] = g.add && ok[i] ? as_global(g.add)[off[i]] : 0.0f;
+        prev[i] = g.beta != 0.0f && ok[i] ? as_global(g.C)[off[i]] : 0.0f;
+        bv[i] = g.bias && ok[i] ? as_global(g.bias)[tm] : 0.0f;
+    }
+    for (int c = w; c < chains; c += NW) {
+        const int kbeg = (c >> 1) * g.kchunk, kend = kbeg + g.kchunk < K ? kbeg + g.kchunk : K;
+        floatx4 acc = { 0.0f, 0.0f, 0.0f, 0.0f };
+        for (int k0 = kbeg + 16 * (c & 1); k0 < kend; k0 += 32 * PF) {
+            floatx4 a[PF], b[PF];
+#pragma unroll
+            for (int p = 0; p < PF; p++) {
+                fetch(b[p], B0, nb, boff, kb, k0 + 32 * p, std::integral_constant<bool, VB>());
+                fetch(a[p], A0, ma, aoff, ka, k0 + 32 * p, std::integral_constant<bool, VA>());
+            }
+            __builtin_amdgcn_sched_barrier(0); // every load is out before the first is waited for
+#pragma unroll
+            for (int p = 0; p < PF; p++) {
+                if (k0 + 32 * p >= kend) break; // uniform
+                keep(b[p], k0 + 32 * p, kend, std::integral_constant<bool, VB>());
+                keep(a[p], k0 + 32 * p, kend, std::integral_constant<bool, VA>());
+#pragma unroll
+                for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[p][s], a[p][s], acc, 0, 0, 0);
             }
         }
 #pragma unroll
-        for (int p = 0; p < PF; p++)
-#pragma unroll
-            for (int s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(b[p][s], a[p][s], acc, 0, 0, 0);
+        for (int r = 0; r < 4; r++) red[c][(4 * kq + r) * 16 + il] = acc[r]; // [n][m]
     }
-#pragma unroll
-    for (int r = 0; r < 4; r++) red[w][(4 * kq + r) * 16 + il] = acc[r]; // [n][m]
     __syncthreads();
-    const int t = threadIdx.x, tm = m0 + (t & 15), tn = n0 + (t >> 4);
-    if (t >= 256 || tm >= g.M || tn >= g.N) return;
-    float sum = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NW; j++) sum += red[j][t];
-    const int64_t off = bo * g.sc + bi * g.sc_in + (int64_t)tn * g.ldc + tm;
-    const float extra = g.add ? as_global(g.add)[off] : 0.0f;
-    float v = g.alpha * sum;
-    if (g.beta != 0.0f) v += g.beta * as_global(g.C)[off];
-    if (g.bias) v += as_global(g.bias)[tm];
-    if (g.pre) as_global(g.pre)[off] = v;
-    as_global(g.C)[off] = apply_act(v, g.act) + extra;
+    for (int i = 0; i < NE; i++) {
+        if (!ok[i]) continue;
+        const int e = threadIdx.x + i * 64 * NW;
+        float sum = red[0][e] + red[1][e];
+        if (SPLIT)
+            for (int z = 1; z < g.ksplit; z++) sum += red[2 * z][e] + red[2 * z + 1][e];
+        float v = g.alpha * sum;
+        if (g.beta != 0.0f) v += g.beta * prev[i];
+        v += bv[i];
+        if (g.pre) as_global(g.pre)[off[i]] = v;
+        as_global(g.C)[off[i]] = apply_act(v, g.act) + extra[i];
+    }
 }
 
 // sums the ksplit partial tiles in increasing k order, then the same epilogue
@@ -1555,25 +1637,20 @@ void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec)
 #undef LAUNCH
 }
 
-// whether the columns of a k-contiguous operand may be read 16 bytes at a time
-bool small_vec(const float *p, int k, int64_t ld, int64_t s_out, int64_t s_in)
-{
-    return k % 4 == 0 && ld % 4 == 0 && s_out % 4 == 0 && s_in % 4 == 0 && ((uintptr_t)p & 15) == 0;
-}
-
-template <int NW, int PF>
+template <int NW, int PF, int SPLIT>
 void launch_small(hipStream_t st, int ta, int tb, const GemmArgs &g, ProfRec *rec)
 {
     const dim3 grid((g.M + 15) / 16, (g.N + 15) / 16, g.batch), block(64 * NW);
-    const int va = small_vec(g.A, g.K, g.lda, g.sa, g.sa_in), vb = small_vec(g.B, g.K, g.ldb, g.sb, g.sb_in);
-#define LAUNCH(TA, TB)                                                                                     \
+    const bool va = ta && g.K >= 4, vb = !tb && g.K >= 4;
+    const int64_t am = ta ? g.lda : 1, ak = ta ? 1 : g.lda, bn = tb ? 1 : g.ldb, bk = tb ? g.ldb : 1;
+#define LAUNCH(VA, VB)                                                                                     \
     do {                                                                                                   \
-        if (rec) hipExtLaunchKernelGGL((gemm_small_kernel<NW, PF, TA, TB>), grid, block, 0, st, rec->start, rec->stop, 0, g, va, vb); \
-        else hipLaunchKernelGGL((gemm_small_kernel<NW, PF, TA, TB>), grid, block, 0, st, g, va, vb);       \
+        if (rec) hipExtLaunchKernelGGL((gemm_small_kernel<NW, PF, VA, VB, SPLIT>), grid, block, 0, st, rec->start, rec->stop, 0, g, am, ak, bn, bk); \
+        else hipLaunchKernelGGL((gemm_small_kernel<NW, PF, VA, VB, SPLIT>), grid, block, 0, st, g, am, ak, bn, bk); \
     } while (0)
-    if (!ta && !tb) LAUNCH(0, 0);
-    else if (ta && !tb) LAUNCH(1, 0);
-    else if (!ta && tb) LAUNCH(0, 1);
+    if (!va && !vb) LAUNCH(0, 0);
+    else if (va && !vb) LAUNCH(1, 0);
+    else if (!va && vb) LAUNCH(0, 1);
     else LAUNCH(1, 1);
 #undef LAUNCH
 }
@@ -1645,18 +1722,41 @@ extern "C" int nchip_gemm_pick_ksplit(int m, int n, int k, int batch)
     return s < 1 ? 1 : s;
 }
 
-// Whether an fp32 product goes to the 16 x 16 tiles of gemm_small_kernel.  They read each operand
-// once per 16 rows or columns, at the 10 TB/s that the caches deliver: 128 bytes per tile and k,
-// 10 us at the limit below, which is what the 64 x 64 class needs for the barriers of 400 k.
-// Measured, 64 x 64 class -> this, us: 256 x 16 x 512 18.2 -> 4.9, 512 x 256 x 16 5.0 -> 4.9 (both
-// at the rate of their issue), 352 x 481 x 352 15.8 -> 7.0, 512 x 83 x 2048 (split over k) 14.9 -> 8.3,
-// 512 x 512 x 512 13.4 -> 8.9; past it 512 x 1024 x 512 13.7 -> 15.1, 512 x 512 x 2048 20.6 -> 25.7.
-// One workgroup walks the whole reduction of its tile at 3.5 us per 1024 k, where the 64 x 64 class
-// spreads it over up to 16: 64 x 64 x 2048 13.3 -> 9.6, x 4096 15.4 -> 16.7, x 16384 28.7 -> 58.1.
-extern "C" int nchip_gemm_is_small(int m, int n, int k, int batch)
+// Tile class of an fp32 or bf16-rounding product (nb: batch entries times split-K chunks), from the
+// shape alone.  Measured on MI355X (fp32): small outputs want the most workgroups and the most
+// wavefronts per workgroup (10: 64x64x32, two k groups of 4 wavefronts, four register sets of
+// tiles in flight); once 128x64 tiles still give >= 256 workgroups, 8 wavefronts of 32x32 on a
+// 128x64x32 tile win (4); very large problems use 128x128x32 with 8 wavefronts (7).
+static int gemm_class(int m, int n, int64_t nb)
+{
+    const int64_t tm = (m + 127) / 128;
+    if (tm * ((n + 127) / 128) * nb >= 512 && m >= 128 && n >= 128) return 7;
+    if (tm * ((n + 63) / 64) * nb >= 256 && m >= 128 && n >= 64) return 4;
+    return 10;
+}
+
+// Whether an fp32 product of the 64x64 class is issued by gemm_small_kernel (the same sums; this is
+// about time only).  That kernel reads each operand once per 16 rows or columns, 128 bytes per tile
+// and k from the caches, where the 64x64 class waits for a memory round trip per 32 or 64 k.
+// Measured under a kernel trace, 64x64 class -> this, us (A and B plain / A transposed / B transposed):
+//   256 x 16 x 512      18.2 / 17.8 / 19.0 -> 5.6 / 5.8 / 5.9     128 x 80 x 128   7.3 / 7.1 / 7.8 -> 4.1 / 3.6 / 3.6
+//   352 x 481 x 352     15.8 / 14.9 / 17.0 -> 7.7 / 8.2 / 7.6     352 x 481 x 777 32.8 / 34.1 / 31.8 -> 11.9 / 12.3 / 13.0
+//   512 x 512 x 512     13.7 / 13.2 / 14.1 -> 9.3 / 11.4 / 8.9    512 x 512 x 1000 24.4 / 23.8 / 24.7 -> 14.1 / 18.3 / 14.9
+//   512 x 576 x 777     29.1 / 34.4 / 19.9 -> 15.9 / 18.4 / 21.0  640 x 512 x 640 16.3 / 15.8 / 16.7 -> 16.2 / 21.2 / 20.5
+//   512 x 768 x 256      9.2 / 8.7 / 9.4 -> 8.2 / 9.4 / 8.2       512 x 768 x 512 13.9 / 13.5 / 14.4 -> 12.0 / 15.4 / 15.4
+//   512 of 32 x 32 x 64 10.2 / 10.3 / 10.9 -> 5.0 / 5.5 / 5.2     512 x 1024 x 192 9.3 / 9.0 / 9.5 -> 8.9 / 10.2 / 8.6
+// and split over k, where one workgroup walks all chunks of its tile and no second launch adds them:
+//   512 x 83 x 2048     16.0 / 15.6 / 17.2 -> 9.4 / 10.5 / 9.2    512 x 192 x 2048 16.1 / 15.5 / 16.6 -> 15.6 / 18.6 / 15.8
+//   64 x 64 x 3072      15.1 / 15.9 / 15.3 -> 11.2 / 13.4 / 10.2  512 x 256 x 1500 16.9 / 16.7 / 17.2 -> 17.4 / 17.8 / 18.8
+static bool gemm_is_small(int m, int n, int k, int batch, int ksplit)
 {
     const int64_t tiles = (int64_t)((m + 15) / 16) * ((n + 15) / 16) * batch;
-    return k <= 3072 && tiles <= 2048 && tiles * k <= 3 << 18;
+    return tiles <= 2048 && (k < 1024 ? tiles <= 1152 || tiles * k <= 3 << 17 : k <= 3072 && tiles * k <= 3 << 18) && gemm_class(m, n, (int64_t)batch * ksplit) == 10;
+}
+
+extern "C" int nchip_gemm_is_small(int m, int n, int k, int batch)
+{
+    return !g_force_cfg && gemm_is_small(m, n, k, batch, nchip_gemm_pick_ksplit(m, n, k, batch));
 }
 
 static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float alpha,
@@ -1676,10 +1776,12 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
                 m, n, k, (long)lda, (long)ldb, (long)ldc);
         return -1;
     }
-    const bool invariant = (precision & NCHIP_GEMM_WIDTH_INVARIANT) != 0, sequential = (precision & NCHIP_GEMM_SEQUENTIAL) != 0;
+    const bool invariant = (precision & NCHIP_GEMM_WIDTH_INVARIANT) != 0;
     precision &= 0xff;
     if (ksplit < 1 || invariant) ksplit = 1;
-    if (ksplit > 1 && !workspace) {
+    const bool small_fits = precision == 0 && !dpre && ksplit <= SMALL_KSPLIT && (k + 16) * (lda > ldb ? lda : ldb) < 1 << 29; // (32-bit byte offsets)
+    const bool small = !invariant && !g_force_cfg && small_fits && gemm_is_small(m, n, k, batch, ksplit);
+    if (ksplit > 1 && !workspace && !small) {
         fprintf(stderr, "nchip_gemm: ksplit=%d needs a workspace\n", ksplit);
         return -1;
     }
@@ -1738,24 +1840,9 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
         }
         return 0;
     }
-    // Tile configuration from the shape alone.  Measured on MI355X (fp32):
-    // small outputs want the most workgroups and the most wavefronts per
-    // workgroup (64x64x32, two k groups of 4 wavefronts); once
-    // 128x64 tiles still give >= 256 workgroups, 8 wavefronts of 32x32 on a
-    // 128x64x32 tile win; very large problems use 128x128x32 with 8 wavefronts.
     int cfg = invariant ? 30 : g_force_cfg; // tuning aid: 0 = choose from the shape
-    if (!cfg && precision == 0 && !dpre && !sequential && nchip_gemm_is_small(m, n, k, batch)) {
-        cfg = 40;
-        g.ksplit = ksplit = 1; // (its workgroups split the reduction themselves)
-    }
-    if (cfg == 40 && (precision != 0 || dpre || ksplit > 1 || batch > 65535)) cfg = 10;
-    int64_t nb = (int64_t)batch * ksplit;
-    int64_t t128x64 = (int64_t)((m + 127) / 128) * ((n + 63) / 64) * nb;
-    if (!cfg) {
-        if (t128 >= 512 && m >= 128 && n >= 128) cfg = 7;
-        else if (t128x64 >= 256 && m >= 128 && n >= 64) cfg = 4;
-        else cfg = 10; // 64x64x32, two k groups, four register sets of tiles in flight
-    }
+    if (cfg == 40 && !small_fits) cfg = 10;
+    if (!cfg) cfg = small ? 40 : gemm_class(m, n, (int64_t)batch * ksplit);
     // Large bf16 products are bound by operand traffic from L2, not by the MFMA
     // rate: round both operands to bf16 in memory first (one streaming pass
     // each) and let the tiles load half the bytes.  The rounded values are
@@ -1800,10 +1887,15 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
         else if (cfg == 9) launch_tile<64, 64, 64, 2, 2, 1, 2>(st, ta, tb, g, pr);
         else launch_tile<64, 64, 32, 2, 2, 1, 2>(st, ta, tb, g, pr);
     } else if (cfg == 40) {
-        // (one round trip covers 64, 256 and 512 k; a round trip's worth of k more costs about 1 us)
-        if (k <= 64) launch_small<4, 1>(st, ta, tb, g, pr);
-        else if (k <= 256) launch_small<4, 4>(st, ta, tb, g, pr);
-        else launch_small<16, 2>(st, ta, tb, g, pr);
+        // (wavefronts: the two chains, or as many of the 2 ksplit; blocks in flight: one round trip's)
+        if (ksplit > 4) launch_small<16, 8, 1>(st, ta, tb, g, pr);
+        else if (ksplit > 1) launch_small<8, 8, 1>(st, ta, tb, g, pr);
+        else if (k <= 32) launch_small<2, 1, 0>(st, ta, tb, g, pr);
+        else if (k <= 64) launch_small<2, 2, 0>(st, ta, tb, g, pr);
+        else if (k <= 128) launch_small<2, 4, 0>(st, ta, tb, g, pr);
+        else if (k <= 256) launch_small<2, 8, 0>(st, ta, tb, g, pr);
+        else if (k <= 384) launch_small<2, 12, 0>(st, ta, tb, g, pr);
+        else launch_small<2, 16, 0>(st, ta, tb, g, pr);
     } else if (cfg == 1) {
         launch_tile<128, 128, 16, 2, 2, 0>(st, ta, tb, g, pr);
     } else if (cfg == 2) {
@@ -1832,7 +1924,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
         rec.variant = tile * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 1 ? 1 : 0);
         g_prof.push_back(rec);
     }
-    if (ksplit > 1) {
+    if (ksplit > 1 && cfg != 40) {
         int64_t total = (int64_t)m * n;
         int nb = (int)((total + 255) / 256);
         if (nb > 2048) nb = 2048;

@@ -681,15 +681,11 @@ static void dev_gemm(NCContext *m, bool ta, bool tb, size_t M, size_t N, size_t 
         dev_gemm_bf16_operands(m, ta, tb, M, N, K, alpha, a, b, c, bias, act, pre, addend, want_c16))
         return;
     nc_shadow_invalidate(c);
-    // a forward product's columns have the same bits alone and in a wide matrix (a replayed step
-    // reads them) as long as its reduction is not split; the small-product kernel splits it
-    const bool sequential = forward && K < 1024;
-    const int prec = m->matmul_bf16 | (invariant ? NCHIP_GEMM_WIDTH_INVARIANT : 0) | (sequential ? NCHIP_GEMM_SEQUENTIAL : 0);
-    const bool small = prec == 0 && nchip_gemm_is_small((int)M, (int)N, (int)K, (int)batch);
-    int ks = invariant || small ? 1 : nchip_gemm_pick_ksplit((int)M, (int)N, (int)K, (int)batch);
+    const int prec = m->matmul_bf16 | (invariant ? NCHIP_GEMM_WIDTH_INVARIANT : 0);
+    const int ks = invariant ? 1 : nchip_gemm_pick_ksplit((int)M, (int)N, (int)K, (int)batch);
     size_t cap = 0;
     float *ws = nullptr;
-    if (ks > 1) ws = nc_tmp_f32(m, batch * ks * M * N, &cap);
+    if (ks > 1 && (prec != 0 || !nchip_gemm_is_small((int)M, (int)N, (int)K, (int)batch))) ws = nc_tmp_f32(m, batch * ks * M * N, &cap);
     int rc;
     // a few columns against a weight matrix with a k-major copy: the same chains from the copy
     const float *a_data = nc_f32(a);
@@ -714,7 +710,7 @@ static void dev_gemm(NCContext *m, bool ta, bool tb, size_t M, size_t N, size_t 
                         bias, act, pre, prec, ks, ws);
     if (ws) nc_tmp_free(m, ws, cap);
     if (rc) nc_fatal("gemm failed (m=%zu n=%zu k=%zu)", M, N, K);
-    m->launches += ks > 1 ? 2 : 1;
+    m->launches += ws ? 2 : 1;
 }
 
 // libnc.h:365-373

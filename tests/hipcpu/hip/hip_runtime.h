@@ -204,6 +204,23 @@ template <typename T> static inline T __shfl_down(T v, unsigned d, int width = 6
     return hipcpu_shfl_from(v, s < base + width ? s : lane);
 }
 
+/* v_permlane{32,16}_swap_b32: the odd rows of 32 (16) lanes of the first operand change places
+   with the even rows of the second */
+struct hipcpu_u2 { unsigned v[2]; unsigned operator[](int i) const { return v[i]; } };
+template <int ROW>
+static inline hipcpu_u2 hipcpu_permlane_swap(unsigned a, unsigned b)
+{
+    uint32_t w[2] = { a, b };
+    const uint32_t *tab = hipcpu_wave_exchange(w, 2);
+    const int l = hipcpu_cur->lane, odd = l & ROW;
+    const hipcpu_u2 r = { { odd ? tab[(l ^ ROW) * 16 + 1] : a, odd ? b : tab[(l ^ ROW) * 16] } };
+    hipcpu_wave_barrier();
+    return r;
+}
+#define __builtin_amdgcn_readfirstlane(x) (x) /* used on values that are uniform in the wavefront */
+#define __builtin_amdgcn_permlane32_swap(a, b, fi, bc) hipcpu_permlane_swap<32>(a, b)
+#define __builtin_amdgcn_permlane16_swap(a, b, fi, bc) hipcpu_permlane_swap<16>(a, b)
+
 /* ---- MFMA (lane layouts of the CDNA3/4 ISA guide) ------------------------------------ */
 typedef float hipcpu_f16v __attribute__((ext_vector_type(16)));
 typedef float hipcpu_f4v __attribute__((ext_vector_type(4)));

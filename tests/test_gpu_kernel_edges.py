@@ -1,5 +1,7 @@
 """Kernels at the sizes where they can go wrong - tile edges, remainders, the smallest and
 largest of a range - against the CPU checker or a float64 statement."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -105,6 +107,74 @@ def test_small_products(hip, m, n, k, batch, ta, tb):
     want = 0.5 * (a @ b) + add
     bound = 2.0 ** -24 * ((k + 2) * 0.5 * (np.abs(a) @ np.abs(b)) + 2 * np.abs(add) + np.abs(want))
     assert np.all(np.abs(np.swapaxes(got, 1, 2) - want) <= bound)
+
+
+def _small_products(hip, m, n, k, batch, ta, tb, pads, options):
+    """[small kernel, 64x64 class] results of the products; options: alpha, beta, act, bias, addend"""
+    lib = C.CDLL(hip.lib._name)
+    rng = np.random.default_rng(m + 7 * n + k)
+    st, ci, i64, f32 = C.c_void_p(hip.nc_context_stream(hip.ctx)), C.c_int, C.c_int64, C.c_float
+    ks = lib.nchip_gemm_pick_ksplit(ci(m), ci(n), ci(k), ci(batch))
+    assert lib.nchip_gemm_is_small(ci(m), ci(n), ci(k), ci(batch)) == 1
+    (ra, ca), (rb, cb) = (k, m) if ta else (m, k), (n, k) if tb else (k, n)
+    tensors = []
+
+    def dev(x):
+        tensors.append(hip.tensor(x.astype(np.float32)))
+        return C.c_void_p(hip.nc_tensor_get_ptr(tensors[-1], None))
+
+    bias, ws = dev(rng.standard_normal(m)), dev(np.zeros(batch * ks * m * n))
+    try:
+        for pad in pads:
+            A, B = dev(rng.standard_normal((batch, ca, ra + pad))), dev(rng.standard_normal((batch, cb, rb + pad)))
+            add, c0 = rng.standard_normal((2, batch, n, m + pad))
+            addp = dev(add)
+            for alpha, beta, act, with_bias, with_add in options:
+                got = []
+                for cfg in (0, 10):
+                    lib.nchip_gemm_force_config(cfg)
+                    out, pre = dev(c0), dev(np.zeros_like(c0))
+                    head = [st, ci(ta), ci(tb), ci(m), ci(n), ci(k), f32(alpha), A, i64(ra + pad), i64(ca * (ra + pad)),
+                            B, i64(rb + pad), i64(cb * (rb + pad))]
+                    tail = [ci(0), ci(ks), ws]
+                    if with_add:
+                        rc = lib.nchip_gemm_add(*head, out, i64(m + pad), i64(n * (m + pad)), ci(batch), bias if with_bias else None,
+                                                ci(act), pre, addp, *tail)
+                    else:
+                        rc = lib.nchip_gemm(*head, f32(beta), out, i64(m + pad), i64(n * (m + pad)), ci(batch),
+                                            bias if with_bias else None, ci(act), pre, *tail)
+                    assert rc == 0
+                    got.append([hip.numpy(t) for t in tensors[-2:]])
+                yield (k, pad, alpha, beta, act, with_bias, with_add), got
+    finally:
+        lib.nchip_gemm_force_config(0)
+        hip.free(*tensors)
+
+
+@pytest.mark.parametrize("m,n,k,batch", [(1, 1, 1, 1), (16, 16, 16, 1), (17, 15, 63, 3), (33, 7, 65, 2), (40, 20, 256, 2), (17, 33, 516, 1),
+                                         (50, 3, 777, 1), (33, 17, 1023, 1), (33, 17, 1024, 1), (16, 33, 2048, 1), (33, 5, 1500, 2),
+                                         (20, 18, 3070, 1)])
+@pytest.mark.parametrize("ta", [0, 1])
+@pytest.mark.parametrize("tb", [0, 1])
+def test_small_products_have_the_bits_of_their_tile_class(hip, m, n, k, batch, ta, tb):
+    """The kernel of 16 x 16 tiles issues the sums of the 64x64 class that the shape would otherwise
+    take, split over k or not: the same bits, with every epilogue option of an unforced product,
+    from tight columns and from padded ones."""
+    options = [(1.0, 0.0, 0, 0, 0), (0.5, 0.0, 0, 0, 1), (1.0, 0.0, 1, 1, 0), (0.5, 0.0, 2, 1, 1), (1.0, 1.0, 0, 0, 0), (0.3, 0.7, 0, 1, 0)]
+    for case, (small, tile) in list(_small_products(hip, m, n, k, batch, ta, tb, (0,), options)) + \
+            list(_small_products(hip, m, n, k, batch, ta, tb, (1, 4), options[3:4])):
+        for u, v in zip(small, tile):
+            assert np.array_equal(u, v), (case, np.abs(u - v).max())
+
+
+@pytest.mark.parametrize("ta", [0, 1])
+@pytest.mark.parametrize("tb", [0, 1])
+def test_small_products_at_every_remainder_of_k(hip, ta, tb):
+    """Every remainder of 16 and 32 k behind each number of blocks that a round trip covers (64, 128,
+    256, 384 and 512 k)."""
+    for k in [*range(1, 34), *range(61, 82), *range(125, 146, 3), *range(255, 290, 2), *range(383, 403, 3), *range(511, 530)]:
+        for case, (small, tile) in _small_products(hip, 16, 3, k, 1, ta, tb, (0,), [(1.0, 0.0, 0, 0, 0)]):
+            assert np.array_equal(small[0], tile[0]), (case, np.abs(small[0] - tile[0]).max())
 
 
 @pytest.mark.parametrize("n,h", [(1, 1), (3, 4), (5, 7), (513, 12), (2048, 96)])
