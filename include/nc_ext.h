@@ -100,8 +100,8 @@ NCTensor *nc_relpos_attention_step(NCTensor *q, NCTensor *kv_cache, NCTensor *kv
    before the segment and receive the one after it.  Result: h of every step (C, B * T).
    Gradients flow to pre, u, g and b.  Consumes pre and u and each g[j], b[j]; borrows h and c.
    Returns NULL, with nothing consumed, where the library has no such form for the arguments
-   (libnc_ref.so: always; bf16 products, width-invariant products, more than 1024 units): the
-   caller then issues the op-by-op sequence.  No counterpart in the reference. */
+   (libnc_ref.so: always; bf16 products, width-invariant products, more than 1024 units, 1048560
+   streams or 2^24 columns): the caller then issues the op-by-op sequence.  No counterpart in the reference. */
 NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCTensor **b, int n_gate, int type,
                         float eps, NCTensor *h, NCTensor *c);
 

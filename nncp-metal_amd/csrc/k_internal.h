@@ -106,6 +106,8 @@ void k_pad_bwd(hipStream_t st, const float *gy, float *gx, int64_t n_in, int64_t
 // All pointers of a step address its first column; columns of z / da / dz are rows long, of the
 // others C, of rstd ng.
 #define K_LSTM_MAX_UNITS 1024
+#define K_LSTM_MAX_COLUMNS ((size_t)1 << 24)      // B times steps
+#define K_LSTM_MAX_STREAMS ((size_t)65535 * 16)   // B: 16 of them per workgroup row, at most 65535 rows to a grid
 #define K_LSTM_SLICES 4 // of the backward product's reduction
 struct KLstmParams { const float *b[4], *g[4]; };
 struct KLstmGrads { float *db[4], *dg[4]; };

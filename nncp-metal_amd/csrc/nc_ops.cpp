@@ -1293,7 +1293,8 @@ extern "C" NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCT
     for (int i = 0; i < count; i++)
         if (all[i]->type != NC_TYPE_F32 || !nc_is_contig(all[i])) return nullptr;
     const size_t N = nc_numel(pre) / rows, T = N / B;
-    if (pre->dims[0] != rows || N != T * B || T < 1 || N > (1u << 24) || u->n_dims != 2 || u->dims[0] != rows || u->dims[1] != C ||
+    if (N > K_LSTM_MAX_COLUMNS || B > K_LSTM_MAX_STREAMS) return nullptr;
+    if (pre->dims[0] != rows || N != T * B || T < 1 || u->n_dims != 2 || u->dims[0] != rows || u->dims[1] != C ||
         nc_numel(c) != C * B)
         nc_fatal("nc_lstm_layer: shapes do not fit %zu units, %zu streams, %d gates", C, B, n_gate);
     for (int j = 0; j < n_gate; j++)

@@ -90,6 +90,19 @@ def test_lstm_layer_sizes(hosts, cells, batch, seg, variant):
     ref.close()
 
 
+@pytest.mark.parametrize("streams,steps", [(65535 * 16 + 1, 1), (1, (1 << 24) + 1)])
+def test_lstm_layer_refuses_what_its_launches_cannot_hold(hip, streams, steps):
+    """More streams than a grid has rows for, more columns than its indices are laid out for: NULL,
+    with nothing consumed or written, and the caller issues the sequence of ops."""
+    def dev(*shape):                       # (column-major sizes)
+        return hip.nc_new_tensor(hip.dev, 0, len(shape), (C.c_size_t * 8)(*shape))
+    pre, u, h, c = dev(3, streams * steps), dev(3, 1), dev(1, streams), dev(1, streams)
+    b = (C.c_void_p * 3)(*[dev(1) for _ in range(3)])
+    assert not hip.nc_lstm_layer(pre, u, None, b, 3, 2, 1e-5, h, c)
+    hip.nc_synchronize(hip.dev)
+    hip.free(pre, u, h, c, *b)
+
+
 @pytest.mark.parametrize("m,n,k,batch", [(1, 1, 1, 1), (16, 16, 16, 1), (17, 15, 63, 3), (33, 7, 64, 2), (31, 5, 65, 1), (40, 20, 256, 2),
                                          (18, 33, 257, 1), (48, 9, 512, 1), (50, 3, 777, 1), (16, 83, 2048, 1), (352, 481, 352, 1), (20, 18, 3072, 1), (20, 18, 3073, 1)])
 @pytest.mark.parametrize("ta", [0, 1])
