@@ -104,6 +104,9 @@ NCTensor *nc_relpos_attention_step(NCTensor *q, NCTensor *kv_cache, NCTensor *kv
    streams or 2^24 columns): the caller then issues the op-by-op sequence.  No counterpart in the reference. */
 NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCTensor **b, int n_gate, int type,
                         float eps, NCTensor *h, NCTensor *c);
+/* Whether nc_lstm_layer takes such a layer on this device in the modes now set, its tensors f32 and
+   contiguous: what a caller asks before it prepares the layer's input. */
+BOOL nc_lstm_layer_fits(NCDevice *d, int n_gate, size_t n_units, size_t n_streams, size_t n_steps);
 
 /* Gated GELU: for x of 2 h along axis 0 the h values gelu(x[0 .. h)) x[h .. 2h), nc_split, nc_gelu
    and nc_mul (nncp.c:943-947) in one pass each way.  Consumes x.  Returns NULL, with nothing

@@ -1277,13 +1277,20 @@ extern "C" NCTensor *nc_relpos_attention_step(NCTensor *q, NCTensor *kv_cache, N
 // Saved for the backward pass: the normalised gate sums (rows, N), 1/rms (n_gate, N), the states c_0 .. c_T
 // (C, N + B) and h_0 .. h_T, the packed biases and gains, and u.
 constexpr int LSTM_MAX_GATES = 4;
+extern "C" BOOL nc_lstm_layer_fits(NCDevice *d, int n_gate, size_t C, size_t B, size_t T)
+{
+    const NCContext *m = d->ctx;
+    return d->is_hip && !m->matmul_bf16 && !m->matmul_invariant && (n_gate == 3 || n_gate == LSTM_MAX_GATES) && C >= 1 &&
+           C <= K_LSTM_MAX_UNITS && B >= 1 && B <= K_LSTM_MAX_STREAMS && T <= K_LSTM_MAX_COLUMNS / B;
+}
+
 extern "C" NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCTensor **b, int n_gate, int type,
                                    float eps, NCTensor *h, NCTensor *c)
 {
     NCContext *m = nc_ctx(pre);
-    if (!pre->dev->is_hip || m->matmul_bf16 || m->matmul_invariant || (n_gate != 3 && n_gate != LSTM_MAX_GATES) || h->n_dims != 2) return nullptr;
+    if (h->n_dims != 2 || h->node || c->node) return nullptr;
     const size_t C = h->dims[0], B = h->dims[1], rows = C * n_gate;
-    if (C < 1 || B < 1 || C > K_LSTM_MAX_UNITS || h->node || c->node) return nullptr;
+    if (!nc_lstm_layer_fits(pre->dev, n_gate, C, B, 1)) return nullptr;
     NCTensor *all[4 + 2 * LSTM_MAX_GATES] = { pre, u, h, c }; // then each gate's bias and gain
     int count = 4;
     for (int j = 0; j < n_gate; j++) {
@@ -1293,7 +1300,7 @@ extern "C" NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCT
     for (int i = 0; i < count; i++)
         if (all[i]->type != NC_TYPE_F32 || !nc_is_contig(all[i])) return nullptr;
     const size_t N = nc_numel(pre) / rows, T = N / B;
-    if (N > K_LSTM_MAX_COLUMNS || B > K_LSTM_MAX_STREAMS) return nullptr;
+    if (!nc_lstm_layer_fits(pre->dev, n_gate, C, B, T)) return nullptr;
     if (pre->dims[0] != rows || N != T * B || T < 1 || u->n_dims != 2 || u->dims[0] != rows || u->dims[1] != C ||
         nc_numel(c) != C * B)
         nc_fatal("nc_lstm_layer: shapes do not fit %zu units, %zu streams, %d gates", C, B, n_gate);

@@ -160,14 +160,11 @@ static NCTensor *concat_add(NCTensor **tab, int n_in, int n_out)
 }
 
 /* One layer of a whole segment through nc_lstm_layer: x0 (consumed) holds the pre-activations of
-   all steps.  Leaves the state for the next segment in h0 / c0.  NULL (nothing consumed) when
-   the library or the configuration has no such form. */
+   all steps.  Leaves the state for the next segment in h0 / c0. */
 static NCTensor *layer_fused(NNCPModel *s, Cell *lc, NCTensor *x0)
 {
     const NNCPConfig *c = &s->cfg;
     NCTensor *g[MAT_MAX], *b[MAT_MAX], *y, *u;
-    if (lc->p)
-        return NULL;
     for (int j = 0; j < lc->mat_count; j++) {
         b[j] = nc_dup_tensor(lc->b[j]);
         g[j] = c->lstm_use_layer_norm ? nc_dup_tensor(lc->g[j]) : NULL;
@@ -177,25 +174,24 @@ static NCTensor *layer_fused(NNCPModel *s, Cell *lc, NCTensor *x0)
     nc_tensor_copy(lc->c0_prev, lc->c0);
     y = nc_lstm_layer(x0, u, c->lstm_use_layer_norm ? g : NULL, b, lc->mat_count,
                       c->lstm_type == NNCP_LSTM_NORMAL ? 0 : c->lstm_type == NNCP_LSTM_CLAMPED ? 1 : 2, 1e-5f, lc->h0, lc->c0);
-    if (!y) {
-        nc_free_tensor(u);
-        for (int j = 0; j < lc->mat_count; j++) {
-            nc_free_tensor(b[j]);
-            nc_free_tensor(g[j]);
-        }
-    }
+    if (!y)
+        die("nc_lstm_layer refuses a layer that nc_lstm_layer_fits accepted");
     return y;
 }
 
 /* The whole segment, every layer through nc_lstm_layer: the tensors of all steps stay in one
-   piece from the embedding to the output sum.  Returns the input of the output layer, or NULL
-   when the first layer is refused (all layers have the same form). */
+   piece from the embedding to the output sum.  Returns the input of the output layer, or NULL,
+   before anything is issued, when the library or the configuration has no such form (all layers
+   have the same). */
 static NCTensor *lstm_eval_fused(NNCPModel *s, const NCTensor *input)
 {
     const NNCPConfig *c = &s->cfg;
     struct LstmState *ls = s->lstm;
     const int L = c->n_layer, N = c->seg_len * c->batch_size;
-    NCTensor *out[NNCP_N_LAYER_MAX], *below[NNCP_N_LAYER_MAX], *tok, *t1, *y;
+    NCTensor *out[NNCP_N_LAYER_MAX], *below[NNCP_N_LAYER_MAX], *tok, *t1;
+    if (ls->cells[0].p || s->param_type != NC_TYPE_F32 ||
+        !nc_lstm_layer_fits(s->dev, ls->cells[0].mat_count, c->lstm_n_cells, c->batch_size, c->seg_len))
+        return NULL;
     tok = nc_new_tensor_from_tensor_nz(input); /* a copy that ends with its upload (trf_eval) */
     nc_tensor_copy(tok, (NCTensor *)input);
     tok = nc_reshape_1d(nc_tensor_to_device(tok, s->dev), N);
@@ -208,16 +204,9 @@ static NCTensor *lstm_eval_fused(NNCPModel *s, const NCTensor *input)
                 below[n++] = nc_dup_tensor(out[i]);
             t1 = nc_matmul_add(nc_dup_tensor(lc->w), n > 1 ? nc_vconcat(below, n) : below[0], t1, 0, 0, 1.0f);
         }
-        y = layer_fused(s, lc, t1);
-        if (!y) {
-            nc_free_tensor(t1);
-            nc_free_tensor(tok);
-            if (l != 0) die("nc_lstm_layer refuses a layer after the first");
-            return NULL;
-        }
+        out[l] = layer_fused(s, lc, t1);
         nc_free_tensor(lc->h); nc_free_tensor(lc->c);
         lc->h = lc->c = NULL; /* (the state inside a segment is the per-timestep path's) */
-        out[l] = y;
     }
     nc_free_tensor(tok);
     return concat_add(out, L, c->lstm_n_embed_out);

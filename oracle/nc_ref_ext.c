@@ -490,6 +490,12 @@ NCTensor *nc_lstm_layer(NCTensor *pre, NCTensor *u, NCTensor **g, NCTensor **b, 
     return NULL;
 }
 
+BOOL nc_lstm_layer_fits(NCDevice *d, int n_gate, size_t n_units, size_t n_streams, size_t n_steps)
+{
+    (void)d; (void)n_gate; (void)n_units; (void)n_streams; (void)n_steps;
+    return 0;
+}
+
 NCTensor *nc_geglu(NCTensor *x)
 {
     (void)x;

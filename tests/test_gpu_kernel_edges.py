@@ -90,6 +90,27 @@ def test_lstm_layer_sizes(hosts, cells, batch, seg, variant):
     ref.close()
 
 
+@pytest.mark.parametrize("refused", ["bf16 products", "width invariant", "projection"])
+def test_lstm_segment_without_the_layer_form_issues_no_more_than_its_timesteps(hosts, refused):
+    """A configuration that has no per-layer form goes straight to the sequence of ops: for segments of
+    one timestep the evaluation of the whole segment and that of timestep 0 are one sequence, and
+    issue the same launches."""
+    H = M.load_pkg().host
+    m = H.Model(hosts[0], H.make_lstm_config(n_layer=2, lstm_n_cells=24, lstm_n_cells2=40 if refused == "projection" else 24,
+                                             batch_size=3, seg_len=1, n_symbols=31, use_device=1))
+    if refused == "bf16 products":
+        m.nc.nc_set_matmul_bf16(m.ctx, 1)
+    if refused == "width invariant":
+        m.nc.nc_set_matmul_width_invariant(m.ctx, 1)
+    count = []
+    for index in (-1, 0, -1, 0):
+        before = m.nc.nc_get_launch_count(m.ctx)
+        m.eval(np.zeros((1, 3), np.int32), output_index=index)
+        count.append(m.nc.nc_get_launch_count(m.ctx) - before)
+    m.close()
+    assert count[2] == count[3] > 0, count
+
+
 @pytest.mark.parametrize("streams,steps", [(65535 * 16 + 1, 1), (1, (1 << 24) + 1)])
 def test_lstm_layer_refuses_what_its_launches_cannot_hold(hip, streams, steps):
     """More streams than a grid has rows for, more columns than its indices are laid out for: NULL,
