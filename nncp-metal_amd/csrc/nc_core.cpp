@@ -1014,8 +1014,15 @@ extern "C" void nc_tensor_set_rnd_unif(NCTensor *y, float avg, float range, NCRN
             size_t cap;
             float *tmp = nc_tmp_f32(m, n ? n : 1, &cap);
             device_fill(m, tmp, n, rs, 0, avg, range);
-            if (nchip_cast_bf16(m->stream, tmp, (uint16_t *)nc_data(y), (int64_t)n)) nc_fatal("bf16 cast failed");
+            // (the cast writes 16 bytes at a time: a slice that starts off such a unit takes a copy of its result)
+            size_t hcap = 0;
+            uint16_t *dst = (uint16_t *)nc_data(y), *half = ((uintptr_t)dst & 15) == 0 ? dst : (uint16_t *)nc_tmp_f32(m, n / 2 + 1, &hcap);
+            if (nchip_cast_bf16(m->stream, tmp, half, (int64_t)n)) nc_fatal("bf16 cast failed");
             m->launches++;
+            if (half != dst) {
+                hip_check(hipMemcpyAsync(dst, half, n * sizeof(uint16_t), hipMemcpyDeviceToDevice, m->stream), "hipMemcpyAsync d2d");
+                nc_tmp_free(m, half, hcap);
+            }
             nc_tmp_free(m, tmp, cap);
         }
         return;

@@ -33,6 +33,21 @@ def test_random_fill_across_runs_and_wavefronts(hip, ref, n):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("first,last", [(0, 40), (1, 40), (3, 4), (8, 33), (37, 40)])
+def test_random_fill_of_a_bf16_range(hip, ref, first, last):
+    """A range of a bf16 tensor at any start: the checker's bits, and its neighbours untouched."""
+    got = []
+    for nc in (hip, ref):
+        rs = nc.lib.nc_rnd_init(nc.dev, 5)
+        t = nc.nc_convert(nc.tensor(np.full(40, 2.0, np.float32)), 1)
+        a = nc.nc_slice_alias(t, 0, first, last)
+        nc.lib.nc_tensor_set_rnd_unif(a, 0.5, 0.25, rs)
+        nc.free(a)
+        got.append(nc.numpy(t, free=True))
+        nc.lib.nc_rnd_end(rs)
+    assert np.array_equal(*got)
+
+
 @pytest.mark.parametrize("shape", [(2, 3, 5, 8), (2, 3, 5, 7), (3, 1, 4, 4), (1, 1, 1, 1), (7, 2, 33, 12)])
 def test_permuted_copies_and_broadcasts(hip, shape):
     """Leading axes of whole 16-byte units and others, through the strided copy (a head split and
