@@ -111,8 +111,10 @@ BOOL nc_lstm_layer_fits(NCDevice *d, int n_gate, size_t n_units, size_t n_stream
 /* Gated GELU: for x of 2 h along axis 0 the h values gelu(x[0 .. h)) x[h .. 2h), nc_split, nc_gelu
    and nc_mul (nncp.c:943-947) in one pass each way.  Consumes x.  Returns NULL, with nothing
    consumed, where the library has no such form (libnc_ref.so: always; an odd axis 0, another
-   item type, host tensors): the caller then issues the three. */
-NCTensor *nc_geglu(NCTensor *x);
+   item type, host tensors): the caller then issues the three.  (Not under the name nc_geglu, which
+   libnc.h:253-256 declares in its own form: a program compiled against that header must not be
+   linked to this one.) */
+NCTensor *nc_gelu_gate(NCTensor *x);
 
 /* When non-zero, the forward products of nc_matmul / nc_matmul_add / nc_linear
    use one tile class and one reduction order whatever the number of columns,

@@ -89,7 +89,7 @@ _PROTOS = {
     "nc_convert": (_P, [_P, _I]), "nc_add": (_P, [_P, _P]), "nc_mul": (_P, [_P, _P]),
     "nc_masked_fill": (_P, [_P, _P, _F, _I]),
     "nc_sigmoid": (_P, [_P]), "nc_tanh": (_P, [_P]), "nc_relu": (_P, [_P]),
-    "nc_gelu": (_P, [_P]), "nc_geglu": (_P, [_P]), "nc_gated_swish": (_P, [_P, _P, _F]),
+    "nc_gelu": (_P, [_P]), "nc_gelu_gate": (_P, [_P]), "nc_gated_swish": (_P, [_P, _P, _F]),
     "nc_lstm_layer": (_P, [_P, _P, C.POINTER(_P), C.POINTER(_P), _I, _I, _F, _P, _P]),
     "nc_lstm_clamped": (_P, [_P, _P, _P, _P]), "nc_lerp": (_P, [_P, _P, _P]),
     "nc_reshape_1d": (_P, [_P, _SZ]), "nc_reshape_2d": (_P, [_P, _SZ, _SZ]),

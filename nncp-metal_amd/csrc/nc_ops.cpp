@@ -257,7 +257,7 @@ extern "C" NCTensor *nc_gelu(NCTensor *x) { return unary_op(x, KU_GELU); }      
 
 // nc_ext.h.  (the result and the gradient are operands of the products around them: in bf16 mode
 // their bf16 copies come out of the same pass)
-extern "C" NCTensor *nc_geglu(NCTensor *x)
+extern "C" NCTensor *nc_gelu_gate(NCTensor *x)
 {
     if (!x->dev->is_hip || x->type != NC_TYPE_F32 || x->n_dims < 1 || x->dims[0] % 2) return nullptr;
     x = nc_contig(x);

@@ -524,7 +524,7 @@ static NCTensor *attention_fused(NNCPModel *s, int l, NCTensor *x, NCTensor *res
 /* gelu(first half of x) * second half, in one pass where the library has it */
 static NCTensor *geglu(NCTensor *x)
 {
-    NCTensor *tab[2], *y = nc_geglu(x);
+    NCTensor *tab[2], *y = nc_gelu_gate(x);
     if (y)
         return y;
     nc_split(tab, x, 2, NULL, 0);

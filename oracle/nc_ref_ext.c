@@ -496,7 +496,7 @@ BOOL nc_lstm_layer_fits(NCDevice *d, int n_gate, size_t n_units, size_t n_stream
     return 0;
 }
 
-NCTensor *nc_geglu(NCTensor *x)
+NCTensor *nc_gelu_gate(NCTensor *x)
 {
     (void)x;
     return NULL;

@@ -31,6 +31,15 @@ def test_checker_exports_the_same_abi():
     assert not missing, missing
 
 
+def test_additions_leave_the_reference_header_names_alone():
+    """A function that libnc.h declares and this library does not implement stays undefined: an
+    addition under its name would link with other arguments."""
+    pkg = load_pkg()
+    for path in (pkg.binding.HIP_LIB, os.path.join(ROOT, "oracle", "libnc_ref.so")):
+        lib = ctypes.CDLL(path)
+        assert not [n for n in ("nc_geglu", "nc_apply") if hasattr(lib, n)], path
+
+
 def test_binding_covers_the_link_set_of_the_reference_host():
     """The 90 symbols nncp.c + cp_utils.c leave undefined (nm -u on the objects
     compiled from the reference sources) must all be exported."""

@@ -238,7 +238,7 @@ def test_geglu_is_its_sequence(hip, n, h, bf16):
     got = []
     hip.nc_set_matmul_bf16(hip.ctx, bf16)
     try:
-        for build in (lambda nc, t: nc.nc_geglu(t), cases._split_build):
+        for build in (lambda nc, t: nc.nc_gelu_gate(t), cases._split_build):
             got.append(cases.Case("geglu", [x.shape], build, None).run(hip, [x], w))
             y = build(hip, hip.tensor(x))
             got[-1] += (hip.numpy(hip.nc_matmul(hip.tensor(a), y), free=True),)
