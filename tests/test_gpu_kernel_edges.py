@@ -11,7 +11,7 @@ import modelutil as M
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 3, 255, 257, 16384, 16385, 65537, 300001])
+@pytest.mark.parametrize("n", [1, 3, 255, 257, 16384, 16385, 65537, 300001, (1 << 20) + 77])
 def test_random_fill_across_runs_and_wavefronts(hip, ref, n):
     """A fill starts every run of 256 elements and every wavefront of 64 runs from a state it
     jumps to: each element, and the state the fill leaves behind (seen by the next one), is the
@@ -31,6 +31,19 @@ def test_random_fill_across_runs_and_wavefronts(hip, ref, n):
         got.append(one)
     for a, b in zip(*got):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def test_random_fill_takes_every_jump(hip, ref):
+    """8193 wavefronts and a bit: the start state of one is a product over the bits of its index, so
+    all fourteen jump matrices are taken, each alone and with others."""
+    n, got = (1 << 27) + 16384 + 5, []
+    for nc in (hip, ref):
+        rs = nc.lib.nc_rnd_init(nc.dev, 77)
+        t = nc.nc_new_tensor_nz(nc.dev, 0, 1, (C.c_size_t * 1)(n))
+        nc.lib.nc_tensor_set_rnd_unif(t, 0.5, 0.25, rs)
+        got.append(nc.numpy(t, free=True).view(np.uint32))
+        nc.lib.nc_rnd_end(rs)
+    assert np.array_equal(*got)
 
 
 @pytest.mark.parametrize("first,last", [(0, 40), (1, 40), (3, 4), (8, 33), (37, 40)])
@@ -103,6 +116,51 @@ def test_lstm_layer_sizes(hosts, cells, batch, seg, variant):
         assert M.rel_l2(w_h[k], w_r[k]) <= (1e-4 if w_r[k].size == 1 else 1e-5), (k, M.rel_l2(w_h[k], w_r[k]))
     hip.close()
     ref.close()
+
+
+@pytest.mark.parametrize("cells,batch,seg,variant", [
+    (33, 5, 6, dict()), (130, 17, 5, dict(lstm_type=0, lstm_use_layer_norm=0)), (70, 9, 8, dict(lstm_type=2))])
+def test_lstm_layer_against_float64(hosts, cells, batch, seg, variant):
+    """The per-layer kernels sum in another order than the sequence of ops: whether that loses
+    accuracy is decided by a float64 evaluation of the segment.  Probabilities and every gradient (exposed by
+    one step of plain SGD at a rate that lifts it above the weights, w0 - w1 = 2^20 g) are no further
+    from it than twice what the checker's sequence is, each kind of tensor taken together (a gain's
+    gradient is one number, the sum of many terms of both signs).  Measured, per layer against
+    sequence: probabilities 0.9-1.3e-7 against
+    1.2-1.8e-7, recurrent weights 1.8-2.4e-7 against 1.9-2.9e-7, biases 1.4-2.0e-7 against
+    1.4-2.7e-7, gains 1.8-2.3e-7 against 2.4-2.5e-7."""
+    import torch
+    from test_lstm_torch import lstm_forward_torch
+    H, lr = M.load_pkg().host, float(1 << 20)
+    cfg = dict(n_layer=2, lstm_n_cells=cells, batch_size=batch, seg_len=seg, n_symbols=31, seed=5)
+    cfg.update(variant)
+    rng = np.random.default_rng(cells)
+    tok, tgt = rng.integers(0, 31, size=(2, seg, batch)).astype(np.int32)
+    got = []
+    for host, dev in zip(hosts, (1, 0)):
+        m = H.Model(host, H.make_lstm_config(**dict(cfg, use_device=dev, nb_threads=4, sgd_opt=M.sgd(lr))))
+        noise = np.random.default_rng(1)
+        for k in m.param_names():                    # biases and gains away from their initial 0 / 1
+            if k[0] in "bg" or k == "fc_b":
+                m.set_param(k, m.get_param(k) + 0.3 * noise.standard_normal(m.get_param(k).shape).astype(np.float32))
+        w0 = m.params()
+        p, _ = m.train_step(tok, tgt, lr)
+        w1 = m.params()
+        got.append((p, {k: (w0[k].astype(np.float64) - w1[k]) / lr for k in w0}))
+        m.close()
+    w = {k: torch.tensor(v.astype(np.float64), requires_grad=True) for k, v in w0.items()}
+    logp, _, _ = lstm_forward_torch(w, tok, cfg)
+    (-logp.gather(2, torch.as_tensor(tgt, dtype=torch.long).unsqueeze(2)).mean()).backward()
+    want = logp.exp().detach().numpy()
+    kinds = {"probabilities": (got[0][0], got[1][0], want)}
+    for kind in ("u", "w", "ws", "b", "g", "fc_w", "fc_b"):
+        names = [k for k in w if k.rstrip("_0123456789") == kind]
+        if names:
+            kinds[kind] = [np.concatenate([np.ravel(t[k]) for k in names])
+                           for t in (got[0][1], got[1][1], {k: w[k].grad.numpy() for k in names})]
+    errors = {k: (M.rel_l2(a, x), M.rel_l2(b, x)) for k, (a, b, x) in kinds.items()}
+    print(" ".join("%s %.1e/%.1e" % (k, *e) for k, e in errors.items()))
+    assert len(errors) >= 7 and all(a <= 2.0 * b for a, b in errors.values()), errors
 
 
 @pytest.mark.parametrize("refused", ["bf16 products", "width invariant", "projection"])

@@ -35,11 +35,11 @@ def emulated():
     return dict(os.environ, NNCP_TEST_HIP_LIB=EMU_LIB, NNCP_TEST_HOST_HIP_LIB=EMU_HOST)
 
 
-# Largest shapes of three op tests: a minute or minutes each as fibers, and the same kernels and code paths as
+# Largest shapes of four tests: a minute or minutes each as fibers, and the same kernels and code paths as
 # the smaller shapes of the same tests that do run here (the GPU run has all of them)
 OPS_LEFT_TO_THE_GPU = ("not (k_major_weight_copies and (512-2048-32 or 1024-1024-33 or 2048-512-32)) and "
                        "not (few_column_products and (512-2048-32 or 2048-512-32)) and "
-                       "not (embedding_gradient and 16384-64-4096)")
+                       "not (embedding_gradient and 16384-64-4096) and not takes_every_jump")
 
 
 def _pytest(env, args):
@@ -68,7 +68,7 @@ def test_gpu_parity_tests_pass_on_the_cpu_build(emulated):
                              "not (file_container and (reference or bf16)) and not full_size and "
                              "not (properties_small and bf16) and not 100_steps and not enwik8_profile and "
                              "not (memory_window and 0)"])
-    edges = _pytest(emulated, ["-n", "3", "tests/test_gpu_kernel_edges.py"])
+    edges = _pytest(emulated, ["-n", "3", "tests/test_gpu_kernel_edges.py", "-k", OPS_LEFT_TO_THE_GPU])
     out_ops, out_model = ops.communicate(timeout=1500)[0], model.communicate(timeout=1500)[0]
     out_new, out_edges = new.communicate(timeout=1500)[0], edges.communicate(timeout=1500)[0]
     assert ops.returncode == 0, out_ops[-3000:]
