@@ -65,9 +65,12 @@ void k_lstm_clamped_bwd(hipStream_t st, const float *cp, const float *in, const 
 // y = a * b * ... helpers for backward of mul: t = g * other[i % nb]
 // (k_binary_prefix with KB_MUL covers it)
 
-// out[i] = sum_o x[i + o*inner], o < outer, fixed order; tmp: nsplit*inner floats
+// columns of 2h: y = gelu(x[0 .. h)) x[h .. 2h), and its gradient for both halves (y16 / dx16: the
+// result once more as bf16, may be NULL)
 void k_geglu_fwd(hipStream_t st, const float *x, float *y, uint16_t *y16, int64_t h, int64_t cols);
 void k_geglu_bwd(hipStream_t st, const float *x, const float *g, float *dx, uint16_t *dx16, int64_t h, int64_t cols);
+
+// out[i] = sum_o x[i + o*inner], o < outer, fixed order; tmp: nsplit*inner floats
 int k_reduce_trailing_nsplit(int64_t inner, int64_t outer);
 // out = [y0 +] the sums over the outer axis; returns the number of launches: one where that axis
 // has at most K_REDUCE_ONCE entries

@@ -521,10 +521,10 @@ static NCTensor *attention_fused(NNCPModel *s, int l, NCTensor *x, NCTensor *res
     return nc_matmul_add(nc_dup_tensor(tl->w_o), att, res, 0, 0, 1.0f);
 }
 
-/* gelu(first half of x) * second half, in one pass where the library has it */
-static NCTensor *geglu(NCTensor *x)
+/* gelu(first half of x) * second half; one_pass: in one pass where the library has it */
+static NCTensor *geglu(NCTensor *x, int one_pass)
 {
-    NCTensor *tab[2], *y = nc_gelu_gate(x);
+    NCTensor *tab[2], *y = one_pass ? nc_gelu_gate(x) : NULL;
     if (y)
         return y;
     nc_split(tab, x, 2, NULL, 0);
@@ -548,7 +548,7 @@ static NCTensor *feed_forward(NNCPModel *s, int l, NCTensor *x, NCTensor *res)
         return nc_linear(nc_dup_tensor(tl->ff2), t0, tl->ff_bias2 ? nc_dup_tensor(tl->ff_bias2) : NULL, NC_ACT_NONE);
     }
     if (s->fused_now && act == NNCP_FF_GEGLU) {
-        t0 = geglu(nc_linear(nc_dup_tensor(tl->ff1), x, tl->ff_bias1 ? nc_dup_tensor(tl->ff_bias1) : NULL, NC_ACT_NONE));
+        t0 = geglu(nc_linear(nc_dup_tensor(tl->ff1), x, tl->ff_bias1 ? nc_dup_tensor(tl->ff_bias1) : NULL, NC_ACT_NONE), 1);
         if (res)
             return nc_linear_add(nc_dup_tensor(tl->ff2), t0, tl->ff_bias2 ? nc_dup_tensor(tl->ff_bias2) : NULL,
                                  NC_ACT_NONE, res);
@@ -564,12 +564,7 @@ static NCTensor *feed_forward(NNCPModel *s, int l, NCTensor *x, NCTensor *res)
     case NNCP_FF_RELU: t0 = nc_relu(t0); break;
     case NNCP_FF_GELU: t0 = nc_gelu(t0); break;
     case NNCP_FF_GEGLU:
-        if (c->fused) {
-            t0 = geglu(t0);
-            break;
-        }
-        nc_split(tab, t0, 2, NULL, 0);
-        t0 = nc_mul(nc_gelu(tab[0]), tab[1]);
+        t0 = geglu(t0, c->fused);
         break;
     case NNCP_FF_GATED_SILU:
         nc_split(tab, t0, 2, NULL, 0);
