@@ -36,12 +36,10 @@ extern "C" {
    (nearest-even) on load, fp32 accumulation on the bf16 MFMA units.
    ksplit > 1 splits the reduction over that many workgroups whose partial
    tiles are summed in a fixed order by a second kernel; it needs
-   `workspace` of at least batch*ksplit*m*n floats (NULL will do where
-   nchip_gemm_is_small and no rows are skipped: lda, ldb tight).  The tile class
-   is chosen from m, n, batch and ksplit;
-   inside a class every output element is a fixed sequence of MFMA
-   accumulations over k = 0..K-1 (the 64x64 class: two interleaved chains, added),
-   whatever m, n, the number of columns and the kernel that issues it.  With
+   `workspace` of at least batch*ksplit*m*n floats.  The tile class is chosen
+   from m, n, batch and ksplit; inside a class every output element is a fixed
+   sequence of MFMA accumulations over k = 0..K-1 (the 64x64 class: two
+   interleaved chains, added), whatever m, n and the kernel that issues it.  With
    NCHIP_GEMM_WIDTH_INVARIANT the class does not depend on the shape either. */
 int nchip_gemm(void *stream, int ta, int tb, int m, int n, int k, float alpha,
                const float *A, int64_t lda, int64_t stride_a,
@@ -232,7 +230,7 @@ void nchip_gemm_bf16_source(int mode);
 /* Chooses ksplit for nchip_gemm from the shape alone (never from data). */
 int nchip_gemm_pick_ksplit(int m, int n, int k, int batch);
 /* 1 when an fp32 product of this shape without an activation gradient, at the ksplit chosen
-   above, is one launch of the small-product kernel (the 64x64 class's sums) and takes no workspace */
+   above, is one launch of the small-product kernel (the 64x64 class's sums) */
 int nchip_gemm_is_small(int m, int n, int k, int batch);
 
 /* Relative-position causal attention, forward (nncp.c:722-800 fused).

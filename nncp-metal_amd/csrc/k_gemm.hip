@@ -1779,9 +1779,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     const bool invariant = (precision & NCHIP_GEMM_WIDTH_INVARIANT) != 0;
     precision &= 0xff;
     if (ksplit < 1 || invariant) ksplit = 1;
-    const bool small_fits = precision == 0 && !dpre && ksplit <= SMALL_KSPLIT && (k + 16) * (lda > ldb ? lda : ldb) < 1 << 29; // (32-bit byte offsets)
-    const bool small = !invariant && !g_force_cfg && small_fits && gemm_is_small(m, n, k, batch, ksplit);
-    if (ksplit > 1 && !workspace && !small) {
+    if (ksplit > 1 && !workspace) {
         fprintf(stderr, "nchip_gemm: ksplit=%d needs a workspace\n", ksplit);
         return -1;
     }
@@ -1840,6 +1838,8 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
         }
         return 0;
     }
+    const bool small_fits = precision == 0 && !dpre && ksplit <= SMALL_KSPLIT && (k + 16) * (lda > ldb ? lda : ldb) < 1 << 29; // (32-bit byte offsets)
+    const bool small = !invariant && !g_force_cfg && small_fits && gemm_is_small(m, n, k, batch, ksplit);
     int cfg = invariant ? 30 : g_force_cfg; // tuning aid: 0 = choose from the shape
     if (cfg == 40 && !small_fits) cfg = 10;
     if (!cfg) cfg = small ? 40 : gemm_class(m, n, (int64_t)batch * ksplit);

@@ -685,7 +685,7 @@ static void dev_gemm(NCContext *m, bool ta, bool tb, size_t M, size_t N, size_t 
     const int ks = invariant ? 1 : nchip_gemm_pick_ksplit((int)M, (int)N, (int)K, (int)batch);
     size_t cap = 0;
     float *ws = nullptr;
-    if (ks > 1 && (prec != 0 || !nchip_gemm_is_small((int)M, (int)N, (int)K, (int)batch))) ws = nc_tmp_f32(m, batch * ks * M * N, &cap);
+    if (ks > 1) ws = nc_tmp_f32(m, batch * ks * M * N, &cap);
     int rc;
     // a few columns against a weight matrix with a k-major copy: the same chains from the copy
     const float *a_data = nc_f32(a);
@@ -710,7 +710,7 @@ static void dev_gemm(NCContext *m, bool ta, bool tb, size_t M, size_t N, size_t 
                         bias, act, pre, prec, ks, ws);
     if (ws) nc_tmp_free(m, ws, cap);
     if (rc) nc_fatal("gemm failed (m=%zu n=%zu k=%zu)", M, N, K);
-    m->launches += ws ? 2 : 1;
+    m->launches += ks > 1 && !(prec == 0 && nchip_gemm_is_small((int)M, (int)N, (int)K, (int)batch)) ? 2 : 1;
 }
 
 // libnc.h:365-373

@@ -284,6 +284,19 @@ def test_small_products_at_every_remainder_of_k(hip, ta, tb):
             assert np.array_equal(small[0], tile[0]), (case, np.abs(small[0] - tile[0]).max())
 
 
+def test_a_split_product_without_a_workspace_is_refused(hip):
+    """Whatever kernel the shape would go to: -1, and nothing written."""
+    lib = C.CDLL(hip.lib._name)
+    t = [hip.tensor(np.full((64, 64), 2.0, np.float32)) for _ in range(3)]
+    a, b, c = (C.c_void_p(hip.nc_tensor_get_ptr(x, None)) for x in t)
+    for k, n in ((64, 8), (16, 64)):
+        assert lib.nchip_gemm(C.c_void_p(hip.nc_context_stream(hip.ctx)), 0, 0, 8, n, k, C.c_float(1), a, C.c_int64(64), C.c_int64(0),
+                              b, C.c_int64(64), C.c_int64(0), C.c_float(0), c, C.c_int64(64), C.c_int64(0), 1,
+                              None, 0, None, 0, 2, None) == -1
+    assert np.all(hip.numpy(t[2]) == 2.0)
+    hip.free(*t)
+
+
 @pytest.mark.parametrize("n,h", [(1, 1), (3, 4), (5, 7), (513, 12), (2048, 96)])
 @pytest.mark.parametrize("bf16", [0, 1])
 def test_geglu_is_its_sequence(hip, n, h, bf16):
