@@ -332,88 +332,127 @@ __global__ __launch_bounds__(TPB) void cdf_lookup_kernel(const uint16_t *cdf, co
 
 // Many targets per column: first turn the column's CDF into the full inverse
 // table inv[t] = symbol of target value t (65536 uint16 entries, 128 KiB of
-// LDS; each entry by the same search, read from the cached CDF), after which
-// a lookup is one LDS read.  Entry t depends on the CDF alone, so the result
-// is the one the search gives.
-constexpr int INV_NT = 1024;
+// LDS), after which a lookup is one LDS read.  The table is a scatter and a
+// running maximum: entry cdf[s] receives s, every other entry 0, and the symbol
+// of t is the largest value at or below t - what the search over the ascending
+// CDF gives.  It takes 4 us a workgroup (a search per entry, as it was built
+// before, 28); the lookups that follow are bound by memory and by the random
+// 2-byte LDS reads behind each 16-byte load.  64 x 16384, 10^6 lookups a column,
+// 256 MB: 64.7 -> 48.0 us; one column of 10^6: 33.6 -> 9.6 us.
+typedef unsigned short ushortx2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int INV_NT = 1024, INV_ROWS = 65536 / (8 * INV_NT); // a row: 8 entries of every thread
+__device__ __forceinline__ uint32_t max2(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(ushortx2, a), __builtin_bit_cast(ushortx2, b)));
+}
 __global__ __launch_bounds__(INV_NT) void cdf_lookup_table_kernel(const uint16_t *cdf, const uint16_t *target,
-                                                                  uint16_t *sym, int v, int64_t m, int steps,
-                                                                  int vec)
+                                                                  uint16_t *sym, int v, int64_t m, int vec)
 {
     extern __shared__ __attribute__((aligned(16))) uint16_t inv[];
-    __shared__ uint16_t coarse[INV_NT + 1];
+    __shared__ uint16_t row_max[INV_ROWS * INV_NT / 64]; // of every row and wavefront, in table order
     const uint16_t *c = cdf + (int64_t)blockIdx.y * v;
-    {   // the symbol of every 64th target value, by the full search
-        int lo = 0, hi = v;
-        unsigned int tv = threadIdx.x * 64;
-        for (int s = 0; s < steps; s++) {
-            int mid = (lo + hi) >> 1;
-            bool le = c[mid] <= tv;
-            lo = le ? mid : lo;
-            hi = le ? hi : mid;
-        }
-        coarse[threadIdx.x] = (uint16_t)lo;
-        if (threadIdx.x == 0) coarse[INV_NT] = (uint16_t)(v - 1);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    u32x4 *inv4 = reinterpret_cast<u32x4 *>(inv);
+#pragma unroll
+    for (int j = 0; j < INV_ROWS; j++) inv4[j * INV_NT + t] = u32x4{ 0, 0, 0, 0 };
+    __syncthreads();
+#pragma unroll 4
+    for (int s = t; s < v; s += INV_NT) {
+        const unsigned int here = c[s], next = s + 1 < v ? c[s + 1] : 65536u;
+        if (next > here) inv[here] = (uint16_t)s; // (one symbol an entry: the last of those that share a value)
     }
     __syncthreads();
-    // the symbols of target values 64 b .. 64 b + 63 lie between coarse[b] and
-    // coarse[b + 1], at most 65 candidates (every symbol has frequency >= 1):
-    // 7 halvings finish each of them; eight run side by side
-    for (int t0 = threadIdx.x; t0 < 65536; t0 += 8 * INV_NT) {
-        int lo[8], hi[8];
+    u32x4 r[INV_ROWS];
+    uint32_t top[INV_ROWS / 2]; // the maxima of rows 2 i and 2 i + 1 up to this lane
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            int bkt = (t0 + j * INV_NT) >> 6;
-            lo[j] = coarse[bkt];
-            hi[j] = coarse[bkt + 1] + 1;
+    for (int j = 0; j < INV_ROWS; j++) {
+        r[j] = inv4[j * INV_NT + t];
+        uint32_t run = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            r[j][e] = max2(max2(r[j][e], r[j][e] << 16), run);
+            run = (r[j][e] >> 16) * 0x10001u;
         }
+        top[j / 2] = j & 1 ? (top[j / 2] & 0xffffu) | (run & 0xffff0000u) : run & 0xffffu;
+    }
 #pragma unroll
-        for (int s = 0; s < 7; s++) {
-            unsigned int cv[8];
-            int mid[8];
+    for (int i = 0; i < INV_ROWS / 2; i++)
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                mid[j] = (lo[j] + hi[j]) >> 1;
-                cv[j] = c[mid[j]];
-            }
+        for (int d = 1; d < 64; d <<= 1) top[i] = max2(top[i], __shfl_up(top[i], d, 64)); // (a lane without a source sees its own)
+    if (lane == 63) {
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                bool le = cv[j] <= (unsigned int)(t0 + j * INV_NT);
-                lo[j] = le ? mid[j] : lo[j];
-                hi[j] = le ? hi[j] : mid[j];
-            }
-        }
+        for (int j = 0; j < INV_ROWS; j++) row_max[j * (INV_NT / 64) + wave] = (uint16_t)(top[j / 2] >> (j & 1) * 16);
+    }
+    __syncthreads();
+    static_assert(INV_ROWS * INV_NT / 64 == 128, "two row maxima a lane");
+    uint32_t pre = reinterpret_cast<const uint32_t *>(row_max)[lane];
+    pre = max2(pre, pre << 16);
+    uint32_t upto = pre >> 16; // the maximum of everything up to row maximum 2 lane + 1
 #pragma unroll
-        for (int j = 0; j < 8; j++) inv[t0 + j * INV_NT] = (uint16_t)lo[j];
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(upto, d, 64);
+        upto = o > upto ? o : upto;
+    }
+    uint32_t before = __shfl_up(upto, 1, 64);
+    if (lane == 0) before = 0;
+    pre = max2(pre, before * 0x10001u);
+#pragma unroll
+    for (int j = 0; j < INV_ROWS; j++) {
+        const int i = j * (INV_NT / 64) + wave - 1; // the row maximum before this wavefront's part of row j
+        uint32_t base = (__shfl(pre, (i < 0 ? 0 : i) >> 1, 64) >> (i & 1) * 16) & 0xffffu;
+        if (i < 0) base = 0;
+        uint32_t left = (__shfl_up(top[j / 2], 1, 64) >> (j & 1) * 16) & 0xffffu;
+        if (lane == 0) left = 0;
+        base = (left > base ? left : base) * 0x10001u;
+#pragma unroll
+        for (int e = 0; e < 4; e++) r[j][e] = max2(r[j][e], base);
+        inv4[j * INV_NT + t] = r[j];
     }
     __syncthreads();
     const uint16_t *tp = target + (int64_t)blockIdx.y * m;
     uint16_t *sp = sym + (int64_t)blockIdx.y * m;
-    // this workgroup's share of the column, cut at multiples of 4 targets
-    int64_t quads = (m + 3) >> 2;
-    int64_t per = (quads + gridDim.x - 1) / gridDim.x;
-    int64_t q0 = per * blockIdx.x, q1 = q0 + per < quads ? q0 + per : quads;
-    if (vec) {
-        // four 8-byte loads in flight per lane (index clamped, store guarded)
-        for (int64_t q = q0 + threadIdx.x; q < q1; q += 4 * INV_NT) {
-            uint2 tv[4];
+    // units of 8 targets from the first 16-byte boundary of the column on (vec: its symbols have theirs
+    // at the same place), this workgroup's share of them; the first workgroup takes what is left
+    const int64_t head0 = vec ? ((16 - ((uintptr_t)tp & 15)) & 15) >> 1 : m, head = head0 < m ? head0 : m;
+    const int64_t units = (m - head) >> 3, per = (units + gridDim.x - 1) / gridDim.x;
+    const int64_t u0 = per * blockIdx.x, u1 = u0 + per < units ? u0 + per : units;
+    const u32x4 *t4 = reinterpret_cast<const u32x4 *>(tp + head);
+    u32x4 *s4 = reinterpret_cast<u32x4 *>(sp + head);
+    // two units a lane in flight while the two before them are looked up (index clamped, store guarded)
+    u32x4 cur[2], nxt[2];
+    if (u0 < u1) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                int64_t qj = q + j * INV_NT;
-                tv[j] = *reinterpret_cast<const uint2 *>(tp + 4 * (qj < q1 ? qj : q));
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                int64_t qj = q + j * INV_NT;
-                uint2 r;
-                r.x = (unsigned int)inv[tv[j].x & 0xffffu] | ((unsigned int)inv[tv[j].x >> 16] << 16);
-                r.y = (unsigned int)inv[tv[j].y & 0xffffu] | ((unsigned int)inv[tv[j].y >> 16] << 16);
-                if (qj < q1) *reinterpret_cast<uint2 *>(sp + 4 * qj) = r;
-            }
+        for (int j = 0; j < 2; j++) {
+            const int64_t u = u0 + t + j * INV_NT;
+            cur[j] = t4[u < u1 ? u : u1 - 1];
         }
-    } else {
-        int64_t i1 = 4 * q1 < m ? 4 * q1 : m;
-        for (int64_t i = 4 * q0 + threadIdx.x; i < i1; i += INV_NT) sp[i] = inv[tp[i]];
+    }
+    for (int64_t u = u0 + t; u - t < u1; u += 2 * INV_NT) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const int64_t uj = u + (2 + j) * INV_NT;
+            nxt[j] = t4[uj < u1 ? uj : u1 - 1];
+        }
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            u32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                o[e] = (uint32_t)inv[cur[j][e] & 0xffffu] | (uint32_t)inv[cur[j][e] >> 16] << 16;
+            if (u + j * INV_NT < u1) s4[u + j * INV_NT] = o;
+            cur[j] = nxt[j];
+        }
+    }
+    if (vec) {
+        if (blockIdx.x == 0) {
+            if (t < head) sp[t] = inv[tp[t]];
+            const int64_t rest = head + 8 * units + t;
+            if (t < 8 && rest < m) sp[rest] = inv[tp[rest]];
+        }
+    } else { // targets and symbols aligned differently: one at a time
+        const int64_t share = (m + gridDim.x - 1) / gridDim.x, i1 = share * (blockIdx.x + 1);
+        for (int64_t i = share * blockIdx.x + t; i < (i1 < m ? i1 : m); i += INV_NT) sp[i] = inv[tp[i]];
     }
 }
 
@@ -555,6 +594,8 @@ extern "C" int nchip_cdf_path(void *stream, const uint16_t *cdf, const int32_t *
     return 0;
 }
 
+constexpr int64_t CDF_TABLE_COST = 32768; // lookups a workgroup does in the time it builds its table in
+
 extern "C" int nchip_cdf_lookup(void *stream, const uint16_t *cdf, const uint16_t *target,
                                 uint16_t *sym, int v, int64_t m, int64_t n)
 {
@@ -567,17 +608,23 @@ extern "C" int nchip_cdf_lookup(void *stream, const uint16_t *cdf, const uint16_
     int64_t bx = (m + TPB * 16 - 1) / (TPB * 16);
     int64_t cap = (4096 + n - 1) / n;
     if (bx > cap) bx = cap;
-    // the table costs 65536 searches per workgroup: worth it from a few times
-    // that many targets per workgroup on
+    // Table or search, both measured (us; v x columns, lookups a column): 256 x 64, 32768 6.5 search,
+    // 7.3 table; 65536 9.1, 8.2; 10^6 99, 43; 1000 x 40, 65536 8.8, 7.7; 2048 x 8, 2000 5.1, 7.0, 4001
+    // 8.2, 7.0; 16384 x 1, 1000 5.2, 9.3, 4001 13.2, 9.3; 16384 x 64, 10^6 576, 48.  A search is
+    // log2 v dependent LDS reads behind the staging of its column, a table two passes over LDS.
     static const bool table_ok = allow_table_lds();
-    if (table_ok && m >= 4 * 65536) {
-        int64_t split = (256 + n - 1) / n; // workgroups per column: one per CU (the table fills its LDS)
-        if (split > m / (2 * 65536)) split = m / (2 * 65536);
-        if (split < 1) split = 1;
-        // 8-byte accesses need every column (m targets apart) to start aligned
-        int vec = (m & 3) == 0 && ((uintptr_t)target & 7) == 0 && ((uintptr_t)sym & 7) == 0;
+    if (table_ok && (v >= 2048 ? m >= 4000 : m >= 32768 && m * n >= 4 << 20)) {
+        // one workgroup a CU (the table fills its LDS): the split of a column whose rounds of
+        // workgroups, each a table and a share of at least 4096 lookups, take the least time
+        int64_t split = 1, best = INT64_MAX;
+        for (int64_t s = 1; s == 1 || (s <= 256 && s <= m >> 12); s++) {
+            const int64_t cost = (s * n + 255) / 256 * (CDF_TABLE_COST + (m + s - 1) / s);
+            if (cost < best) { best = cost; split = s; }
+        }
+        // 16-byte accesses from each column's first boundary on: the same place in targets and symbols
+        const int vec = (((uintptr_t)target ^ (uintptr_t)sym) & 15) == 0;
         hipLaunchKernelGGL(cdf_lookup_table_kernel, dim3((unsigned)split, (unsigned)n), dim3(INV_NT), 65536 * 2,
-                           (hipStream_t)stream, cdf, target, sym, v, m, steps, vec);
+                           (hipStream_t)stream, cdf, target, sym, v, m, vec);
     } else {
         dim3 grid((unsigned)bx, (unsigned)n);
         if (v <= 16384)

@@ -359,3 +359,25 @@ def test_gradients_of_a_parameter_used_three_times(hip, m, k, cols, ta):
     want = sum(g.astype(np.float64).sum(0) for g in gs) + 2.0 * b
     size = sum(g.sum(0) for g in f[1]) + 2 * np.abs(b)
     assert np.all(np.abs(grads.get(pb).reshape(m) - want) <= 2.0 ** -24 * (cols + 8) * (size + np.abs(want)))
+
+
+@pytest.mark.parametrize("v,n,m,to,so", [(2048, 2, 4000, 0, 0), (2049, 3, 4007, 3, 3), (16385, 1, 8195, 1, 0),
+                                         (65535, 1, 4001, 7, 7), (300, 33, 131073, 0, 0)])
+def test_lookup_table_inverts_an_ascending_cdf(hip, v, n, m, to, so):
+    """The inverse table of nchip_cdf_lookup, with columns that start `to` / `so` elements off a 16-byte
+    boundary: runs of one target and of thousands, entries that share a value (the last one's
+    symbol), a first entry above zero (symbol 0 below it)."""
+    rng, lib = np.random.default_rng(v), C.CDLL(hip.lib._name)
+    c = np.sort(rng.integers(0, 65536, (n, v)) if v > 1000 else 65535 * rng.random((n, v)) ** 8, axis=1).astype(np.uint16)
+    t = rng.integers(0, 65536, (n, m)).astype(np.uint16)
+    t[:, :3], t[:, -2:] = [[0, 65535, c[0, v // 2]]], [[c[0, 0], 65535]]
+    c_t, t_t = hip.tensor(c), hip.tensor(np.concatenate([np.zeros(to, np.uint16), t.ravel()]))
+    s_t = hip.tensor(np.full(so + n * m + 8, 0xabcd, np.uint16))
+    ptr = [C.c_void_p(hip.nc_tensor_get_ptr(x, None) + o) for x, o in ((c_t, 0), (t_t, 2 * to), (s_t, 2 * so))]
+    assert lib.nchip_cdf_lookup(C.c_void_p(hip.nc_context_stream(hip.ctx)), *ptr, C.c_int(v), C.c_int64(m), C.c_int64(n)) == 0
+    got = hip.numpy(s_t)
+    assert (got[:so] == 0xabcd).all() and (got[so + n * m:] == 0xabcd).all()
+    want = [np.maximum(np.searchsorted(c[r], t[r], side="right") - 1, 0) for r in range(n)]
+    assert np.array_equal(got[so:so + n * m].reshape(n, m), want)
+    for x in (c_t, t_t, s_t):
+        hip.free(x)
