@@ -98,12 +98,14 @@ typedef struct {
     float alpha;
 } NchipGemmProblem;
 int nchip_gemm_grouped_tiles(int m, int n);
+int nchip_gemm_grouped_tiles256(int m, int n); /* the same for precision 3 */
 /* precision 0: fp32; 1: fp32 operands rounded to bf16 in the tile loader; 2: the operand
    pointers of the table address bf16 copies (2 bytes per element, same layout and leading
    dimensions as the fp32 matrices they were rounded from), read with unguarded 16-byte
    loads - every k and k2 a multiple of 64, every row-contiguous operand extent (m with
    ta = 0, n with tb = 1) a multiple of 128, leading dimensions multiples of 8, bases 16-byte
-   aligned; the caller checks.  C is fp32 in all three. */
+   aligned; the caller checks; 3: as 2 in 256x256 tiles, tile_start and total_tiles counted by
+   nchip_gemm_grouped_tiles256.  C is fp32 in all of them. */
 int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmProblem *dev_table,
                        int n_problems, int total_tiles, int precision, double total_flops);
 
@@ -111,10 +113,9 @@ int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmProblem *dev
    from memory: A16 / B16 address the bf16 copies of the fp32 matrices (element for element,
    same column-major layout and leading dimensions, no padding), accumulation in fp32 on
    v_mfma_f32_32x32x16_bf16.  The values are those of nchip_gemm with precision 1 up to the
-   order of the k sum inside a tile class.  Unguarded 16-byte loads throughout: k a multiple
-   of 64, leading dimensions multiples of 8, bases 16-byte aligned, and an operand whose long
-   axis is contiguous (A with ta = 0, B with tb = 1) must fill whole tiles of the class the
-   shape selects (128 or 64 rows / columns).  Returns 1 when the shape does not fit (nothing
+   order of the k sum.  Unguarded 16-byte loads throughout: k a multiple of 64, leading
+   dimensions multiples of 8, bases 16-byte aligned, and an operand whose long axis is
+   contiguous (A with ta = 0, B with tb = 1) a multiple of 64 along it.  Returns 1 when the shape does not fit (nothing
    launched: the caller takes another route), 0 when launched, negative on error.
      pre / addend / dpre+dact / rowsum+rows_written: as in nchip_gemm_add, nchip_gemm_dact and
      nchip_gemm_dact_rowsum (all optional);
@@ -138,7 +139,8 @@ typedef struct {
     int *rows_written;
 } NchipGemmBf16Args;
 int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a);
-/* tuning aid: 0 = tile class from the shape, 1 = 128x128, 2 = 128x64, 3 = 64x64 (all 64 deep) */
+/* tuning aid: 0 = tile class from the shape, 1 = 128x128, 2 = 128x64, 3 = 64x64, 4 = 256x256,
+   5 = 128x128 with 8 wavefronts (all 64 deep) */
 void nchip_gemm_bf16_operands_class(int cls);
 
 /* Optional timing of every GEMM launch with HIP events on the launch stream.

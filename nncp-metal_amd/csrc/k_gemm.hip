@@ -19,7 +19,7 @@
 //
 // precision 1 rounds both operands to bf16 (nearest-even) while they are written to LDS and
 // feeds v_mfma_f32_32x32x16_bf16 (fp32 accumulate); large products go through bf16 copies of
-// the operands instead (cast_bf16_kernel + the BF16 = 2 tile kernels).
+// the operands instead (cast_bf16_kernel + gemm_dma_kernel).
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 #include <stdint.h>
@@ -33,6 +33,7 @@
 #include "k_bf16.h"
 #include "k_act.h"
 #include "k_norm_inline.h"
+#include "k_lds_dma.h"
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -261,90 +262,6 @@ struct TileLoaderBf16 {
             } else {
                 lds[(k >> 1) * (BT + PAD) + i] = pack_bf16(r[v][0], r[v][1]);
                 lds[((k >> 1) + 1) * (BT + PAD) + i] = pack_bf16(r[v][2], r[v][3]);
-            }
-        }
-    }
-};
-
-// Loader for operands that are already bf16 in memory (same column-major
-// layout as the fp32 matrix they were rounded from, padded: the k extent is a
-// whole number of tiles with zeros in the padding, and the allocation runs at
-// least one tile past the last row so reads need no guard).  Same LDS layout
-// as above.  Every load is 16 bytes (8 values):
-//   MAJOR = 1: rows k and k+1 of 8 consecutive columns i -> 8 words, two
-//              16-byte LDS writes;
-//   MAJOR = 0: 8 consecutive k of one column i (row index clamped at the
-//              edge) -> 4 words that already are k pairs, 4 LDS writes.
-template <int BT, int BK, int MAJOR, int NT>
-struct TileLoaderBf16Src {
-    static constexpr int NU = MAJOR ? (BT / 8) * (BK / 2) : BT * (BK / 8); // 16-byte units per tile
-    static constexpr int NV = (NU + NT - 1) / NT;
-    static_assert(NU % 64 == 0 && (NU >= NT ? NU % NT == 0 : true), "whole wavefronts take part or sit out");
-    u32x4 r[NV][MAJOR ? 2 : 1];
-
-    __device__ __forceinline__ static void coords(int v, int t, int &i, int &k)
-    {
-        int idx = t + v * NT;
-        if (MAJOR) { i = (idx % (BT / 8)) * 8; k = (idx / (BT / 8)) * 2; }
-        else       { i = idx / (BK / 8);       k = (idx % (BK / 8)) * 8; }
-    }
-
-    __device__ __forceinline__ void load(const float *pf, int64_t ld, int i0, int k0,
-                                         int imax, int kmax, bool fast, int t)
-    {
-        (void)kmax; (void)fast;
-        const uint16_t *p = reinterpret_cast<const uint16_t *>(pf);
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-            if (NU < NT && t >= NU) break;
-            int i, k;
-            coords(v, t, i, k);
-            if (MAJOR) {
-                const uint16_t *src = p + (int64_t)(k0 + k) * ld + (i0 + i);
-                r[v][0] = *as_global(reinterpret_cast<const u32x4 *>(src));
-                r[v][1] = *as_global(reinterpret_cast<const u32x4 *>(src + ld));
-            } else {
-                int row = i0 + i < imax ? i0 + i : imax - 1;
-                r[v][0] = *as_global(reinterpret_cast<const u32x4 *>(p + (int64_t)row * ld + (k0 + k)));
-            }
-        }
-    }
-
-    // MAJOR = 1 writes the word-pair layout of TileLoaderBf16 (rows of k pairs,
-    // BT + PAD words each); the two 16-byte halves of a unit go out in an
-    // order that alternates every 4 lanes, so the 8 lanes served together
-    // cover all 32 banks.  MAJOR = 0 keeps k contiguous: row i holds its
-    // BK / 2 words, SQ words apart, and a unit is one 16-byte write.
-    static constexpr int SQ = BK / 2 + 4;
-    __device__ __forceinline__ void store(uint32_t *lds, int t) const
-    {
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-            if (NU < NT && t >= NU) break;
-            int i, k;
-            coords(v, t, i, k);
-            if (MAJOR) {
-                const uint32_t a[4] = { r[v][0][0], r[v][0][1], r[v][0][2], r[v][0][3] };
-                const uint32_t b[4] = { r[v][1][0], r[v][1][1], r[v][1][2], r[v][1][3] };
-                uint32_t w[8];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    w[2 * e] = (a[e] & 0xffffu) | (b[e] << 16);
-                    w[2 * e + 1] = (a[e] >> 16) | (b[e] & 0xffff0000u);
-                }
-                const bool hi_first = ((t >> 2) & 1) != 0;
-                uint32_t *dst = lds + (k >> 1) * (BT + PAD) + i;
-                uint32_t f[4], g[4]; // first and second write, chosen word by word (register selects)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    f[e] = hi_first ? w[4 + e] : w[e];
-                    g[e] = hi_first ? w[e] : w[4 + e];
-                }
-                const int o1 = hi_first ? 4 : 0;
-                *reinterpret_cast<u32x4 *>(dst + o1) = u32x4{ f[0], f[1], f[2], f[3] };
-                *reinterpret_cast<u32x4 *>(dst + (4 - o1)) = u32x4{ g[0], g[1], g[2], g[3] };
-            } else {
-                *reinterpret_cast<u32x4 *>(lds + i * SQ + (k >> 1)) = r[v][0];
             }
         }
     }
@@ -857,49 +774,17 @@ __global__ __launch_bounds__(256) void gemm_fewcol_mfma(GemmArgs g)
     *Cp = v + extra;
 }
 
-// KW = 2 doubles the wavefronts of a workgroup without shrinking its tile: the
-// two groups of WM x WN wavefronts share the LDS tiles and split every 32-deep
-// k slab, group 0 taking k%32 < 16 and group 1 the rest; group 1 hands its
-// accumulators over through LDS at the end (C = chain0 + chain1, fixed order).
-// NACC = 2 (the width-invariant class): each k group keeps two accumulator sets and gives
-// the first four MFMA steps of every 32-deep slab to one, the last four to the other, so a
-// product is four chains - chain c takes k%32 in [8c, 8c+8) - summed as (c0 + c1) + (c2 + c3).
-// The products are the same; the order of the additions is what a kernel with four
-// wavefronts per row tile can reproduce (gemm_skinny_nn).
-template <int BM, int BN, int BK, int WM, int WN, int TA, int TB, int BF16, int KW = 1, int PF = 2, int SA = (BF16 == 2), int NACC = 1, int FRAG = 0>
-__global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
+// The tile of this workgroup and, in a grouped launch, the problem that owns it (g receives that
+// problem's operands and extents; A2 / B2 its second k range, from k1 on).
+template <int BM, int BN>
+__device__ __forceinline__ void find_tile(GemmArgs &g, int &tile_m, int &tile_n, const float *&A2, const float *&B2, int &k1)
 {
-    GemmArgs g = g0;
-    static_assert(NACC == 1 || (NACC == 2 && BF16 == 0 && KW == 2 && BK == 32), "two accumulator sets: fp32 64-wide class only");
-    static_assert(KW == 1 || (KW == 2 && BK % 32 == 0), "k groups split 32-deep slabs");
-    constexpr int NT = 64 * WM * WN * KW;                 // threads: KW groups of WM x WN wavefronts
-    constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN); // 32x32 MFMA tiles per wavefront
-    constexpr int WTM = BM / WM, WTN = BN / WN;           // wavefront tile
-    // in 32-bit words; bf16 sources with k contiguous keep rows of BK/2 + 4 words
-    constexpr int SQ = BK / 2 + 4;
-    // fp32 row strides of the LDS tiles (see TileLoader)
-    constexpr int RSA = BM + (TA ? FPAD_K : PAD), RSB = BN + (TB ? PAD : FPAD_K);
-    constexpr int LDS_A = BF16 == 2 && TA ? BM * SQ : (BF16 ? (BK / 2) * (BM + PAD) : BK * RSA);
-    constexpr int LDS_B = BF16 == 2 && !TB ? BN * SQ : (BF16 ? (BK / 2) * (BN + PAD) : BK * RSB);
-    static_assert(KW == 1 || BM * BN <= 2 * (LDS_A + LDS_B), "accumulator hand-over must fit in the tile buffers");
-    // tile buffers above the 64 KiB a static array may take come from the
-    // launch's dynamic allocation instead
-    constexpr bool BIG_LDS = 2 * (LDS_A + LDS_B) * 4 > 65536;
-    __shared__ __attribute__((aligned(16))) float smem_static[BIG_LDS ? 4 : 2 * (LDS_A + LDS_B)];
-    extern __shared__ __attribute__((aligned(16))) float smem_dynamic[];
-    float *const smem = BIG_LDS ? smem_dynamic : smem_static;
-
-    const int t = threadIdx.x, lane = t & 63;
-    const int kg = (t >> 6) / (WM * WN), wave = (t >> 6) % (WM * WN);
-    const int wm = wave % WM, wn = wave / WM;
-
     // XCD-aware tile order: the hardware deals consecutive workgroup ids round
     // robin over the 8 XCDs; give each XCD a contiguous run of tiles so tiles
     // that share an A/B panel also share an L2.
     int bid = blockIdx.x;
-    // second k range of a grouped problem: k tiles from k1 on read A2 / B2
-    const float *A2 = nullptr, *B2 = nullptr;
-    int k1 = 0x7fffffff;
+    A2 = B2 = nullptr;
+    k1 = 0x7fffffff;
     if (g.grp) {
         // grouped launch: consecutive workgroup ids go to the XCDs in turn; hand each XCD
         // GC consecutive tiles of the list at a time (neighbours in a tile column, which share
@@ -935,7 +820,6 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
     // Tile order inside an XCD's run: bands of gm tile rows, column by column
     // inside a band, so the workgroups in flight on one XCD form a block about
     // as wide as it is tall and share both A and B panels in that XCD's L2.
-    int tile_m, tile_n;
     if (g.gm > 1) {
         const int band = g.gm * g.tiles_n, bi = bid / band, first = bi * g.gm;
         const int rows = min(g.tiles_m - first, g.gm), r = bid - bi * band;
@@ -945,6 +829,364 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
         tile_m = bid % g.tiles_m;
         tile_n = bid / g.tiles_m;
     }
+}
+
+// f(0), f(1), ... with constants: arrays indexed by them stay in registers whatever the unroller's limits
+template <typename F, int... I>
+__device__ __forceinline__ void each_constant(F f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>()), ...);
+}
+
+// Products of operands that are bf16 in memory, staged by DMA: global memory to LDS without a
+// register in between, ST stages of 64 k in flight, so that a stage is asked for ST - 1 stages
+// before it is read and a wavefront's registers hold accumulators and fragments only (256 x 256
+// tiles fit).  The sums are those of every bf16 class: one chain of v_mfma_f32_32x32x16_bf16 over
+// k for each element, in increasing k.
+//
+// A stage holds each operand as it lies in memory, in units of 16 bytes.  k contiguous: rows of 64 k,
+// unit c of row i in place c ^ (i & 7), a fragment is one 16-byte read.  Long axis contiguous: rows
+// of one k, and a fragment is two transposing reads of 4 k x 16 each; 32-byte granules (16 values)
+// are stored in place q ^ f(k) so that the four rows of a read lie in different banks.  The
+// swizzles are applied to the global address, a DMA being linear in LDS.
+//
+// Bound by the matrix units and LDS together (a 128 x 64 wavefront tile reads 6 KB for 8 MFMAs) on
+// large shapes: 16384 x 1024 x 4096 227 us with register staging, 122 now (1.12 PFLOP/s); on small ones
+// by one memory round trip and the epilogue: 512 x 2048 x 512 6.8 -> 5.0 us.
+//
+// The stage of step it + 1 is waited for before the last quarter of step it, whose MFMAs cover the
+// barrier and the first fragment reads of the next; that barrier also says that stage it has
+// been read, and its place is refilled at once.
+constexpr int BOX_LD = 36; // words between the columns of an accumulator tile in LDS
+template <int BM, int BN, int WM, int WN, int ST, int TA, int TB>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
+{
+    GemmArgs g = g0;
+    constexpr int NT = 64 * WM * WN;
+    constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN), WTM = BM / WM, WTN = BN / WN;
+    constexpr int NVA = BM * 8 / NT, NVB = BN * 8 / NT, NL = NVA + NVB; // 16-byte loads a lane and stage
+    constexpr int STAGE = (BM + BN) * 64;
+    static_assert(NVA * NT == BM * 8 && NVB * NT == BN * 8, "whole loads");
+    static_assert(ST >= 2 && (ST - 1) * NL <= 63, "the memory counter has six bits");
+    static_assert(WM * WN * 32 * BOX_LD * 4 <= ST * STAGE * 2, "the epilogue's corners fit where the stages were");
+    extern __shared__ __attribute__((aligned(16))) uint16_t stages_lds[];
+    uint16_t NCHIP_LDS *const stages = (uint16_t NCHIP_LDS *)stages_lds;
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int wm = wave % WM, wn = wave / WM, hi = lane >> 5;
+
+    int tile_m, tile_n;
+    const float *A2, *B2;
+    int k1;
+    find_tile<BM, BN>(g, tile_m, tile_n, A2, B2, k1);
+    const int m0 = tile_m * BM, n0 = tile_n * BN, nk = g.K / 64, it2 = k1 / 64;
+
+    // this lane's byte offsets inside a stage's panel of an operand; rows and units past the edge
+    // repeat the last one (their results are not stored)
+    auto offsets = [&](auto &off, auto kcontig, auto extent, int64_t ld, int i0, int imax) {
+        constexpr int BT = decltype(extent)::value, NV = BT * 8 / NT;
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+            const int p = t + v * NT;
+            if constexpr (decltype(kcontig)::value) {
+                const int i = p / 8, row = i0 + i < imax ? i : imax - 1 - i0;
+                off[v] = (uint32_t)(2 * (row * ld + ((p & 7) ^ (i & 7)) * 8));
+            } else {
+                constexpr int U = BT / 8, SH = BT >= 128 ? 1 : 0;
+                const int k = p / U, u = p % U, i = (((u >> 1) ^ ((k & 3) << SH)) * 2 + (u & 1)) * 8;
+                off[v] = (uint32_t)(2 * (k * ld + (i0 + i + 8 <= imax ? i : imax - 8 - i0)));
+            }
+        }
+    };
+    uint32_t oa[NVA], ob[NVB];
+    // (a long axis that is no multiple of 8 lies in a copy whose columns are padded to one)
+    offsets(oa, std::integral_constant<bool, TA != 0>(), std::integral_constant<int, BM>(), g.lda, m0, TA ? g.M : (g.M + 7) & ~7);
+    offsets(ob, std::integral_constant<bool, TB == 0>(), std::integral_constant<int, BN>(), g.ldb, n0, TB ? (g.N + 7) & ~7 : g.N);
+    const int64_t ea = TA ? m0 * g.lda : m0, eb = TB ? n0 : n0 * g.ldb;
+    const int64_t sa = TA ? 64 : 64 * g.lda, sb = TB ? 64 * g.ldb : 64; // elements from stage to stage
+    const uint16_t *pa = reinterpret_cast<const uint16_t *>(g.A) + ea, *pb = reinterpret_cast<const uint16_t *>(g.B) + eb;
+    int to = 0, asked = 0; // where the next stage goes, its number
+    auto issue = [&]() {
+        if (asked == it2) {
+            pa = reinterpret_cast<const uint16_t *>(A2) + ea;
+            pb = reinterpret_cast<const uint16_t *>(B2) + eb;
+        }
+        uint16_t NCHIP_LDS *dst = stages + to * STAGE + wave * 512;
+#pragma unroll
+        for (int v = 0; v < NVA; v++) lds_dma16(dst + v * NT * 8, pa, oa[v]);
+#pragma unroll
+        for (int v = 0; v < NVB; v++) lds_dma16(dst + BM * 64 + v * NT * 8, pb, ob[v]);
+        pa += sa; pb += sb;
+        asked++;
+        to = to + 1 < ST ? to + 1 : 0;
+    };
+
+    // fragments of quarter u of a stage's panel: offsets of lane and tile, then constants
+    auto fragment = [&](const uint16_t NCHIP_LDS *panel, auto kcontig, auto extent, int at, int j, int u) -> u32x4 {
+        constexpr int BT = decltype(extent)::value;
+        if constexpr (decltype(kcontig)::value) {
+            return *reinterpret_cast<const u32x4 NCHIP_LDS *>(panel + (at + j * 32 + (lane & 31)) * 64 + (((u * 2 + hi) ^ (lane & 7)) * 8));
+        } else {
+            constexpr int SH = BT >= 128 ? 1 : 0;
+            const int k = u * 16 + hi * 8 + ((lane & 15) >> 2);
+            const int q = (at / 16 + j * 2 + ((lane >> 4) & 1)) ^ ((k & 3) << SH);
+            const uint16_t NCHIP_LDS *r = panel + k * BT + q * 16 + (lane & 3) * 4;
+            const uint2 lo = lds_read_columns(r), up = lds_read_columns(r + 4 * BT);
+            return u32x4{ lo.x, lo.y, up.x, up.y };
+        }
+    };
+    floatx16 acc[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; i++)
+#pragma unroll
+        for (int j = 0; j < TM; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+    u32x4 fa[2][TM], fb[2][TN];
+    auto fetch = [&](int stage, int u, int set) {
+        const uint16_t NCHIP_LDS *s = stages + stage * STAGE;
+#pragma unroll
+        for (int j = 0; j < TM; j++)
+            fa[set][j] = fragment(s, std::integral_constant<bool, TA != 0>(), std::integral_constant<int, BM>(), wm * WTM, j, u);
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+            fb[set][i] = fragment(s + BM * 64, std::integral_constant<bool, TB == 0>(), std::integral_constant<int, BN>(), wn * WTN, i, u);
+    };
+    auto multiply = [&](int set) {
+        typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+#pragma unroll
+            for (int j = 0; j < TM; j++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fb[set][i]),
+                                                                    __builtin_bit_cast(bf16x8, fa[set][j]), acc[i][j], 0, 0, 0);
+    };
+    // waits until `younger` stages, at most ST - 2, are in flight
+    auto arrive = [&](int younger) {
+        if (ST > 2 && younger >= ST - 2) { lds_dma_barrier<(ST - 2) * NL>(); return; }
+        if (ST > 3 && younger == 1) { lds_dma_barrier<NL>(); return; }
+        if (ST > 4 && younger == 2) { lds_dma_barrier<2 * NL>(); return; }
+        if (ST > 5 && younger == 3) { lds_dma_barrier<3 * NL>(); return; }
+        lds_dma_barrier<0>(); // (from here on: everything)
+    };
+
+#pragma unroll
+    for (int s = 0; s < ST; s++)
+        if (s < nk) issue();
+    // (with fewer stages than ST all of them are waited for)
+    if (nk >= ST) lds_dma_barrier<(ST - 1) * NL>(); else lds_dma_barrier<0>();
+    fetch(0, 0, 0);
+    int at = 0; // the stage being read
+    auto body = [&](auto more, int it) {
+#pragma unroll
+        for (int u = 0; u < 3; u++) {
+            fetch(at, u + 1, (u + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(u & 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (decltype(more)::value) lds_dma_barrier<(ST - 2) * NL>();
+        else arrive(nk - 2 - it);
+        at = at + 1 < ST ? at + 1 : 0;
+        if (decltype(more)::value) issue();
+        fetch(at, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int it = 0;
+    for (; it + ST < nk; it++) body(std::true_type(), it);
+    for (; it + 1 < nk; it++) body(std::false_type(), it);
+    fetch(at, 1, 1);
+    multiply(0);
+    fetch(at, 2, 0);
+    multiply(1);
+    fetch(at, 3, 1);
+    multiply(0);
+    multiply(1);
+
+    // Epilogue.  Every 32 x 32 accumulator tile passes through a corner of LDS (the stages are dead)
+    // so that a lane holds four consecutive rows m of columns nl, nl + 8, nl + 16, nl + 24 and moves
+    // them 16 bytes at a time, and what the next tile reads is on its way while this one is
+    // finished: a tile that loads, computes and stores alone is a memory round trip of its own.
+    lds_dma_barrier<0>();
+    float NCHIP_LDS *const box = (float NCHIP_LDS *)stages + wave * (32 * BOX_LD);
+    const int ml = (lane & 7) * 4, nl = lane >> 3;
+    const bool full = (m0 + BM <= g.M) && (n0 + BN <= g.N); // uniform
+    const bool wide = ((g.M | g.ldc) & 3) == 0 && (((uintptr_t)g.C | (uintptr_t)g.pre | (uintptr_t)g.add | (uintptr_t)g.dpre | (uintptr_t)g.bias | (uintptr_t)g.rowsum | (uintptr_t)(2 * (uintptr_t)g.c16)) & 15) == 0;
+    // what a tile reads besides its accumulators: beta C or the addend (never both), else the
+    // pre-activation (with an addend that one is read where it is used)
+    const float *const first = g.beta != 0.0f ? g.C : g.add, *const operand = first ? first : g.dpre;
+    floatx4 next[4], bias_next;
+    auto load4 = [&](const float *p, int64_t at, int left) -> floatx4 { // left: rows of the matrix from here on
+        floatx4 v = { 0.0f, 0.0f, 0.0f, 0.0f };
+        if (left <= 0) return v;
+        if (wide) return *reinterpret_cast<const floatx4 NCHIP_GLOBAL *>(as_global(p) + at);
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = e < left ? as_global(p)[at + e] : 0.0f;
+        return v;
+    };
+    auto store4 = [&](float *p, int64_t at, int left, const floatx4 &v) {
+        if (wide) { *reinterpret_cast<floatx4 NCHIP_GLOBAL *>(as_global(p) + at) = v; return; }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (e < left) as_global(p)[at + e] = v[e];
+    };
+    auto ask = [&](int tile) {
+        const int m = m0 + wm * WTM + tile % TM * 32 + ml, nb = n0 + wn * WTN + tile / TM * 32 + nl;
+        if (g.bias) bias_next = load4(g.bias, m, g.M - m);
+        if (operand) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) next[q] = load4(operand, (int64_t)(nb + 8 * q) * g.ldc + m, full || nb + 8 * q < g.N ? g.M - m : 0);
+        }
+    };
+    bias_next = floatx4{ 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+    for (int q = 0; q < 4; q++) next[q] = bias_next;
+    ask(0);
+#pragma unroll 1
+    for (int tile = 0; tile < TM * TN; tile++) { // (one copy of this code: unrolled it would not fit the instruction cache)
+        each_constant([&](auto index) {
+            constexpr int t0 = decltype(index)::value;
+            if (tile == t0) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) box[((r >> 2) * 8 + (r & 3) + hi * 4) * BOX_LD + (lane & 31)] = acc[t0 / TM][t0 % TM][r];
+            }
+        }, std::make_integer_sequence<int, TM * TN>());
+        __builtin_amdgcn_wave_barrier();
+        floatx4 x[4], y[4];
+        const floatx4 bv = bias_next;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            x[q] = *reinterpret_cast<const floatx4 NCHIP_LDS *>(box + (nl + 8 * q) * BOX_LD + ml);
+            y[q] = next[q];
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (tile + 1 < TM * TN) ask(tile + 1);
+        const int m = m0 + wm * WTM + tile % TM * 32 + ml, nb = n0 + wn * WTN + tile / TM * 32 + nl;
+        int left[4];
+        const int64_t at0 = (int64_t)nb * g.ldc + m;
+        auto at = [&](int q) { return at0 + 8 * q * g.ldc; };
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            left[q] = full || nb + 8 * q < g.N ? g.M - m : 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                x[q][e] = g.alpha * x[q][e];
+                if (g.beta != 0.0f) x[q][e] += g.beta * y[q][e];
+                x[q][e] += bv[e];
+            }
+        }
+        if (g.pre) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                if (left[q] > 0) store4(g.pre, at(q), left[q], x[q]);
+        }
+        if (g.act == ACT_GELU_FAST) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[q][e] = nchip_gelu_fast(x[q][e]);
+        } else if (g.act == NCHIP_ACT_RELU) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[q][e] = x[q][e] > 0.0f ? x[q][e] : 0.0f;
+        }
+        if (g.add) {
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[q][e] += y[q][e];
+        }
+        if (g.dpre) { // gradient through an activation: times act'(pre-activation)
+            if (first) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) y[q] = load4(g.dpre, at(q), left[q]);
+            }
+            if (g.dact == ACT_GELU_FAST) {
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[q][e] *= nchip_gelu_grad_fast(y[q][e]);
+            } else if (g.dact == NCHIP_ACT_RELU) {
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) x[q][e] *= y[q][e] > 0.0f ? 1.0f : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (left[q] > 0) store4(g.C, at(q), left[q], x[q]);
+        if (g.c16) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                uint16_t NCHIP_GLOBAL *h = as_global(g.c16) + at(q);
+                if (wide && left[q] > 0) {
+                    *reinterpret_cast<uint2 NCHIP_GLOBAL *>(h) = make_uint2(pack_bf16(x[q][0], x[q][1]), pack_bf16(x[q][2], x[q][3]));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (e < left[q]) h[e] = f32_to_bf16_rne(x[q][e]);
+                }
+            }
+        }
+        if (g.rowsum) { // one partial row per half of the tile's columns (n % 8 below 4, from 4 on)
+            floatx4 sum = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) sum[e] += left[q] > 0 ? x[q][e] : 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                sum[e] += __shfl_xor(sum[e], 8, 64);
+                sum[e] += __shfl_xor(sum[e], 16, 64);
+            }
+            if ((lane & 24) == 0 && m < g.M)
+                store4(g.rowsum, (int64_t)(((tile_n * WN + wn) * TN + tile / TM) * 2 + hi) * g.M + m, g.M - m, sum);
+        }
+    }
+}
+
+// KW = 2 doubles the wavefronts of a workgroup without shrinking its tile: the
+// two groups of WM x WN wavefronts share the LDS tiles and split every 32-deep
+// k slab, group 0 taking k%32 < 16 and group 1 the rest; group 1 hands its
+// accumulators over through LDS at the end (C = chain0 + chain1, fixed order).
+// NACC = 2 (the width-invariant class): each k group keeps two accumulator sets and gives
+// the first four MFMA steps of every 32-deep slab to one, the last four to the other, so a
+// product is four chains - chain c takes k%32 in [8c, 8c+8) - summed as (c0 + c1) + (c2 + c3).
+// The products are the same; the order of the additions is what a kernel with four
+// wavefronts per row tile can reproduce (gemm_skinny_nn).
+template <int BM, int BN, int BK, int WM, int WN, int TA, int TB, int BF16, int KW = 1, int PF = 2, int NACC = 1, int FRAG = 0>
+__global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
+{
+    GemmArgs g = g0;
+    static_assert(NACC == 1 || (NACC == 2 && BF16 == 0 && KW == 2 && BK == 32), "two accumulator sets: fp32 64-wide class only");
+    static_assert(KW == 1 || (KW == 2 && BK % 32 == 0), "k groups split 32-deep slabs");
+    constexpr int NT = 64 * WM * WN * KW;                 // threads: KW groups of WM x WN wavefronts
+    constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN); // 32x32 MFMA tiles per wavefront
+    constexpr int WTM = BM / WM, WTN = BN / WN;           // wavefront tile
+    // fp32 row strides of the LDS tiles (see TileLoader)
+    constexpr int RSA = BM + (TA ? FPAD_K : PAD), RSB = BN + (TB ? PAD : FPAD_K);
+    constexpr int LDS_A = BF16 ? (BK / 2) * (BM + PAD) : BK * RSA; // in 32-bit words
+    constexpr int LDS_B = BF16 ? (BK / 2) * (BN + PAD) : BK * RSB;
+    static_assert(KW == 1 || BM * BN <= 2 * (LDS_A + LDS_B), "accumulator hand-over must fit in the tile buffers");
+    // tile buffers above the 64 KiB a static array may take come from the
+    // launch's dynamic allocation instead
+    constexpr bool BIG_LDS = 2 * (LDS_A + LDS_B) * 4 > 65536;
+    __shared__ __attribute__((aligned(16))) float smem_static[BIG_LDS ? 4 : 2 * (LDS_A + LDS_B)];
+    extern __shared__ __attribute__((aligned(16))) float smem_dynamic[];
+    float *const smem = BIG_LDS ? smem_dynamic : smem_static;
+
+    const int t = threadIdx.x, lane = t & 63;
+    const int kg = (t >> 6) / (WM * WN), wave = (t >> 6) % (WM * WN);
+    const int wm = wave % WM, wn = wave / WM;
+
+    int tile_m, tile_n;
+    // second k range of a grouped problem: k tiles from k1 on read A2 / B2
+    const float *A2, *B2;
+    int k1;
+    find_tile<BM, BN>(g, tile_m, tile_n, A2, B2, k1);
     const int bz = blockIdx.y;
     const int b = bz / g.ksplit, kz = bz % g.ksplit;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
@@ -956,18 +1198,15 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
     const float *B = g.B + (int64_t)b_out * g.sb + (int64_t)b_in * g.sb_in;
 
     // fast (vector, unguarded) loads need whole tiles and 16-byte alignment
-    // (bf16 sources are padded and aligned by construction: always fast)
-    const bool a_full = BF16 == 2 || ((m0 + BM <= g.M) && (g.lda % 4 == 0) && (((uintptr_t)A & 15) == 0));
-    const bool b_full = BF16 == 2 || ((n0 + BN <= g.N) && (g.ldb % 4 == 0) && (((uintptr_t)B & 15) == 0));
+    const bool a_full = (m0 + BM <= g.M) && (g.lda % 4 == 0) && (((uintptr_t)A & 15) == 0);
+    const bool b_full = (n0 + BN <= g.N) && (g.ldb % 4 == 0) && (((uintptr_t)B & 15) == 0);
 
     // PF register sets: while tile it is computed, tiles it+1 .. it+PF are landing
     // or in flight, so a load has PF compute phases to arrive.  Two sets are
     // enough for the wide classes; the 64x64 class, whose tiles are consumed in
     // half the time, keeps four.
-    using LoaderA = std::conditional_t<BF16 == 2, TileLoaderBf16Src<BM, BK, TA ? 0 : 1, NT>,
-                    std::conditional_t<BF16 == 1, TileLoaderBf16<BM, BK, TA ? 0 : 1, NT>, TileLoader<BM, BK, TA ? 0 : 1, NT>>>;
-    using LoaderB = std::conditional_t<BF16 == 2, TileLoaderBf16Src<BN, BK, TB ? 1 : 0, NT>,
-                    std::conditional_t<BF16 == 1, TileLoaderBf16<BN, BK, TB ? 1 : 0, NT>, TileLoader<BN, BK, TB ? 1 : 0, NT>>>;
+    using LoaderA = std::conditional_t<BF16 == 1, TileLoaderBf16<BM, BK, TA ? 0 : 1, NT>, TileLoader<BM, BK, TA ? 0 : 1, NT>>;
+    using LoaderB = std::conditional_t<BF16 == 1, TileLoaderBf16<BN, BK, TB ? 1 : 0, NT>, TileLoader<BN, BK, TB ? 1 : 0, NT>>;
     LoaderA la[PF];
     LoaderB lb[PF];
 
@@ -999,23 +1238,13 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
                 u32x4 fa[TM], fb[TN];
 #pragma unroll
                 for (int j = 0; j < TM; j++) {
-                    if constexpr (BF16 == 2 && TA != 0) { // k-contiguous rows: one 16-byte read
-                        fa[j] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint32_t *>(sa) +
-                                (wm * WTM + j * 32 + (lane & 31)) * SQ + row0 + (lane >> 5) * 4);
-                    } else {
-                        const uint32_t *q = wa + row0 * (BM + PAD) + j * 32;
-                        fa[j] = u32x4{ q[0], q[BM + PAD], q[2 * (BM + PAD)], q[3 * (BM + PAD)] };
-                    }
+                    const uint32_t *q = wa + row0 * (BM + PAD) + j * 32;
+                    fa[j] = u32x4{ q[0], q[BM + PAD], q[2 * (BM + PAD)], q[3 * (BM + PAD)] };
                 }
 #pragma unroll
                 for (int i = 0; i < TN; i++) {
-                    if constexpr (BF16 == 2 && TB == 0) {
-                        fb[i] = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint32_t *>(sb) +
-                                (wn * WTN + i * 32 + (lane & 31)) * SQ + row0 + (lane >> 5) * 4);
-                    } else {
-                        const uint32_t *q = wb + row0 * (BN + PAD) + i * 32;
-                        fb[i] = u32x4{ q[0], q[BN + PAD], q[2 * (BN + PAD)], q[3 * (BN + PAD)] };
-                    }
+                    const uint32_t *q = wb + row0 * (BN + PAD) + i * 32;
+                    fb[i] = u32x4{ q[0], q[BN + PAD], q[2 * (BN + PAD)], q[3 * (BN + PAD)] };
                 }
 #pragma unroll
                 for (int i = 0; i < TN; i++)
@@ -1138,79 +1367,6 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
 #endif
     const int nk = (kend - kbeg + BK - 1) / BK;
     const int nk_full = (kend - kbeg) / BK; // tiles with a complete k range
-    if constexpr (SA != 0) {
-        // Store-ahead order: the LDS writes of the next tile go out BEFORE the
-        // MFMAs of the current one (into the other buffer, which every
-        // wavefront left at the last barrier) and overlap with them; one
-        // barrier per tile, after the MFMAs.  Register set (i % PF) holds tile
-        // i from its load until that write; it is reloaded with tile i + PF
-        // right after.
-        auto fetch = [&](int tile, auto fast_tag, auto &la, auto &lb) {
-            constexpr bool FAST = decltype(fast_tag)::value;
-            const int k0 = kbeg + tile * BK;
-            const bool kf = FAST || (k0 + BK <= kend);
-            const bool second = k0 >= k1; // uniform
-            const float *Ak = second ? A2 : A, *Bk = second ? B2 : B;
-            const int kr = second ? k0 - k1 : k0, ke = second ? kend - k1 : (kend < k1 ? kend : k1);
-            la.load(Ak, g.lda, m0, kr, g.M, ke, FAST || (a_full && kf), t);
-            lb.load(Bk, g.ldb, n0, kr, g.N, ke, FAST || (b_full && kf), t);
-        };
-        auto park = [&](int tile, auto &la, auto &lb) {
-            float *sa = smem + (tile & 1) * (LDS_A + LDS_B);
-            if constexpr (BF16 != 0) {
-                la.store(reinterpret_cast<uint32_t *>(sa), t);
-                lb.store(reinterpret_cast<uint32_t *>(sa + LDS_A), t);
-            } else {
-                la.store_f32(sa, t);
-                lb.store_f32(sa + LDS_A, t);
-            }
-        };
-        auto body = [&](int cur, auto fast_tag, auto &na, auto &nb) {
-            constexpr bool FAST = decltype(fast_tag)::value;
-            if (FAST || cur + 1 < nk) {
-                park(cur + 1, na, nb);
-                if (FAST || cur + 1 + PF < nk) fetch(cur + 1 + PF, fast_tag, na, nb);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            const float *sa = smem + (cur & 1) * (LDS_A + LDS_B);
-            compute(sa, sa + LDS_A);
-            __syncthreads();
-        };
-        int it = 0;
-        if (a_full && b_full && 2 * PF < nk_full) {
-            // Steady state: every tile fetched here is complete.  The first PF + 1 tiles are
-            // fetched by the same straight-line sequence as inside the loop, with nothing
-            // conditional between them and the loop: the compiler then sees one and the same
-            // queue of outstanding loads on entry and on the back edge and waits for the
-            // oldest register set only (s_waitcnt vmcnt(n)).  With a conditional fetch in
-            // front of the loop it assumes the worst path and drains every load in flight at
-            // the top of each trip - which is what the prefetch is there to avoid.
-#pragma unroll
-            for (int j = 0; j < PF; j++) {
-                fetch(j, std::true_type(), la[j], lb[j]);
-                __builtin_amdgcn_sched_barrier(0); // oldest tile first, as on the back edge
-            }
-            park(0, la[0], lb[0]);
-            fetch(PF, std::true_type(), la[0], lb[0]);
-            __syncthreads();
-            for (; it + 2 * PF < nk_full; it += PF) {
-#pragma unroll
-                for (int j = 0; j < PF; j++) body(it + j, std::true_type(), la[(j + 1) % PF], lb[(j + 1) % PF]);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < PF; j++)
-                if (j < nk) fetch(j, std::false_type(), la[j], lb[j]);
-            if (nk > 0) park(0, la[0], lb[0]);
-            if (PF < nk) fetch(PF, std::false_type(), la[0], lb[0]);
-            __syncthreads();
-        }
-        for (; it < nk; it += PF) {
-#pragma unroll
-            for (int j = 0; j < PF; j++)
-                if (it + j < nk) body(it + j, std::false_type(), la[(j + 1) % PF], lb[(j + 1) % PF]);
-        }
-    } else {
     int it = 0;
     if (a_full && b_full && 2 * PF - 1 < nk_full) {
         // steady state: tiles it+PF .. it+2PF-1 are complete, unguarded vector loads.  The
@@ -1241,7 +1397,6 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
 #pragma unroll
         for (int j = 0; j < PF; j++)
             if (it % PF == j) step(it, nk, std::false_type(), la[j], lb[j]);
-    }
     }
 
 #ifdef NCHIP_GEMM_CLOCKS
@@ -1601,15 +1756,14 @@ int g_bf16ops_cls = getenv("NCHIP_GEMM_BF16OPS_CLASS") ? atoi(getenv("NCHIP_GEMM
 template <int BM, int BN, int BK, int TA, int TB, int BF16>
 constexpr size_t lds_dynamic_bytes()
 {
-    constexpr int SQ = BK / 2 + 4;
-    constexpr size_t a = BF16 == 2 && TA ? BM * SQ : (BF16 ? (BK / 2) * (BM + PAD) : BK * (BM + (TA ? FPAD_K : PAD)));
-    constexpr size_t b = BF16 == 2 && !TB ? BN * SQ : (BF16 ? (BK / 2) * (BN + PAD) : BK * (BN + (TB ? PAD : FPAD_K)));
+    constexpr size_t a = BF16 ? (BK / 2) * (BM + PAD) : BK * (BM + (TA ? FPAD_K : PAD));
+    constexpr size_t b = BF16 ? (BK / 2) * (BN + PAD) : BK * (BN + (TB ? PAD : FPAD_K));
     constexpr size_t bytes = 2 * (a + b) * sizeof(float);
     static_assert(bytes <= 160 * 1024, "tile buffers exceed LDS");
     return bytes > 65536 ? bytes : 0;
 }
 
-template <int BM, int BN, int BK, int WM, int WN, int BF16, int KW = 1, int PF = 2, int SA = (BF16 == 2), int NACC = 1, int FRAG = 0>
+template <int BM, int BN, int BK, int WM, int WN, int BF16, int KW = 1, int PF = 2, int NACC = 1, int FRAG = 0>
 void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec)
 {
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -1622,19 +1776,75 @@ void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec)
         constexpr size_t dyn = lds_dynamic_bytes<BM, BN, BK, TA, TB, BF16>();                              \
         if (dyn) {                                                                                         \
             static const bool ok = hipFuncSetAttribute(                                                    \
-                reinterpret_cast<const void *>(gemm_kernel<BM, BN, BK, WM, WN, TA, TB, BF16, KW, PF, SA, NACC, FRAG>),     \
+                reinterpret_cast<const void *>(gemm_kernel<BM, BN, BK, WM, WN, TA, TB, BF16, KW, PF, NACC, FRAG>),     \
                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn) == hipSuccess;                       \
             if (!ok) { fprintf(stderr, "nchip_gemm: cannot reserve %zu bytes of LDS\n", dyn); abort(); }  \
         }                                                                                                  \
-        if (rec) hipExtLaunchKernelGGL((gemm_kernel<BM, BN, BK, WM, WN, TA, TB, BF16, KW, PF, SA, NACC, FRAG>), grid, block, dyn, \
+        if (rec) hipExtLaunchKernelGGL((gemm_kernel<BM, BN, BK, WM, WN, TA, TB, BF16, KW, PF, NACC, FRAG>), grid, block, dyn, \
                                        st, rec->start, rec->stop, 0, g);                                   \
-        else hipLaunchKernelGGL((gemm_kernel<BM, BN, BK, WM, WN, TA, TB, BF16, KW, PF, SA, NACC, FRAG>), grid, block, dyn, st, g); \
+        else hipLaunchKernelGGL((gemm_kernel<BM, BN, BK, WM, WN, TA, TB, BF16, KW, PF, NACC, FRAG>), grid, block, dyn, st, g); \
     } while (0)
     if (!ta && !tb) LAUNCH(0, 0);
     else if (ta && !tb) LAUNCH(1, 0);
     else if (!ta && tb) LAUNCH(0, 1);
     else LAUNCH(1, 1);
 #undef LAUNCH
+}
+
+template <int BM, int BN, int WM, int WN, int ST>
+void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int grouped_tiles = 0)
+{
+    g.tiles_m = (g.M + BM - 1) / BM;
+    g.tiles_n = (g.N + BN - 1) / BN;
+    g.gm = g_force_gm >= 0 ? g_force_gm : 8;
+    constexpr size_t dyn = (size_t)(BM + BN) * 64 * 2 * ST;
+    static_assert(dyn <= 160 * 1024, "stages exceed LDS");
+    dim3 grid(grouped_tiles ? grouped_tiles : g.tiles_m * g.tiles_n), block(64 * WM * WN);
+#define LAUNCH(TA, TB)                                                                                     \
+    do {                                                                                                   \
+        static const bool ok = hipFuncSetAttribute(                                                        \
+            reinterpret_cast<const void *>(gemm_dma_kernel<BM, BN, WM, WN, ST, TA, TB>),                    \
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn) == hipSuccess;                           \
+        if (!ok) { fprintf(stderr, "nchip_gemm: cannot reserve %zu bytes of LDS\n", dyn); abort(); }      \
+        if (rec) hipExtLaunchKernelGGL((gemm_dma_kernel<BM, BN, WM, WN, ST, TA, TB>), grid, block, dyn, st, rec->start, rec->stop, 0, g); \
+        else hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, WM, WN, ST, TA, TB>), grid, block, dyn, st, g);   \
+    } while (0)
+    if (!ta && !tb) LAUNCH(0, 0);
+    else if (ta && !tb) LAUNCH(1, 0);
+    else if (!ta && tb) LAUNCH(0, 1);
+    else LAUNCH(1, 1);
+#undef LAUNCH
+}
+
+// Tile class of a product of bf16 operands, from the tile counts.  One 256 x 256 tile fills a CU
+// (128 KB of stages, 256 registers): it is taken when its rounds of 256 workgroups are at least
+// seven eighths full; below that two workgroups of 128 x 128 and two stages share a CU as long as
+// there are that many; a single round gets 8 wavefronts a tile and four stages; then smaller tiles
+// until the chip is covered.  Measured, us (m x n x k; classes 4 / 1 / 5 / 2 / 3; before = tiles
+// staged through registers, best class):
+//   16384 x 4096 x 1024   155 / 162 / 207 / 197 / 246   before 204
+//   4096 x 4096 x 1024     44 /  46 /  59 /  58 /  69   before  56
+//   2048 x 4096 x 1024     32 /  24 /  29 /  31 /  36   before  31
+//   1024 x 4096 x 4096     96 /  59 /  43 /  53 /  64   before  52
+//   1024 x 2048 x 3072     71 /  39 /  30 /  24 /  28   before  33
+//   512 x 2048 x 2048      47 /  21 /  19 /  13 /  10   before  13
+static int dma_class(int m, int n)
+{
+    auto tiles = [&](int bm, int bn) { return (int64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
+    const int64_t t256 = tiles(256, 256), t128 = tiles(128, 128);
+    if (8 * t256 >= 7 * 256 * ((t256 + 255) / 256)) return 4;
+    if (t128 >= 448) return 1;
+    if (t128 >= 224) return 5;
+    return tiles(128, 64) >= 224 && m >= 128 ? 2 : 3;
+}
+
+static void launch_dma_class(hipStream_t st, int cls, int ta, int tb, GemmArgs &g, ProfRec *rec)
+{
+    if (cls == 4) launch_dma<256, 256, 2, 4, 2>(st, ta, tb, g, rec);
+    else if (cls == 1) launch_dma<128, 128, 2, 2, 2>(st, ta, tb, g, rec);
+    else if (cls == 5) launch_dma<128, 128, 2, 4, 4>(st, ta, tb, g, rec);
+    else if (cls == 2) launch_dma<128, 64, 2, 2, 3>(st, ta, tb, g, rec);
+    else launch_dma<64, 64, 2, 2, 4>(st, ta, tb, g, rec);
 }
 
 template <int NW, int PF, int SPLIT>
@@ -1800,8 +2010,6 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     g.alpha = alpha; g.beta = beta; g.act = act_for_precision(act, precision);
     g.grp = nullptr; g.n_grp = 0;
     hipStream_t st = (hipStream_t)stream;
-    // tile choice from the shape only: large tiles when they still fill the chip
-    int64_t t128 = (int64_t)((m + 127) / 128) * ((n + 127) / 128) * batch * ksplit;
     ProfRec rec;
     if (g_prof_on) {
         (void)hipEventCreate(&rec.start);
@@ -1849,7 +2057,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     // the ones the conversion inside the tile loader would produce, so the
     // result is the same either way.
     bool from_bf16 = false;
-    if (precision == 1 && batch == 1 && ksplit == 1 && !invariant &&
+    if (precision == 1 && batch == 1 && ksplit == 1 && !invariant && k > 0 &&
         (g_bf16src == 2 || (g_bf16src == 1 && m >= 128 && n >= 128 && k >= 256 &&
                             2.0 * m * n * (double)k >= g_bf16src_min_flops))) {
         const int kpad = (k + 63) / 64 * 64;
@@ -1874,13 +2082,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
         *rowsum_rows = (n + bn - 1) / bn * bn / 16;
     }
     if (from_bf16) {
-        // 64x64 per wavefront, 64-deep tiles: with enough tiles for two workgroups
-        // per CU four wavefronts each do best; below that, eight wavefronts in
-        // two k groups share one tile
-        const bool four = g_force_cfg == 13 || (g_force_cfg != 11 && g_force_cfg != 7 && t128 >= 512);
-        if (g_force_cfg == 7) launch_tile<128, 128, 32, 4, 2, 2>(st, ta, tb, g, pr);
-        else if (four) launch_tile<128, 128, 64, 2, 2, 2, 1>(st, ta, tb, g, pr);
-        else launch_tile<128, 128, 64, 2, 2, 2, 2>(st, ta, tb, g, pr);
+        launch_dma_class(st, dma_class(m, n), ta, tb, g, pr);
     } else if (precision == 1) {
         if (cfg == 7) launch_tile<128, 128, 32, 4, 2, 1>(st, ta, tb, g, pr);
         else if (cfg == 4) launch_tile<128, 64, 32, 4, 2, 1>(st, ta, tb, g, pr);
@@ -1907,7 +2109,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     } else if (cfg == 6) {
         launch_tile<64, 128, 16, 2, 2, 0>(st, ta, tb, g, pr);
     } else if (cfg == 7) {
-        launch_tile<128, 128, 32, 4, 2, 0, 1, 2, 0, 1, 1>(st, ta, tb, g, pr); // rolling fragment window: two accumulator tiles per wavefront
+        launch_tile<128, 128, 32, 4, 2, 0, 1, 2, 1, 1>(st, ta, tb, g, pr); // rolling fragment window: two accumulator tiles per wavefront
     } else if (cfg == 8) {
         launch_tile<64, 64, 32, 2, 2, 0, 2>(st, ta, tb, g, pr);
     } else if (cfg == 9) {
@@ -1915,7 +2117,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     } else if (cfg == 10) {
         launch_tile<64, 64, 32, 2, 2, 0, 2, 4>(st, ta, tb, g, pr);
     } else if (cfg == 30) { // the width-invariant class: four chains per element
-        launch_tile<64, 64, 32, 2, 2, 0, 2, 4, 0, 2>(st, ta, tb, g, pr);
+        launch_tile<64, 64, 32, 2, 2, 0, 2, 4, 2>(st, ta, tb, g, pr);
     } else {
         launch_tile<64, 64, 16, 2, 2, 0>(st, ta, tb, g, pr);
     }
@@ -1975,7 +2177,7 @@ extern "C" int nchip_gemm_dact(void *stream, int ta, int tb, int m, int n, int k
 // nchip_gemm_dact that also leaves partial row sums of C: rowsum holds nchip_gemm_rowsum_rows(n)
 // rows of m floats, of which *rows_written are written (row p = the sum over 16 columns of C;
 // 0 when this product's kernel does not write them: the caller then sums C itself)
-extern "C" int nchip_gemm_rowsum_rows(int n) { return (n + 127) / 128 * 8; }
+extern "C" int nchip_gemm_rowsum_rows(int n) { return (n + 255) / 256 * 16; } // (the widest tile's)
 
 extern "C" int nchip_gemm_dact_rowsum(void *stream, int ta, int tb, int m, int n, int k, float alpha,
                                       const float *A, int64_t lda, const float *B, int64_t ldb,
@@ -2135,9 +2337,8 @@ extern "C" int nchip_widen_bf16(void *stream, const uint16_t *src, float *dst, i
 // Product whose operands are already bf16 in memory (the rounded copies of the fp32 matrices,
 // element for element in the same column-major layout: no padding).  Unguarded 16-byte loads
 // throughout, so the shapes must fit: k a multiple of 64; an operand whose long axis is
-// contiguous (A with ta = 0, B with tb = 1) must fill whole tiles (m resp. n a multiple of
-// 128: every tile class divides it); leading dimensions multiples of 8 elements; 16-byte
-// aligned bases.  Returns 1 when they do not (nothing launched: the caller takes another
+// contiguous (A with ta = 0, B with tb = 1) a multiple of 64 along it; leading dimensions
+// multiples of 8 elements; 16-byte aligned bases.  Returns 1 when they do not (nothing launched: the caller takes another
 // route).  Epilogue options as in the fp32-operand calls; c16, when given, receives the
 // result rounded to bf16 next to C.
 extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a)
@@ -2149,7 +2350,7 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
         fprintf(stderr, "nchip_gemm_bf16_operands: bad arguments (m=%d n=%d k=%d)\n", m, n, k);
         return -1;
     }
-    if (k % 64 || a->lda % 8 || a->ldb % 8 || (((uintptr_t)a->A16 | (uintptr_t)a->B16) & 15) != 0)
+    if (k % 64 || a->lda % 8 || a->ldb % 8 || (!ta && m % 64) || (tb && n % 64) || (((uintptr_t)a->A16 | (uintptr_t)a->B16) & 15) != 0)
         return 1;
     GemmArgs g;
     memset(&g, 0, sizeof(g));
@@ -2160,17 +2361,9 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
     g.batch_in = 1; g.M = m; g.N = n; g.K = k; g.batch = 1; g.ksplit = 1; g.kchunk = k;
     g.alpha = a->alpha; g.beta = 0.0f; g.act = act_for_precision(a->act, 2);
     hipStream_t st = (hipStream_t)stream;
-    // tile class from the tile counts: the largest tile that still gives every CU a workgroup
-    const int64_t t128 = (int64_t)((m + 127) / 128) * ((n + 127) / 128);
-    const int64_t t128x64 = (int64_t)((m + 127) / 128) * ((n + 63) / 64);
-    int cls = g_bf16ops_cls;
-    if (cls < 1 || cls > 3) cls = t128 >= 224 ? 1 : (t128x64 >= 224 && m >= 128 ? 2 : 3);
-    {
-        const int bm = cls == 3 ? 64 : 128, bn = cls == 1 ? 128 : 64;
-        if ((!ta && m % bm) || (tb && n % bn)) return 1; // row-contiguous operands need whole tiles
-    }
+    const int cls = g_bf16ops_cls >= 1 && g_bf16ops_cls <= 5 ? g_bf16ops_cls : dma_class(m, n);
     if (a->rowsum && a->rows_written && a->dpre) {
-        const int bn = cls == 1 ? 128 : 64;
+        const int bn = cls == 4 ? 256 : (cls == 1 || cls == 5 ? 128 : 64);
         g.rowsum = a->rowsum;
         *a->rows_written = (n + bn - 1) / bn * bn / 16;
     }
@@ -2179,15 +2372,10 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
         (void)hipEventCreate(&rec.start);
         (void)hipEventCreate(&rec.stop);
         rec.flops = 2.0 * m * n * (double)k;
-        rec.variant = 32 + cls * 4 + ta * 2 + tb; // the bf16-operand classes
+        rec.variant = 64 + cls * 4 + ta * 2 + tb; // the bf16-operand classes
     }
     ProfRec *pr = g_prof_on ? &rec : nullptr;
-    // (measured on the C3 and C4 shapes: deeper prefetch - 3 or 4 register sets - changes nothing
-    // once the loop waits for its oldest set only; 256 x 128 tiles with 8 wavefronts run at the
-    // rate of the 128 x 128 class, 256 x 256 tiles spill)
-    if (cls == 1) launch_tile<128, 128, 64, 2, 2, 2, 1>(st, ta, tb, g, pr);
-    else if (cls == 2) launch_tile<128, 64, 64, 2, 2, 2, 1>(st, ta, tb, g, pr);
-    else launch_tile<64, 64, 64, 2, 2, 2, 1>(st, ta, tb, g, pr);
+    launch_dma_class(st, cls, ta, tb, g, pr);
     if (g_prof_on) g_prof.push_back(rec);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -2197,7 +2385,8 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
     return 0;
 }
 
-// tuning aid: 0 = choose the bf16-operand tile class from the shape, 1 = 128x128, 2 = 128x64, 3 = 64x64
+// tuning aid: 0 = choose the bf16-operand tile class from the shape, 1 = 128x128, 2 = 128x64, 3 = 64x64, 4 = 256x256,
+// 5 = 128x128 with 8 wavefronts
 extern "C" void nchip_gemm_bf16_operands_class(int cls) { g_bf16ops_cls = cls; }
 
 // ---- profiling entry points ---------------------------------------------------
@@ -2209,7 +2398,7 @@ extern "C" void nchip_gemm_profile_enable(int on)
 extern "C" int nchip_gemm_profile_read(int max_variants, char (*names)[48], int64_t *launches,
                                        double *flops, double *seconds)
 {
-    constexpr int NVAR = 64;
+    constexpr int NVAR = 88;
     double fl[NVAR] = { 0 }, sec[NVAR] = { 0 };
     int64_t cnt[NVAR] = { 0 };
     for (ProfRec &r : g_prof) {
@@ -2227,15 +2416,17 @@ extern "C" int nchip_gemm_profile_read(int max_variants, char (*names)[48], int6
     g_prof.clear();
     static const char *tiles_f32[4] = { "64,64,16,2,2", "128,64,32,4,2", "128,128,32,4,2", "64,64,32,2,2" };
     static const char *tiles_bf16[4] = { "64,64,32,2,2", "128,64,32,4,2", "128,128,32,4,2", "64,64,32,2,2" };
-    static const char *tiles_ops[4] = { "128,128,64,2,2", "128,128,64,2,2", "128,64,64,2,2", "64,64,64,2,2" }; // 0: the grouped launch
+    static const char *tiles_ops[6] = { "256,256,2,4,2", "128,128,2,2,2", "128,64,2,2,3", "64,64,2,2,4", "256,256,2,4,2", "128,128,2,4,4" }; // 0: grouped
     int n = 0;
     for (int v = 0; v < NVAR && n < max_variants; v++) {
         if (!cnt[v]) continue;
-        if (v >= 48) {
+        if (v >= 64) { // operands read as bf16: gemm_dma_kernel<tile, wavefronts, stages, ta, tb>
+            snprintf(names[n], 48, "gemm_dma_kernel<%s,%d,%d%s>", tiles_ops[(v - 64) / 4], (v >> 1) & 1, v & 1,
+                     v < 68 ? ",grouped" : "");
+        } else if (v >= 48) {
             snprintf(names[n], 48, "gemm_small_kernel<%d,%d>", (v >> 2) & 1, (v >> 1) & 1);
-        } else if (v >= 32) { // operands read as bf16: gemm_kernel<tile, ta, tb, 2>
-            snprintf(names[n], 48, "gemm_kernel<%s,%d,%d,2%s>", tiles_ops[(v - 32) / 4], (v >> 1) & 1, v & 1,
-                     v < 36 ? ",grouped" : "");
+        } else if (v >= 32) { // the grouped launch in 128 x 128 tiles
+            snprintf(names[n], 48, "gemm_dma_kernel<128,128,2,2,2,%d,%d,grouped>", (v >> 1) & 1, v & 1);
         } else {
             const bool two_groups = v / 8 == 3 || ((v & 1) && v / 8 == 0);
             snprintf(names[n], 48, "gemm_kernel<%s,%d,%d,%d%s>", (v & 1) ? tiles_bf16[v / 8] : tiles_f32[v / 8],
@@ -2253,6 +2444,11 @@ extern "C" int nchip_gemm_grouped_tiles(int m, int n)
     return ((m + 127) / 128) * ((n + 127) / 128);
 }
 
+extern "C" int nchip_gemm_grouped_tiles256(int m, int n)
+{
+    return ((m + 255) / 256) * ((n + 255) / 256);
+}
+
 extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmProblem *dev_table,
                                   int n_problems, int total_tiles, int precision, double total_flops)
 {
@@ -2267,12 +2463,12 @@ extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmP
     g.batch = 1; g.batch_in = 1; g.ksplit = 1;
     g.beta = 0.0f; g.act = 0;
     hipStream_t st = (hipStream_t)stream;
-    dim3 grid(total_tiles, 1), block(precision == 2 ? 256 : 512);
+    dim3 grid(total_tiles, 1), block(512);
     ProfRec rec;
     if (g_prof_on) {
         (void)hipEventCreate(&rec.start);
         (void)hipEventCreate(&rec.stop);
-        rec.variant = precision == 2 ? 32 + (ta ? 2 : 0) + (tb ? 1 : 0)
+        rec.variant = precision >= 2 ? (precision == 3 ? 64 : 32) + (ta ? 2 : 0) + (tb ? 1 : 0)
                                      : 2 * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 1 ? 1 : 0);
         rec.flops = total_flops;
     }
@@ -2287,17 +2483,17 @@ extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmP
         if (g_prof_on) hipExtLaunchKernelGGL(KERNEL, grid, block, dyn, st, rec.start, rec.stop, 0, g);     \
         else hipLaunchKernelGGL(KERNEL, grid, block, dyn, st, g);                                          \
     } while (0)
-#define GRP(TA, TB, BF) GRP_LAUNCH((gemm_kernel<128, 128, 32, 4, 2, TA, TB, BF, 1, 2, 0, 1, (BF == 0)>), 32, TA, TB, BF)
-#define GRP16(TA, TB) GRP_LAUNCH((gemm_kernel<128, 128, 64, 2, 2, TA, TB, 2, 1>), 64, TA, TB, 2)
-    if (precision == 2) {
-        if (!ta && !tb) GRP16(0, 0); else if (ta && !tb) GRP16(1, 0); else if (!ta && tb) GRP16(0, 1); else GRP16(1, 1);
+#define GRP(TA, TB, BF) GRP_LAUNCH((gemm_kernel<128, 128, 32, 4, 2, TA, TB, BF, 1, 2, 1, (BF == 0)>), 32, TA, TB, BF)
+    if (precision == 3) {
+        launch_dma<256, 256, 2, 4, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+    } else if (precision == 2) {
+        launch_dma<128, 128, 2, 2, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
     } else if (precision == 1) {
         if (!ta && !tb) GRP(0, 0, 1); else if (ta && !tb) GRP(1, 0, 1); else if (!ta && tb) GRP(0, 1, 1); else GRP(1, 1, 1);
     } else {
         if (!ta && !tb) GRP(0, 0, 0); else if (ta && !tb) GRP(1, 0, 0); else if (!ta && tb) GRP(0, 1, 0); else GRP(1, 1, 0);
     }
 #undef GRP
-#undef GRP16
 #undef GRP_LAUNCH
     if (g_prof_on) g_prof.push_back(rec);
     hipError_t e = hipGetLastError();

@@ -1640,6 +1640,12 @@ static void flush_deferred_gemms(NCContext *m)
             }
         }
     }
+    // 256x256 tiles, one a CU, when their rounds of 256 are at least three quarters full; else
+    // 128x128, two a CU.  Measured, us (256 / 128): 12 layers of 512x512 to 2048x512 over 2048
+    // tokens, 578 tiles (2.3 rounds of 256) 213 / 252; 20 layers of 1024x1024 to 4096x1024 over 4096, 2768 / 3635
+    int64_t t256 = 0;
+    for (const DeferredGemm &d : m->deferred) t256 += nchip_gemm_grouped_tiles256(d.m, d.n);
+    const bool wide = from_shadows && 4 * t256 >= 3 * 256 * ((t256 + 255) / 256);
     size_t di = 0;
     for (DeferredGemm &d : m->deferred) {
         NchipGemmProblem p;
@@ -1656,7 +1662,7 @@ static void flush_deferred_gemms(NCContext *m)
         flops += 2.0 * d.m * d.n * (double)(d.k + p.k2);
         p.lda = d.m; p.ldb = d.n; p.ldc = d.m;
         p.tile_start = tiles; p.alpha = d.alpha;
-        tiles += nchip_gemm_grouped_tiles(d.m, d.n);
+        tiles += wide ? nchip_gemm_grouped_tiles256(d.m, d.n) : nchip_gemm_grouped_tiles(d.m, d.n);
         tab.push_back(p);
     }
     size_t bytes = tab.size() * sizeof(NchipGemmProblem), hcap, dcap;
@@ -1665,7 +1671,7 @@ static void flush_deferred_gemms(NCContext *m)
     memcpy(host, tab.data(), bytes);
     hip_check(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, m->stream), "hipMemcpyAsync gemm table");
     if (nchip_gemm_grouped(m->stream, 0, 1, (const NchipGemmProblem *)dev, (int)tab.size(), tiles,
-                           from_shadows ? 2 : m->matmul_bf16, flops))
+                           wide ? 3 : (from_shadows ? 2 : m->matmul_bf16), flops))
         nc_fatal("grouped weight-gradient GEMM failed");
     m->launches++;
     // pinned staging is recycled one flush later, after a wait for the stream

@@ -307,3 +307,72 @@ def test_attention_on_the_bf16_matrix_cores(hip, ref, rng, cfg):
         assert relerr(a, b) <= 1e-2, i
     if K % 8 == 0:
         assert launches <= 5            # 4 casts at most (parameters here have no producer) + the one kernel
+
+
+@pytest.mark.parametrize("ta,tb,m,n,k,pad", [(0, 0, 320, 70, 64, 0), (1, 0, 75, 131, 128, 1), (0, 1, 192, 128, 192, 2),
+                                             (1, 1, 130, 64, 320, 3), (1, 0, 260, 257, 576, 0), (0, 1, 64, 320, 448, 4)])
+def test_tile_classes_give_the_same_bits_at_the_edges_of_tiles_and_stages(hip, raw, rng, ta, tb, m, n, k, pad):
+    """Every class, 1 to 9 stages of 64 k, partial tiles in both directions, columns of C that are not
+    16-byte aligned: one chain over k for each element, so every class writes the same C (and a
+    copy that is its rounding), within fp32 summation error (k roundings of 2^-24) of float64."""
+    lib, st, ptr = raw
+    a = rng.standard_normal((m, k) if ta else (k, m)).astype(np.float32)
+    b = rng.standard_normal((k, n) if tb else (n, k)).astype(np.float32)
+    ra, rb = bf16_round(a), bf16_round(b)
+    am, bm = (ra[0] if not ta else ra[0].T).astype(np.float64), (rb[0] if not tb else rb[0].T).astype(np.float64)
+    pre, add, bias = (rng.standard_normal(s).astype(np.float32) for s in ((n, m + pad), (n, m + pad), (m,)))
+    product, scale = bm @ am, np.abs(bm) @ np.abs(am)
+    lib.nchip_gemm_rowsum_rows.restype = C.c_int
+    rows = lib.nchip_gemm_rowsum_rows(n)
+    first = {}
+    for cls in (1, 2, 3, 4, 5):
+        for mode in ("forward", "backward"):
+            t = dict(a=hip.tensor(ra[1]), b=hip.tensor(rb[1]), pre=hip.tensor(pre), add=hip.tensor(add), bias=hip.tensor(bias),
+                     c=hip.tensor(np.full((n, m + pad), 7.0, np.float32)), c16=hip.tensor(np.full((n, m + pad), 7, np.uint16)),
+                     rs=hip.tensor(np.zeros((rows, m), np.float32)))
+            written = C.c_int(0)
+            g = Args(ta=ta, tb=tb, m=m, n=n, k=k, alpha=1.0, A16=ptr(t["a"]), B16=ptr(t["b"]), lda=k if ta else m,
+                     ldb=n if tb else k, C=ptr(t["c"]), ldc=m + pad, C16=ptr(t["c16"]))
+            if mode == "forward":
+                g.bias, g.act, g.addend, want = ptr(t["bias"]), 2, ptr(t["add"]), np.maximum(product + bias, 0) + add[:, :m]
+            else:
+                g.dpre, g.dact, g.rowsum, g.rows_written = ptr(t["pre"]), 2, ptr(t["rs"]), C.pointer(written)
+                want = product * (pre[:, :m] > 0)
+            lib.nchip_gemm_bf16_operands_class(cls)
+            assert lib.nchip_gemm_bf16_operands(st, C.byref(g)) == 0
+            lib.nchip_gemm_bf16_operands_class(0)
+            c, c16, rs = hip.numpy(t["c"]), hip.numpy(t["c16"]), hip.numpy(t["rs"])
+            hip.free(*t.values())
+            assert np.all(np.abs(c[:, :m] - want) <= 2.0 ** -24 * (k + 2) * (scale + np.abs(bias) + np.abs(add[:, :m])))
+            assert (c[:, m:] == 7.0).all() and (c16[:, m:] == 7).all() and np.array_equal(c16[:, :m], bf16_round(c[:, :m])[1])
+            assert np.array_equal(first.setdefault(mode, c), c)
+            if mode == "backward":  # 16 columns a partial row, added in some order
+                bound = 2.0 ** -24 * 16 * np.abs(c[:, :m]).astype(np.float64).sum(0)
+                assert np.all(np.abs(rs[: written.value].astype(np.float64).sum(0) - c[:, :m].astype(np.float64).sum(0)) <= bound)
+
+
+def test_grouped_launch_in_wide_tiles(hip, raw, rng):
+    """nchip_gemm_grouped with precision 3: problems of 128 rows or columns inside 256-wide tiles, one of
+    two k ranges; the bits of the 128-wide launch."""
+    lib, st, ptr = raw
+    tables = {2: [], 3: []}
+    keep, outs, tiles = [], {2: [], 3: []}, {2: 0, 3: 0}
+    for m, n, k, k2 in [(384, 128, 192, 64), (128, 512, 64, 0), (256, 256, 128, 128)]:
+        d = [hip.tensor(bf16_round(rng.standard_normal((kk, dim)).astype(np.float32))[1])
+             for kk, dim in ((k, m), (k, n), (k2, m), (k2, n)) if kk]
+        keep += d
+        for prec, tile, count in ((2, 128, lib.nchip_gemm_grouped_tiles), (3, 256, lib.nchip_gemm_grouped_tiles256)):
+            out = hip.tensor(np.full((n, m), 5.0, np.float32))
+            tables[prec].append(Problem(A=ptr(d[0]), B=ptr(d[1]), C=ptr(out), A2=ptr(d[2]) if k2 else None,
+                                        B2=ptr(d[3]) if k2 else None, m=m, n=n, k=k, k2=k2, lda=m, ldb=n, ldc=m,
+                                        tile_start=tiles[prec], alpha=0.5))
+            tiles[prec] += -(-m // tile) * -(-n // tile)
+            assert count(m, n) == -(-m // tile) * -(-n // tile)
+            outs[prec].append(out)
+    for prec in (2, 3):
+        table = hip.tensor(np.frombuffer(b"".join(bytes(p) for p in tables[prec]), dtype=np.uint8))
+        assert lib.nchip_gemm_grouped(st, 0, 1, ptr(table), len(tables[prec]), tiles[prec], prec, 1.0) == 0
+        keep.append(table)
+    for two, three in zip(outs[2], outs[3]):
+        assert np.array_equal(hip.numpy(two), hip.numpy(three))
+    hip.free(*keep, *outs[2], *outs[3])
