@@ -105,7 +105,9 @@ int nchip_gemm_grouped_tiles256(int m, int n); /* the same for precision 3 */
    loads - every k and k2 a multiple of 64, every row-contiguous operand extent (m with
    ta = 0, n with tb = 1) a multiple of 128, leading dimensions multiples of 8, bases 16-byte
    aligned; the caller checks; 3: as 2 in 256x256 tiles, tile_start and total_tiles counted by
-   nchip_gemm_grouped_tiles256.  C is fp32 in all of them. */
+   nchip_gemm_grouped_tiles256; 4: fp32 operands as 0, by whole 16-byte units: every k and k2 a
+   multiple of 32, every row-contiguous extent and leading dimension a multiple of 4, bases
+   16-byte aligned.  C is fp32 in all of them. */
 int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmProblem *dev_table,
                        int n_problems, int total_tiles, int precision, double total_flops);
 

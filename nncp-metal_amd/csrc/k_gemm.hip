@@ -845,7 +845,7 @@ __device__ __forceinline__ void each_constant(F f, std::integer_sequence<int, I.
 // k for each element, in increasing k.
 //
 // A stage holds each operand as it lies in memory, in units of 16 bytes.  k contiguous: rows of 64 k,
-// unit c of row i in place c ^ (i & 7), a fragment is one 16-byte read.  Long axis contiguous: rows
+// unit c of row i in place c ^ (i / 2 & 7), a fragment is one 16-byte read.  Long axis contiguous: rows
 // of one k, and a fragment is two transposing reads of 4 k x 16 each; 32-byte granules (16 values)
 // are stored in place q ^ f(k) so that the four rows of a read lie in different banks.  The
 // swizzles are applied to the global address, a DMA being linear in LDS.
@@ -857,28 +857,59 @@ __device__ __forceinline__ void each_constant(F f, std::integer_sequence<int, I.
 // The stage of step it + 1 is waited for before the last quarter of step it, whose MFMAs cover the
 // barrier and the first fragment reads of the next; that barrier also says that stage it has
 // been read, and its place is refilled at once.
+//
+// F32: the same for fp32 operands, stages of 32 k.  v_mfma_f32_32x32x2_f32 takes one value a lane, k = 2 u +
+// lane / 32 of step u: rows of one k are stored with their odd rows' halves of 64 exchanged, so that the
+// two halves of a wavefront read different banks.  KW = 2 as in gemm_kernel, whose classes' sums
+// these are.  Bound by the matrix pipe (64 cycles a step) but for first loads and epilogue:
+// us before -> now, 512 x 2048 x 512 16.7 -> 14.5, 2048 x 2048 x 512 48.5 -> 42.0, the grouped weight
+// gradients of 12 layers of 512 over 2048 tokens 1571 -> 1361 (133 TFLOP/s).
 constexpr int BOX_LD = 36; // words between the columns of an accumulator tile in LDS
-template <int BM, int BN, int WM, int WN, int ST, int TA, int TB>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
+template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int TA, int TB>
+__global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0)
 {
     GemmArgs g = g0;
-    constexpr int NT = 64 * WM * WN;
+    constexpr int NG = WM * WN, NT = 64 * NG * KW;
     constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN), WTM = BM / WM, WTN = BN / WN;
+    constexpr int E = F32 ? 4 : 2, V = 16 / E, BK = 128 / E; // bytes of an element, elements of a unit, k of a stage
     constexpr int NVA = BM * 8 / NT, NVB = BN * 8 / NT, NL = NVA + NVB; // 16-byte loads a lane and stage
-    constexpr int STAGE = (BM + BN) * 64;
+    constexpr int STAGE = (BM + BN) * 64, NP = KW == 2 ? 2 : 4, NC = F32 ? NP : 1; // a stage in 16-bit words; parts its k is read in, chunks it is asked for in
+    static_assert(KW == 1 || (F32 && KW == 2 && TM * TN == 1), "k groups: fp32, one accumulator tile a wavefront");
     static_assert(NVA * NT == BM * 8 && NVB * NT == BN * 8, "whole loads");
     static_assert(ST >= 2 && (ST - 1) * NL <= 63, "the memory counter has six bits");
-    static_assert(WM * WN * 32 * BOX_LD * 4 <= ST * STAGE * 2, "the epilogue's corners fit where the stages were");
+    static_assert(NG * KW * 32 * BOX_LD * 4 <= ST * STAGE * 2, "the epilogue's corners fit where the stages were");
     extern __shared__ __attribute__((aligned(16))) uint16_t stages_lds[];
     uint16_t NCHIP_LDS *const stages = (uint16_t NCHIP_LDS *)stages_lds;
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int wm = wave % WM, wn = wave / WM, hi = lane >> 5;
+    const int kg = wave / NG, wm = wave % NG % WM, wn = wave % NG / WM, hi = lane >> 5;
 
     int tile_m, tile_n;
     const float *A2, *B2;
     int k1;
     find_tile<BM, BN>(g, tile_m, tile_n, A2, B2, k1);
-    const int m0 = tile_m * BM, n0 = tile_n * BN, nk = g.K / 64, it2 = k1 / 64;
+    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    int kbeg = 0, kend = g.K;
+    int64_t off_a = 0, off_b = 0;
+    if constexpr (F32) { // batch entry and k chunk
+        const int b = blockIdx.y / g.ksplit, kz = blockIdx.y % g.ksplit, out = b / g.batch_in, in = b % g.batch_in;
+        if (!g.grp) { kbeg = kz * g.kchunk; kend = min(g.K, kbeg + g.kchunk); }
+        off_a = out * g.sa + in * g.sa_in;
+        off_b = out * g.sb + in * g.sb_in;
+        const int64_t off_c = out * g.sc + in * g.sc_in;
+        if (g.ksplit > 1) { // the chunk's sum alone, for gemm_splitk_reduce
+            g.C = g.ws + ((int64_t)kz * g.batch + b) * g.M * g.N;
+            g.ldc = g.M;
+            g.bias = g.add = g.dpre = nullptr;
+            g.pre = g.rowsum = nullptr;
+            g.alpha = 1.0f; g.beta = 0.0f; g.act = NCHIP_ACT_NONE;
+        } else {
+            g.C += off_c;
+            if (g.pre) g.pre += off_c;
+            if (g.add) g.add += off_c;
+            if (g.dpre) g.dpre += off_c;
+        }
+    }
+    const int nk = (kend - kbeg) / BK, it2 = k1 / BK;
 
     // this lane's byte offsets inside a stage's panel of an operand; rows and units past the edge
     // repeat the last one (their results are not stored)
@@ -889,42 +920,61 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
             const int p = t + v * NT;
             if constexpr (decltype(kcontig)::value) {
                 const int i = p / 8, row = i0 + i < imax ? i : imax - 1 - i0;
-                off[v] = (uint32_t)(2 * (row * ld + ((p & 7) ^ (i & 7)) * 8));
+                off[v] = (uint32_t)(E * (row * ld + ((p ^ i >> 1) & 7) * V));
             } else {
-                constexpr int U = BT / 8, SH = BT >= 128 ? 1 : 0;
-                const int k = p / U, u = p % U, i = (((u >> 1) ^ ((k & 3) << SH)) * 2 + (u & 1)) * 8;
-                off[v] = (uint32_t)(2 * (k * ld + (i0 + i + 8 <= imax ? i : imax - 8 - i0)));
+                constexpr int U = BT / V, SH = BT >= 128 ? 1 : 0;
+                const int k = p / U, u = p % U;
+                const int i = F32 ? (u ^ (k & 1) << 3) * V : (((u >> 1) ^ ((k & 3) << SH)) * 2 + (u & 1)) * V;
+                off[v] = (uint32_t)(E * (k * ld + (i0 + i + V <= imax ? i : imax - V - i0)));
             }
         }
     };
     uint32_t oa[NVA], ob[NVB];
-    // (a long axis that is no multiple of 8 lies in a copy whose columns are padded to one)
-    offsets(oa, std::integral_constant<bool, TA != 0>(), std::integral_constant<int, BM>(), g.lda, m0, TA ? g.M : (g.M + 7) & ~7);
-    offsets(ob, std::integral_constant<bool, TB == 0>(), std::integral_constant<int, BN>(), g.ldb, n0, TB ? (g.N + 7) & ~7 : g.N);
-    const int64_t ea = TA ? m0 * g.lda : m0, eb = TB ? n0 : n0 * g.ldb;
-    const int64_t sa = TA ? 64 : 64 * g.lda, sb = TB ? 64 * g.ldb : 64; // elements from stage to stage
-    const uint16_t *pa = reinterpret_cast<const uint16_t *>(g.A) + ea, *pb = reinterpret_cast<const uint16_t *>(g.B) + eb;
+    // (a long axis that is no multiple of V lies in a copy whose columns are padded to one)
+    offsets(oa, std::integral_constant<bool, TA != 0>(), std::integral_constant<int, BM>(), g.lda, m0, TA ? g.M : (g.M + V - 1) & ~(V - 1));
+    offsets(ob, std::integral_constant<bool, TB == 0>(), std::integral_constant<int, BN>(), g.ldb, n0, TB ? (g.N + V - 1) & ~(V - 1) : g.N);
+    const int64_t ea = E * (TA ? m0 * g.lda : m0), eb = E * (TB ? n0 : n0 * g.ldb);
+    const int64_t sa = E * (TA ? BK : BK * g.lda), sb = E * (TB ? BK * g.ldb : BK); // bytes from stage to stage
+    const char *pa = reinterpret_cast<const char *>(g.A) + E * (off_a + (TA ? kbeg : kbeg * g.lda)) + ea;
+    const char *pb = reinterpret_cast<const char *>(g.B) + E * (off_b + (TB ? kbeg * g.ldb : kbeg)) + eb;
     int to = 0, asked = 0; // where the next stage goes, its number
-    auto issue = [&]() {
-        if (asked == it2) {
-            pa = reinterpret_cast<const uint16_t *>(A2) + ea;
-            pb = reinterpret_cast<const uint16_t *>(B2) + eb;
+    // chunk c of NC of the next stage's loads
+    auto issue = [&](auto chunk, auto piece) { // piece: an index into the chunk
+        constexpr int c = decltype(chunk)::value, v = c * NL / NC + decltype(piece)::value;
+        if (v == 0 && asked == it2) {
+            pa = reinterpret_cast<const char *>(A2) + ea;
+            pb = reinterpret_cast<const char *>(B2) + eb;
         }
         uint16_t NCHIP_LDS *dst = stages + to * STAGE + wave * 512;
-#pragma unroll
-        for (int v = 0; v < NVA; v++) lds_dma16(dst + v * NT * 8, pa, oa[v]);
-#pragma unroll
-        for (int v = 0; v < NVB; v++) lds_dma16(dst + BM * 64 + v * NT * 8, pb, ob[v]);
-        pa += sa; pb += sb;
-        asked++;
-        to = to + 1 < ST ? to + 1 : 0;
+        if constexpr (v < NVA) lds_dma16(dst + v * NT * 8, pa, oa[v < NVA ? v : 0]);
+        else lds_dma16(dst + BM * 64 + (v - NVA) * NT * 8, pb, ob[v < NVA ? 0 : v - NVA]);
+        if constexpr (v == NL - 1) {
+            pa += sa; pb += sb;
+            asked++;
+            to = to + 1 < ST ? to + 1 : 0;
+        }
+    };
+    auto issue_chunk = [&](auto chunk) {
+        constexpr int c = decltype(chunk)::value;
+        each_constant([&](auto piece) { issue(chunk, piece); }, std::make_integer_sequence<int, (c + 1) * NL / NC - c * NL / NC>());
     };
 
-    // fragments of quarter u of a stage's panel: offsets of lane and tile, then constants
+    // fragments of part u of a stage's panel (bf16: 16 k; fp32: four steps of 2): offsets of lane and
+    // tile, then constants
     auto fragment = [&](const uint16_t NCHIP_LDS *panel, auto kcontig, auto extent, int at, int j, int u) -> u32x4 {
         constexpr int BT = decltype(extent)::value;
-        if constexpr (decltype(kcontig)::value) {
-            return *reinterpret_cast<const u32x4 NCHIP_LDS *>(panel + (at + j * 32 + (lane & 31)) * 64 + (((u * 2 + hi) ^ (lane & 7)) * 8));
+        if constexpr (F32) {
+            const uint32_t NCHIP_LDS *p = (const uint32_t NCHIP_LDS *)panel;
+            const int i = at + j * 32 + (lane & 31), kb = (KW == 2 ? kg * 16 : 0) + u * 8;
+            u32x4 r;
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                if constexpr (decltype(kcontig)::value) r[s] = p[i * 32 + (((kb / 4 + (s >> 1)) ^ (lane >> 1 & 7)) * 4) + 2 * (s & 1) + hi];
+                else r[s] = p[(kb + 2 * s + hi) * BT + (i ^ hi << 5)];
+            }
+            return r;
+        } else if constexpr (decltype(kcontig)::value) {
+            return *reinterpret_cast<const u32x4 NCHIP_LDS *>(panel + (at + j * 32 + (lane & 31)) * 64 + (((u * 2 + hi) ^ (lane >> 1 & 7)) * 8));
         } else {
             constexpr int SH = BT >= 128 ? 1 : 0;
             const int k = u * 16 + hi * 8 + ((lane & 15) >> 2);
@@ -951,14 +1001,32 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
         for (int i = 0; i < TN; i++)
             fb[set][i] = fragment(s + BM * 64, std::integral_constant<bool, TB == 0>(), std::integral_constant<int, BN>(), wn * WTN, i, u);
     };
-    auto multiply = [&](int set) {
+    // the MFMAs of a part (its parity names the fragments' set), with the loads of a chunk between them
+    // where `on`: a load waits its turn at the CU's address unit, and the MFMAs in front of it go on
+    // (fp32, whose MFMAs are long, gains 5-8 %; bf16 loses as much by asking later)
+    auto multiply = [&](auto parity, auto chunk, auto on) {
         typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-#pragma unroll
-        for (int i = 0; i < TN; i++)
-#pragma unroll
-            for (int j = 0; j < TM; j++)
+        constexpr int set = decltype(parity)::value & 1, c = decltype(chunk)::value, NM = (F32 ? 4 : 1) * TM * TN;
+        constexpr int n = c < NC && NC > 1 ? (c + 1) * NL / NC - c * NL / NC : 0;
+        each_constant([&](auto index) {
+            constexpr int q = decltype(index)::value, s = q / (TM * TN), i = q % (TM * TN) / TM, j = q % TM;
+            if constexpr (F32) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[set][i][s]), __uint_as_float(fa[set][j][s]), acc[i][j], 0, 0, 0);
+            } else {
                 acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fb[set][i]),
                                                                     __builtin_bit_cast(bf16x8, fa[set][j]), acc[i][j], 0, 0, 0);
+            }
+            each_constant([&](auto piece) {
+                constexpr int x = decltype(piece)::value;
+                if constexpr ((x + 1) * NM / (n + 1) == q || ((x + 1) * NM / (n + 1) >= NM && q == NM - 1)) {
+                    if (on()) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        issue(chunk, piece);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }, std::make_integer_sequence<int, n>());
+        }, std::make_integer_sequence<int, NM>());
     };
     // waits until `younger` stages, at most ST - 2, are in flight
     auto arrive = [&](int younger) {
@@ -969,54 +1037,64 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
         lds_dma_barrier<0>(); // (from here on: everything)
     };
 
+    // ahead of step it: the stages up to it + ST - 2 and the first chunk of it + ST - 1, whose place
+    // step it - 1 has left
+    using chunks = std::make_integer_sequence<int, NP>;
+    using const0 = std::integral_constant<int, 0>;
+    using const1 = std::integral_constant<int, 1>;
 #pragma unroll
-    for (int s = 0; s < ST; s++)
-        if (s < nk) issue();
+    for (int s = 0; s < ST - 1; s++)
+        if (s < nk) each_constant(issue_chunk, std::make_integer_sequence<int, NC>());
+    if (ST - 1 < nk) issue_chunk(const0());
     // (with fewer stages than ST all of them are waited for)
-    if (nk >= ST) lds_dma_barrier<(ST - 1) * NL>(); else lds_dma_barrier<0>();
+    if (nk >= ST) lds_dma_barrier<(ST - 2) * NL + NL / NC>(); else lds_dma_barrier<0>();
     fetch(0, 0, 0);
     int at = 0; // the stage being read
+    auto no = [] { return false; };
     auto body = [&](auto more, int it) {
-#pragma unroll
-        for (int u = 0; u < 3; u++) {
-            fetch(at, u + 1, (u + 1) & 1);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(u & 1);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if constexpr (decltype(more)::value) lds_dma_barrier<(ST - 2) * NL>();
+        constexpr bool steady = decltype(more)::value;
+        each_constant([&](auto part) {
+            constexpr int u = decltype(part)::value;
+            if constexpr (u < NP - 1) {
+                fetch(at, u + 1, (u + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(part, std::integral_constant<int, u + 1>(), [&] { return steady || it + ST - 1 < nk; });
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }, chunks());
+        if constexpr (steady) lds_dma_barrier<(ST - 2) * NL>();
         else arrive(nk - 2 - it);
         at = at + 1 < ST ? at + 1 : 0;
-        if (decltype(more)::value) issue();
+        if (NC == 1 && (steady || it + ST < nk)) issue_chunk(const0());
         fetch(at, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(1);
+        multiply(const1(), const0(), [&] { return steady || it + ST < nk; });
         __builtin_amdgcn_sched_barrier(0);
     };
     int it = 0;
     for (; it + ST < nk; it++) body(std::true_type(), it);
     for (; it + 1 < nk; it++) body(std::false_type(), it);
-    fetch(at, 1, 1);
-    multiply(0);
-    fetch(at, 2, 0);
-    multiply(1);
-    fetch(at, 3, 1);
-    multiply(0);
-    multiply(1);
+    each_constant([&](auto part) {
+        constexpr int u = decltype(part)::value;
+        if constexpr (u + 1 < NP) fetch(at, u + 1, (u + 1) & 1);
+        multiply(part, const0(), no);
+    }, chunks());
 
     // Epilogue.  Every 32 x 32 accumulator tile passes through a corner of LDS (the stages are dead)
     // so that a lane holds four consecutive rows m of columns nl, nl + 8, nl + 16, nl + 24 and moves
     // them 16 bytes at a time, and what the next tile reads is on its way while this one is
-    // finished: a tile that loads, computes and stores alone is a memory round trip of its own.
+    // finished: a tile that loads, computes and stores alone is a memory round trip of its own.  Two k
+    // groups add their sums (group 0's first) on the way and finish half of the columns each.
     lds_dma_barrier<0>();
-    float NCHIP_LDS *const box = (float NCHIP_LDS *)stages + wave * (32 * BOX_LD);
+    float NCHIP_LDS *const box = (float NCHIP_LDS *)stages + wave * (32 * BOX_LD), *const box0 = (float NCHIP_LDS *)stages + wave % NG * (32 * BOX_LD);
     const int ml = (lane & 7) * 4, nl = lane >> 3;
     const bool full = (m0 + BM <= g.M) && (n0 + BN <= g.N); // uniform
     const bool wide = ((g.M | g.ldc) & 3) == 0 && (((uintptr_t)g.C | (uintptr_t)g.pre | (uintptr_t)g.add | (uintptr_t)g.dpre | (uintptr_t)g.bias | (uintptr_t)g.rowsum | (uintptr_t)(2 * (uintptr_t)g.c16)) & 15) == 0;
     // what a tile reads besides its accumulators: beta C or the addend (never both), else the
     // pre-activation (with an addend that one is read where it is used)
     const float *const first = g.beta != 0.0f ? g.C : g.add, *const operand = first ? first : g.dpre;
-    floatx4 next[4], bias_next;
+    constexpr int NQ = 4 / KW; // 8-column steps a wavefront finishes
+    floatx4 next[NQ], bias_next;
     auto load4 = [&](const float *p, int64_t at, int left) -> floatx4 { // left: rows of the matrix from here on
         floatx4 v = { 0.0f, 0.0f, 0.0f, 0.0f };
         if (left <= 0) return v;
@@ -1032,16 +1110,16 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
             if (e < left) as_global(p)[at + e] = v[e];
     };
     auto ask = [&](int tile) {
-        const int m = m0 + wm * WTM + tile % TM * 32 + ml, nb = n0 + wn * WTN + tile / TM * 32 + nl;
+        const int m = m0 + wm * WTM + tile % TM * 32 + ml, nb = n0 + wn * WTN + tile / TM * 32 + nl + kg * NQ * 8;
         if (g.bias) bias_next = load4(g.bias, m, g.M - m);
         if (operand) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) next[q] = load4(operand, (int64_t)(nb + 8 * q) * g.ldc + m, full || nb + 8 * q < g.N ? g.M - m : 0);
+            for (int q = 0; q < NQ; q++) next[q] = load4(operand, (int64_t)(nb + 8 * q) * g.ldc + m, full || nb + 8 * q < g.N ? g.M - m : 0);
         }
     };
     bias_next = floatx4{ 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-    for (int q = 0; q < 4; q++) next[q] = bias_next;
+    for (int q = 0; q < NQ; q++) next[q] = bias_next;
     ask(0);
 #pragma unroll 1
     for (int tile = 0; tile < TM * TN; tile++) { // (one copy of this code: unrolled it would not fit the instruction cache)
@@ -1052,22 +1130,28 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
                 for (int r = 0; r < 16; r++) box[((r >> 2) * 8 + (r & 3) + hi * 4) * BOX_LD + (lane & 31)] = acc[t0 / TM][t0 % TM][r];
             }
         }, std::make_integer_sequence<int, TM * TN>());
-        __builtin_amdgcn_wave_barrier();
-        floatx4 x[4], y[4];
+        if constexpr (KW == 2) __syncthreads(); else __builtin_amdgcn_wave_barrier();
+        floatx4 x[NQ], y[NQ];
         const floatx4 bv = bias_next;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            x[q] = *reinterpret_cast<const floatx4 NCHIP_LDS *>(box + (nl + 8 * q) * BOX_LD + ml);
+        for (int q = 0; q < NQ; q++) {
+            const float NCHIP_LDS *from = box + (nl + 8 * q) * BOX_LD + ml;
+            if constexpr (KW == 2) {
+                from = box0 + (nl + 8 * (q + kg * NQ)) * BOX_LD + ml;
+                x[q] = *reinterpret_cast<const floatx4 NCHIP_LDS *>(from) + *reinterpret_cast<const floatx4 NCHIP_LDS *>(from + NG * (32 * BOX_LD));
+            } else {
+                x[q] = *reinterpret_cast<const floatx4 NCHIP_LDS *>(from);
+            }
             y[q] = next[q];
         }
         __builtin_amdgcn_wave_barrier();
         if (tile + 1 < TM * TN) ask(tile + 1);
-        const int m = m0 + wm * WTM + tile % TM * 32 + ml, nb = n0 + wn * WTN + tile / TM * 32 + nl;
-        int left[4];
+        const int m = m0 + wm * WTM + tile % TM * 32 + ml, nb = n0 + wn * WTN + tile / TM * 32 + nl + kg * NQ * 8;
+        int left[NQ];
         const int64_t at0 = (int64_t)nb * g.ldc + m;
         auto at = [&](int q) { return at0 + 8 * q * g.ldc; };
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < NQ; q++) {
             left[q] = full || nb + 8 * q < g.N ? g.M - m : 0;
 #pragma unroll
             for (int e = 0; e < 4; e++) {
@@ -1078,49 +1162,49 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
         }
         if (g.pre) {
 #pragma unroll
-            for (int q = 0; q < 4; q++)
+            for (int q = 0; q < NQ; q++)
                 if (left[q] > 0) store4(g.pre, at(q), left[q], x[q]);
         }
-        if (g.act == ACT_GELU_FAST) {
+        if (g.act == (F32 ? NCHIP_ACT_GELU : ACT_GELU_FAST)) {
 #pragma unroll
-            for (int q = 0; q < 4; q++)
+            for (int q = 0; q < NQ; q++)
 #pragma unroll
-                for (int e = 0; e < 4; e++) x[q][e] = nchip_gelu_fast(x[q][e]);
+                for (int e = 0; e < 4; e++) x[q][e] = F32 ? nchip_gelu(x[q][e]) : nchip_gelu_fast(x[q][e]);
         } else if (g.act == NCHIP_ACT_RELU) {
 #pragma unroll
-            for (int q = 0; q < 4; q++)
+            for (int q = 0; q < NQ; q++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) x[q][e] = x[q][e] > 0.0f ? x[q][e] : 0.0f;
         }
         if (g.add) {
 #pragma unroll
-            for (int q = 0; q < 4; q++)
+            for (int q = 0; q < NQ; q++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) x[q][e] += y[q][e];
         }
         if (g.dpre) { // gradient through an activation: times act'(pre-activation)
             if (first) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) y[q] = load4(g.dpre, at(q), left[q]);
+                for (int q = 0; q < NQ; q++) y[q] = load4(g.dpre, at(q), left[q]);
             }
-            if (g.dact == ACT_GELU_FAST) {
+            if (g.dact == (F32 ? NCHIP_ACT_GELU : ACT_GELU_FAST)) {
 #pragma unroll
-                for (int q = 0; q < 4; q++)
+                for (int q = 0; q < NQ; q++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) x[q][e] *= nchip_gelu_grad_fast(y[q][e]);
+                    for (int e = 0; e < 4; e++) x[q][e] *= F32 ? nchip_gelu_grad(y[q][e]) : nchip_gelu_grad_fast(y[q][e]);
             } else if (g.dact == NCHIP_ACT_RELU) {
 #pragma unroll
-                for (int q = 0; q < 4; q++)
+                for (int q = 0; q < NQ; q++)
 #pragma unroll
                     for (int e = 0; e < 4; e++) x[q][e] *= y[q][e] > 0.0f ? 1.0f : 0.0f;
             }
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int q = 0; q < NQ; q++)
             if (left[q] > 0) store4(g.C, at(q), left[q], x[q]);
         if (g.c16) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
+            for (int q = 0; q < NQ; q++) {
                 uint16_t NCHIP_GLOBAL *h = as_global(g.c16) + at(q);
                 if (wide && left[q] > 0) {
                     *reinterpret_cast<uint2 NCHIP_GLOBAL *>(h) = make_uint2(pack_bf16(x[q][0], x[q][1]), pack_bf16(x[q][2], x[q][3]));
@@ -1131,10 +1215,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
                 }
             }
         }
-        if (g.rowsum) { // one partial row per half of the tile's columns (n % 8 below 4, from 4 on)
+        if (g.rowsum) { // one partial row per wavefront and half of its columns (n % 8 below 4, from 4 on)
             floatx4 sum = { 0.0f, 0.0f, 0.0f, 0.0f };
 #pragma unroll
-            for (int q = 0; q < 4; q++)
+            for (int q = 0; q < NQ; q++)
 #pragma unroll
                 for (int e = 0; e < 4; e++) sum[e] += left[q] > 0 ? x[q][e] : 0.0f;
 #pragma unroll
@@ -1143,7 +1227,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_dma_kernel(GemmArgs g0)
                 sum[e] += __shfl_xor(sum[e], 16, 64);
             }
             if ((lane & 24) == 0 && m < g.M)
-                store4(g.rowsum, (int64_t)(((tile_n * WN + wn) * TN + tile / TM) * 2 + hi) * g.M + m, g.M - m, sum);
+                store4(g.rowsum, (int64_t)((((tile_n * WN + wn) * TN + tile / TM) * 2 + hi) * KW + kg) * g.M + m, g.M - m, sum);
         }
     }
 }
@@ -1791,7 +1875,7 @@ void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec)
 #undef LAUNCH
 }
 
-template <int BM, int BN, int WM, int WN, int ST>
+template <int F32, int BM, int BN, int WM, int WN, int KW, int ST>
 void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int grouped_tiles = 0)
 {
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -1799,15 +1883,15 @@ void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int g
     g.gm = g_force_gm >= 0 ? g_force_gm : 8;
     constexpr size_t dyn = (size_t)(BM + BN) * 64 * 2 * ST;
     static_assert(dyn <= 160 * 1024, "stages exceed LDS");
-    dim3 grid(grouped_tiles ? grouped_tiles : g.tiles_m * g.tiles_n), block(64 * WM * WN);
+    dim3 grid(grouped_tiles ? grouped_tiles : g.tiles_m * g.tiles_n, g.batch * g.ksplit), block(64 * WM * WN * KW);
 #define LAUNCH(TA, TB)                                                                                     \
     do {                                                                                                   \
         static const bool ok = hipFuncSetAttribute(                                                        \
-            reinterpret_cast<const void *>(gemm_dma_kernel<BM, BN, WM, WN, ST, TA, TB>),                    \
+            reinterpret_cast<const void *>(gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB>),                    \
             hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn) == hipSuccess;                           \
         if (!ok) { fprintf(stderr, "nchip_gemm: cannot reserve %zu bytes of LDS\n", dyn); abort(); }      \
-        if (rec) hipExtLaunchKernelGGL((gemm_dma_kernel<BM, BN, WM, WN, ST, TA, TB>), grid, block, dyn, st, rec->start, rec->stop, 0, g); \
-        else hipLaunchKernelGGL((gemm_dma_kernel<BM, BN, WM, WN, ST, TA, TB>), grid, block, dyn, st, g);   \
+        if (rec) hipExtLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB>), grid, block, dyn, st, rec->start, rec->stop, 0, g); \
+        else hipLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB>), grid, block, dyn, st, g);   \
     } while (0)
     if (!ta && !tb) LAUNCH(0, 0);
     else if (ta && !tb) LAUNCH(1, 0);
@@ -1840,11 +1924,11 @@ static int dma_class(int m, int n)
 
 static void launch_dma_class(hipStream_t st, int cls, int ta, int tb, GemmArgs &g, ProfRec *rec)
 {
-    if (cls == 4) launch_dma<256, 256, 2, 4, 2>(st, ta, tb, g, rec);
-    else if (cls == 1) launch_dma<128, 128, 2, 2, 2>(st, ta, tb, g, rec);
-    else if (cls == 5) launch_dma<128, 128, 2, 4, 4>(st, ta, tb, g, rec);
-    else if (cls == 2) launch_dma<128, 64, 2, 2, 3>(st, ta, tb, g, rec);
-    else launch_dma<64, 64, 2, 2, 4>(st, ta, tb, g, rec);
+    if (cls == 4) launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, rec);
+    else if (cls == 1) launch_dma<0, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, rec);
+    else if (cls == 5) launch_dma<0, 128, 128, 2, 4, 1, 4>(st, ta, tb, g, rec);
+    else if (cls == 2) launch_dma<0, 128, 64, 2, 2, 1, 3>(st, ta, tb, g, rec);
+    else launch_dma<0, 64, 64, 2, 2, 1, 4>(st, ta, tb, g, rec);
 }
 
 template <int NW, int PF, int SPLIT>
@@ -1964,6 +2048,29 @@ static bool gemm_is_small(int m, int n, int k, int batch, int ksplit)
     return tiles <= 2048 && (k < 1024 ? tiles <= 1152 || tiles * k <= 3 << 17 : k <= 3072 && tiles * k <= 3 << 18) && gemm_class(m, n, (int64_t)batch * ksplit) == 10;
 }
 
+// Whether an fp32 product of class 7, 4 or 10 is issued by gemm_dma_kernel (the same sums; this is about
+// time only): whole stages of 32 k, 16-byte units, 32-bit offsets inside a stage.  The single-chain
+// classes gain everywhere; of the 64x64 class, tiles that the other kernel would guard, more tiles than CUs
+// and operands that need no reads across rows (both K-contiguous reads of a step hit two banks twice),
+// us 64x64 class -> this:
+//   352 x 1066 x 352 16.0 -> 10.3   704 x 1066 x 352 15.9 -> 10.9   512 x 2048 x 512 16.7 -> 14.5
+//   512 x 2048 x 2048 42.5 -> 43.9 (kept out), A transposed 45.9 -> 48.1, x 1024 24.0 -> 26.2 (out), B transposed 43.4 -> 41.5
+//   256 of 64 x 320 x 128, A transposed 36.0 -> 28.6
+// class 4: 2048 x 2048 x 512 48.5 -> 42.0, 1024 x 2048 x 512 24.9 -> 23.7, 256 of 320 x 64 x 128 31.0 -> 24.8
+// class 7: 4096 x 4096 x 1024 300 -> 261, A transposed 291 -> 267, B transposed (4096 x 1024 x 4096) 303 -> 249
+static bool dma_fits_f32(const GemmArgs &g, int ta, int tb)
+{
+    const int64_t any = g.lda | g.ldb | g.sa | g.sb | g.sa_in | g.sb_in | (ta ? 0 : g.M) | (tb ? g.N : 0);
+    return g.K > 0 && g.K % 32 == 0 && (g.ksplit == 1 || g.kchunk % 32 == 0) && any % 4 == 0 &&
+           (((uintptr_t)g.A | (uintptr_t)g.B) & 15) == 0 && g.lda < 1 << 22 && g.ldb < 1 << 22;
+}
+static bool dma_gains_f32(const GemmArgs &g, int cfg, int ta, int tb)
+{
+    if (cfg != 10) return cfg == 7 || cfg == 4;
+    const int64_t tiles = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch * g.ksplit;
+    return g.M % 64 || g.N % 64 || tiles > 256 || tb || (!ta && g.K <= 1024);
+}
+
 extern "C" int nchip_gemm_is_small(int m, int n, int k, int batch)
 {
     return !g_force_cfg && gemm_is_small(m, n, k, batch, nchip_gemm_pick_ksplit(m, n, k, batch));
@@ -2057,7 +2164,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     // the ones the conversion inside the tile loader would produce, so the
     // result is the same either way.
     bool from_bf16 = false;
-    if (precision == 1 && batch == 1 && ksplit == 1 && !invariant && k > 0 &&
+    if (precision == 1 && batch == 1 && ksplit == 1 && !invariant && k > 0 && m < 1 << 21 && n < 1 << 21 && k < 1 << 21 && // (32-bit offsets)
         (g_bf16src == 2 || (g_bf16src == 1 && m >= 128 && n >= 128 && k >= 256 &&
                             2.0 * m * n * (double)k >= g_bf16src_min_flops))) {
         const int kpad = (k + 63) / 64 * 64;
@@ -2073,13 +2180,14 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
             from_bf16 = true;
         }
     }
+    const bool dma = precision == 0 && !g_force_cfg && dma_fits_f32(g, ta, tb) && dma_gains_f32(g, cfg, ta, tb);
     // partial row sums of the result (activation-gradient epilogue): one row per 16 columns of
     // the padded column range; only the plain tile classes write them
     if (rowsum && rowsum_rows && dpre && ksplit == 1 && batch == 1 && !from_bf16 &&
         (cfg == 7 || cfg == 4 || cfg == 10 || cfg == 30)) {
-        const int bn = cfg == 7 ? 128 : 64;
+        const int bn = cfg == 7 && !(dma && tb) ? 128 : 64;
         g.rowsum = rowsum;
-        *rowsum_rows = (n + bn - 1) / bn * bn / 16;
+        *rowsum_rows = (n + bn - 1) / bn * bn / (dma && cfg == 10 ? 8 : 16);
     }
     if (from_bf16) {
         launch_dma_class(st, dma_class(m, n), ta, tb, g, pr);
@@ -2088,6 +2196,10 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
         else if (cfg == 4) launch_tile<128, 64, 32, 4, 2, 1>(st, ta, tb, g, pr);
         else if (cfg == 9) launch_tile<64, 64, 64, 2, 2, 1, 2>(st, ta, tb, g, pr);
         else launch_tile<64, 64, 32, 2, 2, 1, 2>(st, ta, tb, g, pr);
+    } else if (dma) {
+        if (cfg == 10) launch_dma<1, 64, 64, 2, 2, 2, 4>(st, ta, tb, g, pr);
+        else if (cfg == 7 && !tb) launch_dma<1, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, pr);
+        else launch_dma<1, 128, 64, 4, 2, 1, 3>(st, ta, tb, g, pr);
     } else if (cfg == 40) {
         // (wavefronts: the two chains, or as many of the 2 ksplit; blocks in flight: one round trip's)
         if (ksplit > 4) launch_small<16, 8, 1>(st, ta, tb, g, pr);
@@ -2124,6 +2236,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     if (g_prof_on) {
         int tile = cfg == 40 ? 6 : cfg == 7 ? 2 : (cfg == 4 ? 1 : ((cfg == 8 || cfg == 10 || cfg == 30) ? 3 : 0));
         rec.variant = tile * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 1 ? 1 : 0);
+        if (dma) rec.variant = 88 + (cfg == 10 ? 12 : (cfg == 7 && !tb ? 4 : 8)) + (ta ? 2 : 0) + (tb ? 1 : 0);
         g_prof.push_back(rec);
     }
     if (ksplit > 1 && cfg != 40) {
@@ -2177,7 +2290,7 @@ extern "C" int nchip_gemm_dact(void *stream, int ta, int tb, int m, int n, int k
 // nchip_gemm_dact that also leaves partial row sums of C: rowsum holds nchip_gemm_rowsum_rows(n)
 // rows of m floats, of which *rows_written are written (row p = the sum over 16 columns of C;
 // 0 when this product's kernel does not write them: the caller then sums C itself)
-extern "C" int nchip_gemm_rowsum_rows(int n) { return (n + 255) / 256 * 16; } // (the widest tile's)
+extern "C" int nchip_gemm_rowsum_rows(int n) { return (n + 255) / 256 * 32; } // (the widest tile's, two k groups)
 
 extern "C" int nchip_gemm_dact_rowsum(void *stream, int ta, int tb, int m, int n, int k, float alpha,
                                       const float *A, int64_t lda, const float *B, int64_t ldb,
@@ -2350,7 +2463,7 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
         fprintf(stderr, "nchip_gemm_bf16_operands: bad arguments (m=%d n=%d k=%d)\n", m, n, k);
         return -1;
     }
-    if (k % 64 || a->lda % 8 || a->ldb % 8 || (!ta && m % 64) || (tb && n % 64) || (((uintptr_t)a->A16 | (uintptr_t)a->B16) & 15) != 0)
+    if (k % 64 || a->lda % 8 || a->ldb % 8 || a->lda >= 1 << 22 || a->ldb >= 1 << 22 || (!ta && m % 64) || (tb && n % 64) || (((uintptr_t)a->A16 | (uintptr_t)a->B16) & 15) != 0)
         return 1;
     GemmArgs g;
     memset(&g, 0, sizeof(g));
@@ -2398,7 +2511,7 @@ extern "C" void nchip_gemm_profile_enable(int on)
 extern "C" int nchip_gemm_profile_read(int max_variants, char (*names)[48], int64_t *launches,
                                        double *flops, double *seconds)
 {
-    constexpr int NVAR = 88;
+    constexpr int NVAR = 104;
     double fl[NVAR] = { 0 }, sec[NVAR] = { 0 };
     int64_t cnt[NVAR] = { 0 };
     for (ProfRec &r : g_prof) {
@@ -2416,17 +2529,20 @@ extern "C" int nchip_gemm_profile_read(int max_variants, char (*names)[48], int6
     g_prof.clear();
     static const char *tiles_f32[4] = { "64,64,16,2,2", "128,64,32,4,2", "128,128,32,4,2", "64,64,32,2,2" };
     static const char *tiles_bf16[4] = { "64,64,32,2,2", "128,64,32,4,2", "128,128,32,4,2", "64,64,32,2,2" };
-    static const char *tiles_ops[6] = { "256,256,2,4,2", "128,128,2,2,2", "128,64,2,2,3", "64,64,2,2,4", "256,256,2,4,2", "128,128,2,4,4" }; // 0: grouped
+    static const char *tiles_ops[6] = { "256,256,2,4,1,2", "128,128,2,2,1,2", "128,64,2,2,1,3", "64,64,2,2,1,4", "256,256,2,4,1,2", "128,128,2,4,1,4" }; // 0: grouped
+    static const char *tiles_f32_dma[4] = { "128,128,4,2,1,4", "128,128,2,2,1,2", "128,64,4,2,1,3", "64,64,2,2,2,4" }; // 0: grouped
     int n = 0;
     for (int v = 0; v < NVAR && n < max_variants; v++) {
         if (!cnt[v]) continue;
-        if (v >= 64) { // operands read as bf16: gemm_dma_kernel<tile, wavefronts, stages, ta, tb>
-            snprintf(names[n], 48, "gemm_dma_kernel<%s,%d,%d%s>", tiles_ops[(v - 64) / 4], (v >> 1) & 1, v & 1,
+        if (v >= 88) { // fp32 operands staged by DMA
+            snprintf(names[n], 48, "gemm_dma_kernel<1,%s,%d,%d%s>", tiles_f32_dma[(v - 88) / 4], (v >> 1) & 1, v & 1, v < 92 ? ",grouped" : "");
+        } else if (v >= 64) { // operands read as bf16: gemm_dma_kernel<tile, wavefronts, stages, ta, tb>
+            snprintf(names[n], 48, "gemm_dma_kernel<0,%s,%d,%d%s>", tiles_ops[(v - 64) / 4], (v >> 1) & 1, v & 1,
                      v < 68 ? ",grouped" : "");
         } else if (v >= 48) {
             snprintf(names[n], 48, "gemm_small_kernel<%d,%d>", (v >> 2) & 1, (v >> 1) & 1);
         } else if (v >= 32) { // the grouped launch in 128 x 128 tiles
-            snprintf(names[n], 48, "gemm_dma_kernel<128,128,2,2,2,%d,%d,grouped>", (v >> 1) & 1, v & 1);
+            snprintf(names[n], 48, "gemm_dma_kernel<0,128,128,2,2,1,2,%d,%d,grouped>", (v >> 1) & 1, v & 1);
         } else {
             const bool two_groups = v / 8 == 3 || ((v & 1) && v / 8 == 0);
             snprintf(names[n], 48, "gemm_kernel<%s,%d,%d,%d%s>", (v & 1) ? tiles_bf16[v / 8] : tiles_f32[v / 8],
@@ -2468,7 +2584,7 @@ extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmP
     if (g_prof_on) {
         (void)hipEventCreate(&rec.start);
         (void)hipEventCreate(&rec.stop);
-        rec.variant = precision >= 2 ? (precision == 3 ? 64 : 32) + (ta ? 2 : 0) + (tb ? 1 : 0)
+        rec.variant = precision >= 2 ? (precision == 4 ? 88 : precision == 3 ? 64 : 32) + (ta ? 2 : 0) + (tb ? 1 : 0)
                                      : 2 * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 1 ? 1 : 0);
         rec.flops = total_flops;
     }
@@ -2484,10 +2600,12 @@ extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmP
         else hipLaunchKernelGGL(KERNEL, grid, block, dyn, st, g);                                          \
     } while (0)
 #define GRP(TA, TB, BF) GRP_LAUNCH((gemm_kernel<128, 128, 32, 4, 2, TA, TB, BF, 1, 2, 1, (BF == 0)>), 32, TA, TB, BF)
-    if (precision == 3) {
-        launch_dma<256, 256, 2, 4, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+    if (precision == 4) {
+        launch_dma<1, 128, 128, 4, 2, 1, 4>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+    } else if (precision == 3) {
+        launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
     } else if (precision == 2) {
-        launch_dma<128, 128, 2, 2, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+        launch_dma<0, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
     } else if (precision == 1) {
         if (!ta && !tb) GRP(0, 0, 1); else if (ta && !tb) GRP(1, 0, 1); else if (!ta && tb) GRP(0, 1, 1); else GRP(1, 1, 1);
     } else {

@@ -1646,6 +1646,14 @@ static void flush_deferred_gemms(NCContext *m)
     int64_t t256 = 0;
     for (const DeferredGemm &d : m->deferred) t256 += nchip_gemm_grouped_tiles256(d.m, d.n);
     const bool wide = from_shadows && 4 * t256 >= 3 * 256 * ((t256 + 255) / 256);
+    // fp32 by whole 16-byte units where every problem allows: 12 layers of 512x512 to 2048x512 over 2048
+    // tokens 1571 -> 1361 us
+    bool units = !from_shadows && !m->matmul_bf16;
+    for (const DeferredGemm &d : m->deferred) {
+        if (d.k < 32 || d.k % 32 || (d.a2 && d.k2 % 32) || d.m % 4 || d.n % 4 || d.m >= 1 << 22 || d.n >= 1 << 22) units = false;
+        for (const NCTensor *t : { d.a, d.b, d.a2, d.b2 })
+            if (t && ((uintptr_t)nc_f32(t) & 15)) units = false;
+    }
     size_t di = 0;
     for (DeferredGemm &d : m->deferred) {
         NchipGemmProblem p;
@@ -1671,7 +1679,7 @@ static void flush_deferred_gemms(NCContext *m)
     memcpy(host, tab.data(), bytes);
     hip_check(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, m->stream), "hipMemcpyAsync gemm table");
     if (nchip_gemm_grouped(m->stream, 0, 1, (const NchipGemmProblem *)dev, (int)tab.size(), tiles,
-                           wide ? 3 : (from_shadows ? 2 : m->matmul_bf16), flops))
+                           wide ? 3 : (from_shadows ? 2 : (units ? 4 : m->matmul_bf16)), flops))
         nc_fatal("grouped weight-gradient GEMM failed");
     m->launches++;
     // pinned staging is recycled one flush later, after a wait for the stream

@@ -381,3 +381,51 @@ def test_lookup_table_inverts_an_ascending_cdf(hip, v, n, m, to, so):
     assert np.array_equal(got[so:so + n * m].reshape(n, m), want)
     for x in (c_t, t_t, s_t):
         hip.free(x)
+
+
+@pytest.mark.parametrize("cls,ta,tb,m,n,k,batch,ldc", [(10, 0, 0, 100, 67, 288, 40, 100), (10, 1, 0, 101, 68, 320, 40, 101), (10, 0, 1, 100, 68, 288, 40, 103),
+                                                       (10, 1, 1, 99, 64, 288, 44, 100), (4, 0, 0, 132, 67, 32, 80, 132), (4, 1, 0, 133, 66, 96, 80, 133),
+                                                       (4, 0, 1, 136, 72, 160, 70, 136), (7, 1, 0, 131, 129, 64, 130, 132), (7, 0, 1, 132, 132, 32, 130, 132),
+                                                       (7, 0, 0, 260, 130, 128, 90, 260)])
+def test_fp32_products_staged_by_dma_keep_the_sums_of_their_class(hip, cls, ta, tb, m, n, k, batch, ldc):
+    """Partial tiles in both directions, fewer and more stages of 32 k than are in flight: the bits of the
+    tile kernel of the same class, with bias, activation and the pre-activation kept."""
+    lib, rng = C.CDLL(hip.lib._name), np.random.default_rng(m * k + n)
+    p, i, j, f = C.c_void_p, C.c_int, C.c_int64, C.c_float
+    lib.nchip_gemm2.argtypes = [p, i, i, i, i, i, f, p, j, j, j, p, j, j, j, f, p, j, j, j, i, i, p, i, p, i, i, p]
+    a, b = rng.standard_normal((batch, m, k) if ta else (batch, k, m)), rng.standard_normal((batch, k, n) if tb else (batch, n, k))
+    a_t, b_t, bias_t = (hip.tensor(x.astype(np.float32)) for x in (a, b, rng.standard_normal(m)))
+    ptr = lambda t: p(hip.nc_tensor_get_ptr(t, None))
+    got = []
+    for forced in (0, cls):
+        c_t, pre_t = (hip.tensor(np.full((batch, n, ldc), 7.0, np.float32)) for _ in range(2))
+        lib.nchip_gemm_force_config(forced)
+        rc = lib.nchip_gemm2(p(hip.nc_context_stream(hip.ctx)), ta, tb, m, n, k, 1.0, ptr(a_t), k if ta else m, m * k, 0, ptr(b_t),
+                             n if tb else k, n * k, 0, 0.0, ptr(c_t), ldc, n * ldc, 0, batch, 1, ptr(bias_t), 1, ptr(pre_t), 0, 1, None)
+        lib.nchip_gemm_force_config(0)
+        assert rc == 0
+        got.append([hip.numpy(c_t), hip.numpy(pre_t)])
+        hip.free(c_t, pre_t)
+    assert all(np.array_equal(x, y) for x, y in zip(*got))
+    assert all((x[:, :, m:] == 7.0).all() for x in got[0])
+    hip.free(a_t, b_t, bias_t)
+
+
+@pytest.mark.parametrize("m,n,k", [(132, 8200, 64), (100, 4100, 96)])
+def test_fp32_activation_gradient_products_leave_their_row_sums_under_dma(hip, m, n, k):
+    """nchip_gemm_dact_rowsum through the 128x64 and the two-group 64x64 tiles: the partial rows add up to
+    the row sums of C (16 or 8 roundings a partial row, then the sum in float64)."""
+    lib, rng = C.CDLL(hip.lib._name), np.random.default_rng(n)
+    p, i, j = C.c_void_p, C.c_int, C.c_int64
+    lib.nchip_gemm_dact_rowsum.argtypes = [p, i, i, i, i, i, C.c_float, p, j, p, j, p, j, p, i, i, i, p, p, C.POINTER(i)]
+    w, dy, pre = (rng.standard_normal(s).astype(np.float32) for s in ((m, k), (n, k), (n, m)))
+    rows, written = lib.nchip_gemm_rowsum_rows(n), C.c_int(0)
+    w_t, dy_t, pre_t, c_t, rs_t = (hip.tensor(x) for x in (w, dy, pre, np.zeros((n, m), np.float32), np.full((rows, m), 9.0, np.float32)))
+    ptr = lambda t: p(hip.nc_tensor_get_ptr(t, None))
+    assert lib.nchip_gemm_dact_rowsum(p(hip.nc_context_stream(hip.ctx)), 1, 0, m, n, k, 1.0, ptr(w_t), k, ptr(dy_t), k, ptr(c_t), m,
+                                      ptr(pre_t), 2, 0, 1, None, ptr(rs_t), C.byref(written)) == 0
+    c, rs = hip.numpy(c_t).astype(np.float64), hip.numpy(rs_t).astype(np.float64)
+    want = (dy.astype(np.float64) @ w.astype(np.float64).T) * (pre > 0)
+    assert np.all(np.abs(c - want) <= 2.0 ** -24 * (k + 1) * (np.abs(dy) @ np.abs(w).T))
+    assert 0 < written.value <= rows and np.all(np.abs(rs[: written.value].sum(0) - c.sum(0)) <= 2.0 ** -24 * 16 * np.abs(c).sum(0))
+    hip.free(w_t, dy_t, pre_t, c_t, rs_t)
