@@ -38,6 +38,7 @@
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx4_u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float floatx2_u __attribute__((ext_vector_type(2), aligned(4)));
 typedef short shortx8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4))); // a first-class value, unlike the uint4 struct
 
@@ -122,6 +123,13 @@ __device__ __forceinline__ unsigned short f32_to_bf16(float f)
     return (unsigned short)(u >> 16);
 }
 
+__device__ __forceinline__ void wait_for_loads()
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_s_waitcnt(0);
+#endif
+}
+
 // Loads a BT x BK tile (BT = BM or BN) of an operand into registers.
 // MAJOR = 1: the tile's long axis (m or n) is contiguous in memory
 //            (A with ta = 0, B with tb = 1);  element (i, k) at p[i + k*ld].
@@ -156,9 +164,9 @@ struct TileLoader {
             int i, k;
             coords(idx, i, k);
             if (fast) {
-                const float *src = MAJOR ? p + (int64_t)(k0 + k) * ld + (i0 + i)
-                                         : p + (int64_t)(i0 + i) * ld + (k0 + k);
-                r[v] = *as_global(reinterpret_cast<const floatx4 *>(src));
+                const int ii = min(i0 + i, imax - 1); // (see whole_stages)
+                const float *src = MAJOR ? p + (int64_t)(k0 + k) * ld + ii : p + (int64_t)ii * ld + (k0 + k);
+                r[v] = *reinterpret_cast<const floatx4_u NCHIP_GLOBAL *>(as_global(src));
             } else {
                 floatx4 tmp;
 #pragma unroll
@@ -226,13 +234,14 @@ struct TileLoaderBf16 {
             int i, k;
             coords(v, t, i, k);
             if (fast) {
+                const int ii = min(i0 + i, imax - 1);
                 if (MAJOR) {
-                    const float *src = p + (int64_t)(k0 + k) * ld + (i0 + i);
-                    floatx2_t a = *as_global(reinterpret_cast<const floatx2_t *>(src));
-                    floatx2_t b = *as_global(reinterpret_cast<const floatx2_t *>(src + ld));
+                    const float *src = p + (int64_t)(k0 + k) * ld + ii;
+                    floatx2_u a = *reinterpret_cast<const floatx2_u NCHIP_GLOBAL *>(as_global(src));
+                    floatx2_u b = *reinterpret_cast<const floatx2_u NCHIP_GLOBAL *>(as_global(src) + ld);
                     r[v] = floatx4{ a[0], a[1], b[0], b[1] };
                 } else {
-                    r[v] = *as_global(reinterpret_cast<const floatx4 *>(p + (int64_t)(i0 + i) * ld + (k0 + k)));
+                    r[v] = *reinterpret_cast<const floatx4_u NCHIP_GLOBAL *>(as_global(p) + (int64_t)ii * ld + (k0 + k));
                 }
             } else {
                 floatx4 tmp;
@@ -1281,9 +1290,24 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
     const float *A = g.A + (int64_t)b_out * g.sa + (int64_t)b_in * g.sa_in;
     const float *B = g.B + (int64_t)b_out * g.sb + (int64_t)b_in * g.sb_in;
 
-    // fast (vector, unguarded) loads need whole tiles and 16-byte alignment
-    const bool a_full = (m0 + BM <= g.M) && (g.lda % 4 == 0) && (((uintptr_t)A & 15) == 0);
-    const bool b_full = (n0 + BN <= g.N) && (g.ldb % 4 == 0) && (((uintptr_t)B & 15) == 0);
+    // Stages of BK k: nk1 of the first k range, then those of the second; only a range's last stage
+    // may be partial.  The first whole_stages() of a range need no guards: loads of 16 bytes at any
+    // 4-byte alignment, from row / column imax - 1 at the latest (what lies past the edge lands in
+    // results that are not stored).  With the long axis contiguous such a load runs past the edge by up
+    // to 3 values, into the next k: the stage with the range's last k is then left to the guarded loads.
+    // Guarding every value of partial or unaligned tiles made a stage a serial chain of memory round trips
+    // (3.8 us); us: 777 x 352 over 481 and 585 k, five layers' gradients in one launch instead of ten
+    // 573 -> 126, 777 x 481 x 352 in the 64x64 class 19.8 -> 16.1.
+    const bool two = g.grp && A2; // uniform
+    const int end1 = two ? k1 : kend, end2 = kend - k1; // where the ranges end (the second counts from 0)
+    const int nk1 = (end1 - kbeg + BK - 1) / BK, nk = nk1 + (two ? (end2 + BK - 1) / BK : 0);
+    auto whole_stages = [&](int len) {
+        const int la_len = (TA || m0 + BM <= g.M) ? len : len - (g.lda >= 3 ? 1 : 3);
+        const int lb_len = (!TB || n0 + BN <= g.N) ? len : len - (g.ldb >= 3 ? 1 : 3);
+        const int l = min(la_len, lb_len);
+        return l > 0 ? l / BK : 0;
+    };
+    const int whole1 = whole_stages(end1 - kbeg), whole2 = two ? nk1 + whole_stages(end2) : 0;
 
     // PF register sets: while tile it is computed, tiles it+1 .. it+PF are landing
     // or in flight, so a load has PF compute phases to arrive.  Two sets are
@@ -1306,10 +1330,10 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
     // One pipeline step: write the register set holding tile `it` to LDS buffer
     // it&1, barrier, refill that set with tile it+PF (when there is one), then
     // the MFMAs of tile `it`.  One barrier per tile is enough because a buffer
-    // is rewritten only two tiles later.  FAST is a compile-time flag so the
-    // steady-state loop carries no guarded-load code: the guarded path shares
-    // registers with the vector loads and the compiler then serialises every
-    // prefetch behind an s_waitcnt vmcnt(0).
+    // is rewritten only two tiles later.  The steady-state loop carries no
+    // guarded-load code: the guarded path shares registers with the vector
+    // loads and the compiler then serialises every prefetch behind an
+    // s_waitcnt vmcnt(0).
     // the MFMAs of the tile held in LDS at sa / sb
     auto compute = [&](const float *sa, const float *sb) {
         if constexpr (BF16 != 0) {
@@ -1418,8 +1442,18 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
         }
     };
 
-    auto step = [&](int it, int nk, auto fast_tag, auto &la, auto &lb) {
-        constexpr bool FAST = decltype(fast_tag)::value;
+    // stage s without guards, from a range whose stage s starts at k = k0 + s BK
+    auto load_whole = [&](const float *As, const float *Bs, int k0, int s, auto &la, auto &lb) {
+        la.load(As, g.lda, m0, k0 + s * BK, g.M, 0, true, t);
+        lb.load(Bs, g.ldb, n0, k0 + s * BK, g.N, 0, true, t);
+    };
+    auto load = [&](int s, auto &la, auto &lb) {
+        const bool second = s >= nk1, whole = s < (second ? whole2 : whole1); // uniform
+        const int k0 = second ? (s - nk1) * BK : kbeg + s * BK, ke = second ? end2 : end1;
+        la.load(second ? A2 : A, g.lda, m0, k0, g.M, ke, whole, t);
+        lb.load(second ? B2 : B, g.ldb, n0, k0, g.N, ke, whole, t);
+    };
+    auto step = [&](int it, auto next, auto &la, auto &lb) {
         float *sa = smem + (it & 1) * (LDS_A + LDS_B);
         float *sb = sa + LDS_A;
         if constexpr (BF16 != 0) {
@@ -1430,15 +1464,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
             lb.store_f32(sb, t);
         }
         __syncthreads();
-        if (FAST || it + PF < nk) {
-            int k0 = kbeg + (it + PF) * BK;
-            bool kf = FAST || (k0 + BK <= kend);
-            const bool second = k0 >= k1; // uniform
-            const float *Ak = second ? A2 : A, *Bk = second ? B2 : B;
-            const int kr = second ? k0 - k1 : k0, ke = second ? kend - k1 : (kend < k1 ? kend : k1);
-            la.load(Ak, g.lda, m0, kr, g.M, ke, FAST || (a_full && kf), t);
-            lb.load(Bk, g.ldb, n0, kr, g.N, ke, FAST || (b_full && kf), t);
-        }
+        next(it + PF, la, lb);
         // keep the prefetch ahead of the MFMAs: without this fence the
         // scheduler sinks the global loads below the compute block and their
         // latency is paid in full at the next LDS write
@@ -1449,38 +1475,41 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
 #ifdef NCHIP_GEMM_CLOCKS
     long long dbg_c0 = clock64(), dbg_w0 = wall_clock64();
 #endif
-    const int nk = (kend - kbeg + BK - 1) / BK;
-    const int nk_full = (kend - kbeg) / BK; // tiles with a complete k range
     int it = 0;
-    if (a_full && b_full && 2 * PF - 1 < nk_full) {
-        // steady state: tiles it+PF .. it+2PF-1 are complete, unguarded vector loads.  The
-        // first PF tiles are fetched by the same straight-line vector loads as inside the
-        // loop: the compiler then sees one and the same sequence of outstanding loads on
-        // entry and on the back edge and waits for the oldest register set only
-        // (s_waitcnt vmcnt(n)) instead of for everything in flight.
+    // The first PF stages are fetched by the same straight-line vector loads as inside the steady
+    // loop: the compiler then sees one and the same sequence of outstanding loads on entry and on
+    // the back edge and waits for the oldest register set only (s_waitcnt vmcnt(n)) instead of for
+    // everything in flight.
+    if (2 * PF <= whole1) {
 #pragma unroll
         for (int j = 0; j < PF; j++) {
-            la[j].load(A, g.lda, m0, kbeg + j * BK, g.M, kend, true, t);
-            lb[j].load(B, g.ldb, n0, kbeg + j * BK, g.N, kend, true, t);
+            load_whole(A, B, kbeg, j, la[j], lb[j]);
             __builtin_amdgcn_sched_barrier(0); // oldest tile first, as on the back edge
-        }
-        for (; it + 2 * PF - 1 < nk_full; it += PF) {
-#pragma unroll
-            for (int j = 0; j < PF; j++) step(it + j, nk, std::true_type(), la[j], lb[j]);
         }
     } else {
 #pragma unroll
         for (int j = 0; j < PF; j++)
-            if (j < nk) {
-                bool kf = nk_full > j;
-                la[j].load(A, g.lda, m0, kbeg + j * BK, g.M, kend, a_full && kf, t);
-                lb[j].load(B, g.ldb, n0, kbeg + j * BK, g.N, kend, b_full && kf, t);
-            }
+            if (j < nk) load(j, la[j], lb[j]);
+        wait_for_loads();
     }
-    for (; it < nk; it++) { // edge tiles and the k tail (it is a multiple of PF when the loop starts)
+    for (;;) {
+        // steady state: the stages asked for, it + PF .. it + 2 PF - 1, are whole ones of one range
+        const bool second = it + PF >= nk1; // uniform
+        const float *As = second ? A2 : A, *Bs = second ? B2 : B;
+        const int k0 = second ? -nk1 * BK : kbeg, last = (second ? whole2 : whole1) - 2 * PF;
+        for (; it <= last; it += PF) {
+#pragma unroll
+            for (int j = 0; j < PF; j++)
+                step(it + j, [&](int s, auto &la, auto &lb) { load_whole(As, Bs, k0, s, la, lb); }, la[j], lb[j]);
+        }
+        if (it >= nk) break;
+        // around a range's end
 #pragma unroll
         for (int j = 0; j < PF; j++)
-            if (it % PF == j) step(it, nk, std::false_type(), la[j], lb[j]);
+            if (it + j < nk) step(it + j, [&](int s, auto &la, auto &lb) { if (s < nk) load(s, la, lb); }, la[j], lb[j]);
+        it += PF;
+        if (it >= nk) break;
+        wait_for_loads(); // (the steady loop's waits then count its own loads only)
     }
 
 #ifdef NCHIP_GEMM_CLOCKS

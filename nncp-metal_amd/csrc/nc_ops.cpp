@@ -777,7 +777,7 @@ static void matmul_bw(NCNode *nd, NCTensor *g, NCTensor **ga, int ia, int ib)
             m->deferred.push_back(d);
             ga[ia] = da;
         } else if (plain && open_entry && !open_entry->a2 && open_entry->m == (int)s.m &&
-                   open_entry->n == (int)s.k && open_entry->k % 64 == 0 && open_entry->alpha == alpha) {
+                   open_entry->n == (int)s.k && open_entry->alpha == alpha) {
             open_entry->a2 = nc_contig(nc_dup_tensor(g));
             open_entry->b2 = nc_dup_tensor(b);
             open_entry->k2 = (int)s.n;

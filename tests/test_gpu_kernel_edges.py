@@ -429,3 +429,60 @@ def test_fp32_activation_gradient_products_leave_their_row_sums_under_dma(hip, m
     assert np.all(np.abs(c - want) <= 2.0 ** -24 * (k + 1) * (np.abs(dy) @ np.abs(w).T))
     assert 0 < written.value <= rows and np.all(np.abs(rs[: written.value].sum(0) - c.sum(0)) <= 2.0 ** -24 * 16 * np.abs(c).sum(0))
     hip.free(w_t, dy_t, pre_t, c_t, rs_t)
+
+
+@pytest.mark.parametrize("cfg,precision", [(4, 0), (7, 0), (9, 0), (10, 0), (30, 0), (4, 1), (7, 1), (9, 1), (10, 1)])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("m,n,k", [(131, 67, 257), (1, 130, 96), (129, 2, 193), (130, 3, 385), (128, 64, 97)])
+def test_tile_products_at_any_alignment(hip, cfg, precision, ta, tb, m, n, k):
+    """Partial tiles, columns that are no multiple of 4 floats apart and a base 4 bytes off a 16-byte unit: stages
+    without guards up to the last one of a range, whose loads must not pass the operands' ends (they end
+    with their buffers).  Operands are bf16 values, so both precisions form the same products; bound: a
+    rounding per addition."""
+    lib, rng = C.CDLL(hip.lib._name), np.random.default_rng(m * k + n)
+    p, i, j, f = C.c_void_p, C.c_int, C.c_int64, C.c_float
+    lib.nchip_gemm2.argtypes = [p, i, i, i, i, i, f, p, j, j, j, p, j, j, j, f, p, j, j, j, i, i, p, i, p, i, i, p]
+    a, b = rng.standard_normal((m, k) if ta else (k, m)), rng.standard_normal((k, n) if tb else (n, k))
+    a, b = ((x.astype(np.float32).view(np.uint32) & 0xffff0000).view(np.float32) for x in (a, b))
+    a_t, b_t = (hip.tensor(np.concatenate([[np.nan], x.ravel()]).astype(np.float32)) for x in (a, b))
+    c_t = hip.tensor(np.full((n, m), 7.0, np.float32))
+    ptr = lambda t, skip=0: p(hip.nc_tensor_get_ptr(t, None) + 4 * skip)
+    lib.nchip_gemm_force_config(cfg)
+    rc = lib.nchip_gemm2(p(hip.nc_context_stream(hip.ctx)), ta, tb, m, n, k, 1.0, ptr(a_t, 1), k if ta else m, 0, 0, ptr(b_t, 1),
+                         n if tb else k, 0, 0, 0.0, ptr(c_t), m, 0, 0, 1, 1, None, 0, None, precision, 1, None)
+    lib.nchip_gemm_force_config(0)
+    assert rc == 0
+    x, y = (a.T if ta else a).astype(np.float64), (b.T if tb else b).astype(np.float64)  # (k, m), (n, k)
+    assert np.all(np.abs(hip.numpy(c_t) - y @ x) <= 2.0 ** -24 * (k + 1) * (np.abs(y) @ np.abs(x)))
+    hip.free(a_t, b_t, c_t)
+
+
+@pytest.mark.parametrize("m,k,first,second", [(37, 21, 5, 3), (130, 70, 33, 31), (129, 131, 257, 65), (64, 128, 100, 320), (132, 36, 32, 1)])
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_postponed_gradient_of_a_weight_used_over_two_widths(hip, pkg, m, k, first, second, bf16):
+    """One problem of the grouped launch with two ranges of columns, neither a multiple of a stage.  Inputs
+    are bf16 values; bound: a rounding per addition."""
+    B, rng = pkg.binding, np.random.default_rng(m + first)
+    bf = lambda *s: (rng.standard_normal(s).astype(np.float32).view(np.uint32) & 0xffff0000).view(np.float32)
+    xs, gs = [bf(c, k) for c in (first, second)], [bf(c, m) for c in (first, second)]
+    nc = B.NC(hip.lib._name, use_device=True)
+    nc.nc_set_deferred_weight_grad(nc.ctx, 1)
+    nc.nc_set_matmul_bf16(nc.ctx, bf16)
+    h, _ = nc.param(np.zeros((k, m), np.float32))
+    sp = B.SGDOptParams(algo=B.SGD_OPT_BASIC, lr=1.0)
+    opt = nc.nc_sgd_opt_init(nc.ctx, C.byref(sp))
+    nc.nc_sgd_opt_set_all(C.byref(nc.plist), opt)
+    loss = None
+    for x, g in zip(xs, gs):
+        term = nc.nc_sum(nc.nc_mul(nc.nc_matmul(nc.dup(h.value), nc.tensor(x)), nc.tensor(g)))
+        loss = term if loss is None else nc.nc_add(loss, term)
+    nc.lib.nc_backward(loss, nc.nc_new_f32(nc.dev, 1.0), C.cast(nc.lib.sgd_opt_update_var, B.PARAM_UPDATE_FUNC), 0)
+    nc.free(loss)
+    nc.nc_sgd_opt_update(opt)
+    got = -nc.numpy(h.value)
+    nc.nc_sgd_opt_set_all(C.byref(nc.plist), None)
+    nc.nc_sgd_opt_end(opt)
+    nc.close()
+    want = sum(x.astype(np.float64).T @ g for x, g in zip(xs, gs))
+    size = sum(np.abs(x).astype(np.float64).T @ np.abs(g) for x, g in zip(xs, gs))
+    assert np.all(np.abs(got - want) <= 2.0 ** -24 * (first + second + 2) * size)
