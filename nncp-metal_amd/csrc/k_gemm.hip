@@ -1051,43 +1051,45 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
     using chunks = std::make_integer_sequence<int, NP>;
     using const0 = std::integral_constant<int, 0>;
     using const1 = std::integral_constant<int, 1>;
+    if (nk > 0) { // uniform; an empty k range (a chunk past the end, k = 0) has asked for nothing and adds nothing
 #pragma unroll
-    for (int s = 0; s < ST - 1; s++)
-        if (s < nk) each_constant(issue_chunk, std::make_integer_sequence<int, NC>());
-    if (ST - 1 < nk) issue_chunk(const0());
-    // (with fewer stages than ST all of them are waited for)
-    if (nk >= ST) lds_dma_barrier<(ST - 2) * NL + NL / NC>(); else lds_dma_barrier<0>();
-    fetch(0, 0, 0);
-    int at = 0; // the stage being read
-    auto no = [] { return false; };
-    auto body = [&](auto more, int it) {
-        constexpr bool steady = decltype(more)::value;
+        for (int s = 0; s < ST - 1; s++)
+            if (s < nk) each_constant(issue_chunk, std::make_integer_sequence<int, NC>());
+        if (ST - 1 < nk) issue_chunk(const0());
+        // (with fewer stages than ST all of them are waited for)
+        if (nk >= ST) lds_dma_barrier<(ST - 2) * NL + NL / NC>(); else lds_dma_barrier<0>();
+        fetch(0, 0, 0);
+        int at = 0; // the stage being read
+        auto no = [] { return false; };
+        auto body = [&](auto more, int it) {
+            constexpr bool steady = decltype(more)::value;
+            each_constant([&](auto part) {
+                constexpr int u = decltype(part)::value;
+                if constexpr (u < NP - 1) {
+                    fetch(at, u + 1, (u + 1) & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    multiply(part, std::integral_constant<int, u + 1>(), [&] { return steady || it + ST - 1 < nk; });
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }, chunks());
+            if constexpr (steady) lds_dma_barrier<(ST - 2) * NL>();
+            else arrive(nk - 2 - it);
+            at = at + 1 < ST ? at + 1 : 0;
+            if (NC == 1 && (steady || it + ST < nk)) issue_chunk(const0());
+            fetch(at, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(const1(), const0(), [&] { return steady || it + ST < nk; });
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        int it = 0;
+        for (; it + ST < nk; it++) body(std::true_type(), it);
+        for (; it + 1 < nk; it++) body(std::false_type(), it);
         each_constant([&](auto part) {
             constexpr int u = decltype(part)::value;
-            if constexpr (u < NP - 1) {
-                fetch(at, u + 1, (u + 1) & 1);
-                __builtin_amdgcn_sched_barrier(0);
-                multiply(part, std::integral_constant<int, u + 1>(), [&] { return steady || it + ST - 1 < nk; });
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            if constexpr (u + 1 < NP) fetch(at, u + 1, (u + 1) & 1);
+            multiply(part, const0(), no);
         }, chunks());
-        if constexpr (steady) lds_dma_barrier<(ST - 2) * NL>();
-        else arrive(nk - 2 - it);
-        at = at + 1 < ST ? at + 1 : 0;
-        if (NC == 1 && (steady || it + ST < nk)) issue_chunk(const0());
-        fetch(at, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(const1(), const0(), [&] { return steady || it + ST < nk; });
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    int it = 0;
-    for (; it + ST < nk; it++) body(std::true_type(), it);
-    for (; it + 1 < nk; it++) body(std::false_type(), it);
-    each_constant([&](auto part) {
-        constexpr int u = decltype(part)::value;
-        if constexpr (u + 1 < NP) fetch(at, u + 1, (u + 1) & 1);
-        multiply(part, const0(), no);
-    }, chunks());
+    }
 
     // Epilogue.  Every 32 x 32 accumulator tile passes through a corner of LDS (the stages are dead)
     // so that a lane holds four consecutive rows m of columns nl, nl + 8, nl + 16, nl + 24 and moves

@@ -411,6 +411,35 @@ def test_fp32_products_staged_by_dma_keep_the_sums_of_their_class(hip, cls, ta, 
     hip.free(a_t, b_t, bias_t)
 
 
+@pytest.mark.parametrize("cls,ta,tb,m,n,k,batch,ksplit", [(10, 0, 0, 100, 68, 64, 60, 3), (10, 0, 1, 100, 68, 128, 60, 2), (10, 1, 0, 99, 67, 128, 60, 5),
+                                                          (4, 0, 0, 132, 67, 64, 24, 3), (4, 1, 1, 132, 68, 96, 40, 2), (7, 0, 0, 260, 130, 64, 29, 3),
+                                                          (7, 0, 1, 132, 132, 256, 9, 15), (7, 1, 0, 131, 129, 192, 64, 2)])
+def test_fp32_products_split_over_k_under_dma(hip, cls, ta, tb, m, n, k, batch, ksplit):
+    """Chunks of one stage and of several, and splits into more chunks than k has, whose last ones are empty
+    and add nothing: the bits of the tile kernel of the same class, and float64 within a rounding per addition."""
+    lib, rng = C.CDLL(hip.lib._name), np.random.default_rng(m * k + n)
+    p, i, j, f = C.c_void_p, C.c_int, C.c_int64, C.c_float
+    lib.nchip_gemm2.argtypes = [p, i, i, i, i, i, f, p, j, j, j, p, j, j, j, f, p, j, j, j, i, i, p, i, p, i, i, p]
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((batch, m, k) if ta else (batch, k, m), (batch, k, n) if tb else (batch, n, k)))
+    a_t, b_t = hip.tensor(a), hip.tensor(b)
+    ws_t = hip.tensor(np.full(batch * ksplit * m * n, 3.0, np.float32))
+    ptr = lambda t: p(hip.nc_tensor_get_ptr(t, None))
+    got = []
+    for forced in (0, cls):
+        c_t = hip.tensor(np.full((batch, n, m), 7.0, np.float32))
+        lib.nchip_gemm_force_config(forced)
+        rc = lib.nchip_gemm2(p(hip.nc_context_stream(hip.ctx)), ta, tb, m, n, k, 1.0, ptr(a_t), k if ta else m, m * k, 0, ptr(b_t),
+                             n if tb else k, n * k, 0, 0.0, ptr(c_t), m, n * m, 0, batch, 1, None, 0, None, 0, ksplit, ptr(ws_t))
+        lib.nchip_gemm_force_config(0)
+        assert rc == 0
+        got.append(hip.numpy(c_t, free=True))
+    hip.free(a_t, b_t, ws_t)
+    x = (a.transpose(0, 2, 1) if ta else a).astype(np.float64)  # (k, m)
+    y = (b.transpose(0, 2, 1) if tb else b).astype(np.float64)  # (n, k)
+    assert np.array_equal(*got)
+    assert np.all(np.abs(got[0] - y @ x) <= 2.0 ** -24 * (k + 1) * (np.abs(y) @ np.abs(x)))
+
+
 @pytest.mark.parametrize("m,n,k", [(132, 8200, 64), (100, 4100, 96)])
 def test_fp32_activation_gradient_products_leave_their_row_sums_under_dma(hip, m, n, k):
     """nchip_gemm_dact_rowsum through the 128x64 and the two-group 64x64 tiles: the partial rows add up to
