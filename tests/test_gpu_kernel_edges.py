@@ -515,3 +515,42 @@ def test_postponed_gradient_of_a_weight_used_over_two_widths(hip, pkg, m, k, fir
     want = sum(x.astype(np.float64).T @ g for x, g in zip(xs, gs))
     size = sum(np.abs(x).astype(np.float64).T @ np.abs(g) for x, g in zip(xs, gs))
     assert np.all(np.abs(got - want) <= 2.0 ** -24 * (first + second + 2) * size)
+
+
+@pytest.mark.parametrize("m,k,later,earlier", [(37, 21, 5, 3), (130, 70, 33, 31), (352, 352, 585, 481), (128, 128, 64, 100), (128, 256, 448, 33)])
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_postponed_gradient_over_two_widths_is_the_sum_of_two_products(hip, pkg, m, k, later, earlier, bf16):
+    """A weight whose use that is reached first (the later term of the loss) has a number of columns that is no
+    multiple of 64: the bits of the postponed gradient of that use alone plus the product of the other
+    one alone, each in the class of its own shape."""
+    B, rng = pkg.binding, np.random.default_rng(m + later)
+    xs, gs = ([rng.standard_normal((c, d)).astype(np.float32) for c in (earlier, later)] for d in (k, m))
+
+    def gradient(uses, postponed):
+        nc = B.NC(hip.lib._name, use_device=True)
+        nc.nc_set_deferred_weight_grad(nc.ctx, postponed)
+        nc.nc_set_matmul_bf16(nc.ctx, bf16)
+        h, _ = nc.param(np.zeros((k, m), np.float32))
+        sp = B.SGDOptParams(algo=B.SGD_OPT_BASIC, lr=1.0)
+        opt = nc.nc_sgd_opt_init(nc.ctx, C.byref(sp))
+        nc.nc_sgd_opt_set_all(C.byref(nc.plist), opt)
+        loss = None
+        for u in uses:
+            term = nc.nc_sum(nc.nc_mul(nc.nc_matmul(nc.dup(h.value), nc.tensor(xs[u])), nc.tensor(gs[u])))
+            loss = term if loss is None else nc.nc_add(loss, term)
+        nc.lib.nc_backward(loss, nc.nc_new_f32(nc.dev, 1.0), C.cast(nc.lib.sgd_opt_update_var, B.PARAM_UPDATE_FUNC), 0)
+        nc.free(loss)
+        nc.nc_sgd_opt_update(opt)
+        got = -nc.numpy(h.value)
+        nc.nc_sgd_opt_set_all(C.byref(nc.plist), None)
+        nc.nc_sgd_opt_end(opt)
+        nc.close()
+        return got
+
+    # (the later term's use is reached first; with 64 or 448 columns it is joined by the other as a second range)
+    both, alone, other = gradient((0, 1), 1), gradient((1,), 1), gradient((0,), 0)
+    if later % 64:
+        assert np.array_equal(both, alone + other)
+    else:
+        want, size = (sum(f(x).T @ f(g) for x, g in zip(xs, gs)) for f in (lambda a: a.astype(np.float64), lambda a: np.abs(a).astype(np.float64)))
+        assert np.all(np.abs(both - want) <= (2.0 ** -7 * bf16 + 2.0 ** -24 * (later + earlier + 2)) * size)
