@@ -850,8 +850,8 @@ __device__ __forceinline__ void each_constant(F f, std::integer_sequence<int, I.
 // Products of operands that are bf16 in memory, staged by DMA: global memory to LDS without a
 // register in between, ST stages of 64 k in flight, so that a stage is asked for ST - 1 stages
 // before it is read and a wavefront's registers hold accumulators and fragments only (256 x 256
-// tiles fit).  The sums are those of every bf16 class: one chain of v_mfma_f32_32x32x16_bf16 over
-// k for each element, in increasing k.
+// tiles fit).  An element is one chain of v_mfma_f32_32x32x16_bf16 over increasing k or, with NACC = 2,
+// two of them - k % 32 below 16, and from 16 on - that are added (see bf16_two_chains).
 //
 // A stage holds each operand as it lies in memory, in units of 16 bytes.  k contiguous: rows of 64 k,
 // unit c of row i in place c ^ (i / 2 & 7), a fragment is one 16-byte read.  Long axis contiguous: rows
@@ -874,7 +874,7 @@ __device__ __forceinline__ void each_constant(F f, std::integer_sequence<int, I.
 // us before -> now, 512 x 2048 x 512 16.7 -> 14.5, 2048 x 2048 x 512 48.5 -> 42.0, the grouped weight
 // gradients of 12 layers of 512 over 2048 tokens 1571 -> 1361 (133 TFLOP/s).
 constexpr int BOX_LD = 36; // words between the columns of an accumulator tile in LDS
-template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int TA, int TB>
+template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int TA, int TB, int NACC = 1>
 __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0)
 {
     GemmArgs g = g0;
@@ -884,6 +884,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
     constexpr int NVA = BM * 8 / NT, NVB = BN * 8 / NT, NL = NVA + NVB; // 16-byte loads a lane and stage
     constexpr int STAGE = (BM + BN) * 64, NP = KW == 2 ? 2 : 4, NC = F32 ? NP : 1; // a stage in 16-bit words; parts its k is read in, chunks it is asked for in
     static_assert(KW == 1 || (F32 && KW == 2 && TM * TN == 1), "k groups: fp32, one accumulator tile a wavefront");
+    static_assert(NACC == 1 || (!F32 && NACC == 2), "two accumulator sets: bf16");
     static_assert(NVA * NT == BM * 8 && NVB * NT == BN * 8, "whole loads");
     static_assert(ST >= 2 && (ST - 1) * NL <= 63, "the memory counter has six bits");
     static_assert(NG * KW * 32 * BOX_LD * 4 <= ST * STAGE * 2, "the epilogue's corners fit where the stages were");
@@ -993,13 +994,16 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
             return u32x4{ lo.x, lo.y, up.x, up.y };
         }
     };
-    floatx16 acc[TN][TM];
+    floatx16 acc[TN][TM], acc2[NACC == 2 ? TN : 1][NACC == 2 ? TM : 1];
 #pragma unroll
     for (int i = 0; i < TN; i++)
 #pragma unroll
         for (int j = 0; j < TM; j++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; r++) {
+                acc[i][j][r] = 0.0f;
+                if constexpr (NACC == 2) acc2[i][j][r] = 0.0f;
+            }
     u32x4 fa[2][TM], fb[2][TN];
     auto fetch = [&](int stage, int u, int set) {
         const uint16_t NCHIP_LDS *s = stages + stage * STAGE;
@@ -1010,7 +1014,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
         for (int i = 0; i < TN; i++)
             fb[set][i] = fragment(s + BM * 64, std::integral_constant<bool, TB == 0>(), std::integral_constant<int, BN>(), wn * WTN, i, u);
     };
-    // the MFMAs of a part (its parity names the fragments' set), with the loads of a chunk between them
+    // the MFMAs of a part (its parity names the fragments' set and the chain), with the loads of a chunk between them
     // where `on`: a load waits its turn at the CU's address unit, and the MFMAs in front of it go on
     // (fp32, whose MFMAs are long, gains 5-8 %; bf16 loses as much by asking later)
     auto multiply = [&](auto parity, auto chunk, auto on) {
@@ -1022,8 +1026,9 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
             if constexpr (F32) {
                 acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[set][i][s]), __uint_as_float(fa[set][j][s]), acc[i][j], 0, 0, 0);
             } else {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fb[set][i]),
-                                                                    __builtin_bit_cast(bf16x8, fa[set][j]), acc[i][j], 0, 0, 0);
+                floatx16 &chain = *(NACC == 2 && set == 1 ? &acc2[NACC == 2 ? i : 0][NACC == 2 ? j : 0] : &acc[i][j]);
+                chain = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, fb[set][i]),
+                                                                __builtin_bit_cast(bf16x8, fa[set][j]), chain, 0, 0, 0);
             }
             each_constant([&](auto piece) {
                 constexpr int x = decltype(piece)::value;
@@ -1089,6 +1094,14 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
             if constexpr (u + 1 < NP) fetch(at, u + 1, (u + 1) & 1);
             multiply(part, const0(), no);
         }, chunks());
+        if constexpr (NACC == 2) {
+#pragma unroll
+            for (int i = 0; i < TN; i++)
+#pragma unroll
+                for (int j = 0; j < TM; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[i][j][r] += acc2[i][j][r];
+        }
     }
 
     // Epilogue.  Every 32 x 32 accumulator tile passes through a corner of LDS (the stages are dead)
@@ -1906,7 +1919,7 @@ void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec)
 #undef LAUNCH
 }
 
-template <int F32, int BM, int BN, int WM, int WN, int KW, int ST>
+template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int NACC = 1>
 void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int grouped_tiles = 0)
 {
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -1918,11 +1931,11 @@ void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int g
 #define LAUNCH(TA, TB)                                                                                     \
     do {                                                                                                   \
         static const bool ok = hipFuncSetAttribute(                                                        \
-            reinterpret_cast<const void *>(gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB>),                    \
+            reinterpret_cast<const void *>(gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>),                    \
             hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn) == hipSuccess;                           \
         if (!ok) { fprintf(stderr, "nchip_gemm: cannot reserve %zu bytes of LDS\n", dyn); abort(); }      \
-        if (rec) hipExtLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB>), grid, block, dyn, st, rec->start, rec->stop, 0, g); \
-        else hipLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB>), grid, block, dyn, st, g);   \
+        if (rec) hipExtLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>), grid, block, dyn, st, rec->start, rec->stop, 0, g); \
+        else hipLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>), grid, block, dyn, st, g);   \
     } while (0)
     if (!ta && !tb) LAUNCH(0, 0);
     else if (ta && !tb) LAUNCH(1, 0);
@@ -1943,18 +1956,25 @@ void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int g
 //   1024 x 4096 x 4096     96 /  59 /  43 /  53 /  64   before  52
 //   1024 x 2048 x 3072     71 /  39 /  30 /  24 /  28   before  33
 //   512 x 2048 x 2048      47 /  21 /  19 /  13 /  10   before  13
-static int dma_class(int m, int n)
+// (two chains: no room for the second accumulators in 256 x 256 tiles, nor twice a CU in classes of 64 x 64 a wavefront)
+static int dma_class(int m, int n, bool two_chains)
 {
     auto tiles = [&](int bm, int bn) { return (int64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
     const int64_t t256 = tiles(256, 256), t128 = tiles(128, 128);
-    if (8 * t256 >= 7 * 256 * ((t256 + 255) / 256)) return 4;
-    if (t128 >= 448) return 1;
+    if (!two_chains && 8 * t256 >= 7 * 256 * ((t256 + 255) / 256)) return 4;
+    if (!two_chains && t128 >= 448) return 1;
     if (t128 >= 224) return 5;
     return tiles(128, 64) >= 224 && m >= 128 ? 2 : 3;
 }
 
-static void launch_dma_class(hipStream_t st, int cls, int ta, int tb, GemmArgs &g, ProfRec *rec)
+static void launch_dma_class(hipStream_t st, int cls, bool two_chains, int ta, int tb, GemmArgs &g, ProfRec *rec)
 {
+    if (two_chains) {
+        if (cls == 1 || cls == 5) launch_dma<0, 128, 128, 2, 4, 1, 4, 2>(st, ta, tb, g, rec);
+        else if (cls == 2) launch_dma<0, 128, 64, 2, 2, 1, 3, 2>(st, ta, tb, g, rec);
+        else launch_dma<0, 64, 64, 2, 2, 1, 4, 2>(st, ta, tb, g, rec);
+        return;
+    }
     if (cls == 4) launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, rec);
     else if (cls == 1) launch_dma<0, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, rec);
     else if (cls == 5) launch_dma<0, 128, 128, 2, 4, 1, 4>(st, ta, tb, g, rec);
@@ -2058,6 +2078,25 @@ static int gemm_class(int m, int n, int64_t nb)
     if (tm * ((n + 127) / 128) * nb >= 512 && m >= 128 && n >= 128) return 7;
     if (tm * ((n + 63) / 64) * nb >= 256 && m >= 128 && n >= 64) return 4;
     return 10;
+}
+
+// Whether a product with operands rounded to bf16 rounds them in memory first: below that the extra
+// pass over them costs more than the tiles save.
+static bool rounds_in_memory(int m, int n, int k)
+{
+    return k > 0 && (g_bf16src == 2 || (g_bf16src == 1 && m >= 128 && n >= 128 && k >= 256 && 2.0 * m * n * (double)k >= g_bf16src_min_flops));
+}
+
+// Chains over k of an element of such a product: two, added, where the output has few tiles - fewer than
+// 512 of 128x128 from rounded copies, the 64x64 class where the tile loader rounds - and one
+// elsewhere.  Precision, not time, keeps the two: their rms error is 0.70 times that of one chain
+// (k = 1000 to 10000), at the same speed up to 447 tiles and 0.91 times it above (2000 x 3500 x 1000 34.2
+// us in one chain, 37.7 in two).
+static bool bf16_two_chains(int m, int n, int k)
+{
+    if (!rounds_in_memory(m, n, k)) return gemm_class(m, n, 1) == 10;
+    if (g_force_cfg == 11 || g_force_cfg == 13) return g_force_cfg == 11; // tuning aid
+    return (int64_t)((m + 127) / 128) * ((n + 127) / 128) < 512;
 }
 
 // Whether an fp32 product of the 64x64 class is issued by gemm_small_kernel (the same sums; this is
@@ -2195,9 +2234,8 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     // the ones the conversion inside the tile loader would produce, so the
     // result is the same either way.
     bool from_bf16 = false;
-    if (precision == 1 && batch == 1 && ksplit == 1 && !invariant && k > 0 && m < 1 << 21 && n < 1 << 21 && k < 1 << 21 && // (32-bit offsets)
-        (g_bf16src == 2 || (g_bf16src == 1 && m >= 128 && n >= 128 && k >= 256 &&
-                            2.0 * m * n * (double)k >= g_bf16src_min_flops))) {
+    if (precision == 1 && batch == 1 && ksplit == 1 && !invariant && m < 1 << 21 && n < 1 << 21 && k < 1 << 21 && // (32-bit offsets)
+        rounds_in_memory(m, n, k)) {
         const int kpad = (k + 63) / 64 * 64;
         const size_t ea = cast_elems(ta ? k : m, ta ? m : k, ta != 0, kpad);
         const size_t eb = cast_elems(tb ? n : k, tb ? k : n, tb == 0, kpad);
@@ -2221,7 +2259,8 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
         *rowsum_rows = (n + bn - 1) / bn * bn / (dma && cfg == 10 ? 8 : 16);
     }
     if (from_bf16) {
-        launch_dma_class(st, dma_class(m, n), ta, tb, g, pr);
+        const bool two_chains = bf16_two_chains(m, n, k);
+        launch_dma_class(st, dma_class(m, n, two_chains), two_chains, ta, tb, g, pr);
     } else if (precision == 1) {
         if (cfg == 7) launch_tile<128, 128, 32, 4, 2, 1>(st, ta, tb, g, pr);
         else if (cfg == 4) launch_tile<128, 64, 32, 4, 2, 1>(st, ta, tb, g, pr);
@@ -2505,7 +2544,12 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
     g.batch_in = 1; g.M = m; g.N = n; g.K = k; g.batch = 1; g.ksplit = 1; g.kchunk = k;
     g.alpha = a->alpha; g.beta = 0.0f; g.act = act_for_precision(a->act, 2);
     hipStream_t st = (hipStream_t)stream;
-    const int cls = g_bf16ops_cls >= 1 && g_bf16ops_cls <= 5 ? g_bf16ops_cls : dma_class(m, n);
+    // One chain where the operands whose long axis is contiguous fill the tiles that cover the chip (128x128 from
+    // 224 of them on, then 128x64, else 64x64); elsewhere the sums of nchip_gemm with precision 1.
+    const int64_t t128 = (int64_t)((m + 127) / 128) * ((n + 127) / 128), t128x64 = (int64_t)((m + 127) / 128) * ((n + 63) / 64);
+    const int bm = t128 >= 224 || (t128x64 >= 224 && m >= 128) ? 128 : 64, bn = t128 >= 224 ? 128 : 64;
+    const bool whole = (ta || m % bm == 0) && (!tb || n % bn == 0), two_chains = !whole && bf16_two_chains(m, n, k);
+    const int cls = g_bf16ops_cls >= 1 && g_bf16ops_cls <= 5 && !(two_chains && g_bf16ops_cls == 4) ? g_bf16ops_cls : dma_class(m, n, two_chains);
     if (a->rowsum && a->rows_written && a->dpre) {
         const int bn = cls == 4 ? 256 : (cls == 1 || cls == 5 ? 128 : 64);
         g.rowsum = a->rowsum;
@@ -2519,7 +2563,7 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
         rec.variant = 64 + cls * 4 + ta * 2 + tb; // the bf16-operand classes
     }
     ProfRec *pr = g_prof_on ? &rec : nullptr;
-    launch_dma_class(st, cls, ta, tb, g, pr);
+    launch_dma_class(st, cls, two_chains, ta, tb, g, pr);
     if (g_prof_on) g_prof.push_back(rec);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {

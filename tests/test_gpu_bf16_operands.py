@@ -376,3 +376,47 @@ def test_grouped_launch_in_wide_tiles(hip, raw, rng):
     for two, three in zip(outs[2], outs[3]):
         assert np.array_equal(hip.numpy(two), hip.numpy(three))
     hip.free(*keep, *outs[2], *outs[3])
+
+
+def _precision_1(lib, st, ptr, ta, tb, m, n, k, a_t, b_t, c_t):
+    p, i, j, f = C.c_void_p, C.c_int, C.c_int64, C.c_float
+    lib.nchip_gemm.argtypes = [p, i, i, i, i, i, f, p, j, j, p, j, j, f, p, j, j, i, p, i, p, i, i, p]
+    return lib.nchip_gemm(st, ta, tb, m, n, k, 1.0, ptr(a_t), k if ta else m, 0, ptr(b_t), n if tb else k, 0, 0.0, ptr(c_t), m, 0, 1,
+                          None, 0, None, 1, 1, None)
+
+
+@pytest.mark.parametrize("ta,tb,m,n,k", [(0, 0, 100, 67, 64), (1, 0, 130, 131, 200), (0, 1, 257, 96, 352), (1, 1, 65, 300, 129), (0, 1, 128, 256, 1024)])
+def test_products_from_rounded_copies_keep_two_chains_below_512_tiles(hip, raw, rng, ta, tb, m, n, k):
+    """nchip_gemm with precision 1 through rounded copies: the bits of the tile loader's rounding in the 64x64
+    class, which gives an element two chains over k, and with one chain forced those of the 128x128 class."""
+    lib, st, ptr = raw
+    a_t, b_t = (hip.tensor(rng.standard_normal(s).astype(np.float32)) for s in ((m, k) if ta else (k, m), (k, n) if tb else (n, k)))
+    got = []
+    for source, config in ((2, 0), (0, 10), (2, 11), (2, 13), (0, 7)):
+        c_t = hip.tensor(np.full((n, m), 7.0, np.float32))
+        lib.nchip_gemm_bf16_source(source)
+        lib.nchip_gemm_force_config(config)
+        rc = _precision_1(lib, st, ptr, ta, tb, m, n, k, a_t, b_t, c_t)
+        lib.nchip_gemm_force_config(0)
+        lib.nchip_gemm_bf16_source(1)
+        assert rc == 0
+        got.append(hip.numpy(c_t, free=True))
+    hip.free(a_t, b_t)
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[2], got[1])
+    assert np.array_equal(got[3], got[4])
+    assert not np.array_equal(got[0], got[3])
+
+
+@pytest.mark.parametrize("ta,tb,m,n,k", [(0, 0, 192, 7110, 64), (0, 0, 192, 8200, 64), (1, 1, 130, 14272, 64)])
+def test_bf16_operands_that_do_not_fill_their_tiles_have_the_sums_of_the_general_call(hip, raw, rng, ta, tb, m, n, k):
+    """192 rows in 128-wide tiles, columns that are a multiple of 64 and not of 128: the bits of nchip_gemm with
+    precision 1, whose class for the shape has one chain over k or two."""
+    lib, st, ptr = raw
+    a, b = (rng.standard_normal(s).astype(np.float32) for s in ((m, k) if ta else (k, m), (k, n) if tb else (n, k)))
+    a_t, b_t, c_t, d_t, a16, b16 = (hip.tensor(x) for x in (a, b, np.full((n, m), 7.0, np.float32), np.full((n, m), 8.0, np.float32),
+                                                             bf16_round(a)[1], bf16_round(b)[1]))
+    assert _precision_1(lib, st, ptr, ta, tb, m, n, k, a_t, b_t, c_t) == 0
+    g = Args(ta=ta, tb=tb, m=m, n=n, k=k, alpha=1.0, A16=ptr(a16), B16=ptr(b16), lda=k if ta else m, ldb=n if tb else k, C=ptr(d_t), ldc=m)
+    assert lib.nchip_gemm_bf16_operands(st, C.byref(g)) == 0
+    assert np.array_equal(hip.numpy(c_t), hip.numpy(d_t))
+    hip.free(a_t, b_t, c_t, d_t, a16, b16)
