@@ -99,6 +99,10 @@ typedef struct {
 } NchipGemmProblem;
 int nchip_gemm_grouped_tiles(int m, int n);
 int nchip_gemm_grouped_tiles256(int m, int n); /* the same for precision 3 */
+int nchip_gemm_grouped_tiles64(int m, int n);  /* and for precisions 5 and 6 */
+/* whether nchip_gemm (precision 0 or 1, ksplit 1, no forced class) sums an element of this product in two
+   chains over k, k % 32 below 16 and from 16 on, rather than in one */
+int nchip_gemm_two_chains(int m, int n, int k, int precision);
 /* precision 0: fp32; 1: fp32 operands rounded to bf16 in the tile loader; 2: the operand
    pointers of the table address bf16 copies (2 bytes per element, same layout and leading
    dimensions as the fp32 matrices they were rounded from), read with unguarded 16-byte
@@ -107,7 +111,9 @@ int nchip_gemm_grouped_tiles256(int m, int n); /* the same for precision 3 */
    aligned; the caller checks; 3: as 2 in 256x256 tiles, tile_start and total_tiles counted by
    nchip_gemm_grouped_tiles256; 4: fp32 operands as 0, by whole 16-byte units: every k and k2 a
    multiple of 32, every row-contiguous extent and leading dimension a multiple of 4, bases
-   16-byte aligned.  C is fp32 in all of them. */
+   16-byte aligned; 5 and 6: operands as for 0 and 1, in 64x64 tiles and two chains over k, ADDED to
+   what C holds, no A2 / B2; tile_start and total_tiles by nchip_gemm_grouped_tiles64.  C is fp32 in
+   all of them. */
 int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmProblem *dev_table,
                        int n_problems, int total_tiles, int precision, double total_flops);
 

@@ -1892,13 +1892,13 @@ constexpr size_t lds_dynamic_bytes()
 }
 
 template <int BM, int BN, int BK, int WM, int WN, int BF16, int KW = 1, int PF = 2, int NACC = 1, int FRAG = 0>
-void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec)
+void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int grouped_tiles = 0)
 {
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
     g.gm = g_force_gm >= 0 ? g_force_gm : 8;
     g.dbg = 0;
-    dim3 grid(g.tiles_m * g.tiles_n, g.batch * g.ksplit), block(64 * WM * WN * KW);
+    dim3 grid(grouped_tiles ? grouped_tiles : g.tiles_m * g.tiles_n, g.batch * g.ksplit), block(64 * WM * WN * KW);
 #define LAUNCH(TA, TB)                                                                                     \
     do {                                                                                                   \
         constexpr size_t dyn = lds_dynamic_bytes<BM, BN, BK, TA, TB, BF16>();                              \
@@ -2097,6 +2097,11 @@ static bool bf16_two_chains(int m, int n, int k)
     if (!rounds_in_memory(m, n, k)) return gemm_class(m, n, 1) == 10;
     if (g_force_cfg == 11 || g_force_cfg == 13) return g_force_cfg == 11; // tuning aid
     return (int64_t)((m + 127) / 128) * ((n + 127) / 128) < 512;
+}
+
+extern "C" int nchip_gemm_two_chains(int m, int n, int k, int precision)
+{
+    return precision == 1 ? bf16_two_chains(m, n, k) : gemm_class(m, n, 1) == 10;
 }
 
 // Whether an fp32 product of the 64x64 class is issued by gemm_small_kernel (the same sums; this is
@@ -2640,6 +2645,11 @@ extern "C" int nchip_gemm_grouped_tiles256(int m, int n)
     return ((m + 255) / 256) * ((n + 255) / 256);
 }
 
+extern "C" int nchip_gemm_grouped_tiles64(int m, int n)
+{
+    return ((m + 63) / 64) * ((n + 63) / 64);
+}
+
 extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmProblem *dev_table,
                                   int n_problems, int total_tiles, int precision, double total_flops)
 {
@@ -2652,14 +2662,15 @@ extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmP
     // are long enough for the XCDs to finish apart (1692 us)
     { static const int gc = getenv("NCHIP_GRP_CHUNK") ? atoi(getenv("NCHIP_GRP_CHUNK")) : 16; g.grp_chunk = gc; }
     g.batch = 1; g.batch_in = 1; g.ksplit = 1;
-    g.beta = 0.0f; g.act = 0;
+    g.beta = precision >= 5 ? 1.0f : 0.0f; g.act = 0;
     hipStream_t st = (hipStream_t)stream;
     dim3 grid(total_tiles, 1), block(512);
     ProfRec rec;
     if (g_prof_on) {
         (void)hipEventCreate(&rec.start);
         (void)hipEventCreate(&rec.stop);
-        rec.variant = precision >= 2 ? (precision == 4 ? 88 : precision == 3 ? 64 : 32) + (ta ? 2 : 0) + (tb ? 1 : 0)
+        rec.variant = precision >= 5 ? 3 * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 6 ? 1 : 0)
+                    : precision >= 2 ? (precision == 4 ? 88 : precision == 3 ? 64 : 32) + (ta ? 2 : 0) + (tb ? 1 : 0)
                                      : 2 * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 1 ? 1 : 0);
         rec.flops = total_flops;
     }
@@ -2675,7 +2686,11 @@ extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmP
         else hipLaunchKernelGGL(KERNEL, grid, block, dyn, st, g);                                          \
     } while (0)
 #define GRP(TA, TB, BF) GRP_LAUNCH((gemm_kernel<128, 128, 32, 4, 2, TA, TB, BF, 1, 2, 1, (BF == 0)>), 32, TA, TB, BF)
-    if (precision == 4) {
+    if (precision == 6) {
+        launch_tile<64, 64, 32, 2, 2, 1, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+    } else if (precision == 5) {
+        launch_tile<64, 64, 32, 2, 2, 0, 2, 4>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+    } else if (precision == 4) {
         launch_dma<1, 128, 128, 4, 2, 1, 4>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
     } else if (precision == 3) {
         launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);

@@ -47,7 +47,8 @@ struct NCNode;
 struct DeferredGemm {
     NCTensor *a, *b, *c;   // c (m x n) = alpha * (a (m x k) * b^T + a2 (m x k2) * b2^T), b is n x k
     NCTensor *a2, *b2;     // second use of the same weight (or NULL)
-    NCTensor *part;        // the first use's gradient, where the second is a product of its own added to it (else NULL)
+    bool own;              // the second use is a product of its own, added to the first one's:
+    NCTensor *part;        // in a grouped launch behind it (NULL), or alone, from here, where the first one's goes then
     int m, n, k, k2;
     float alpha;
     const NCNode *param;   // the parameter this gradient belongs to

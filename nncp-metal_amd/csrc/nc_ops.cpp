@@ -633,6 +633,12 @@ extern "C" void nc_forget_k_major_weights(NCContext *m)
     m->k_major.clear();
 }
 
+static bool fits_bf16_operands(const NCContext *m, bool ta, bool tb, size_t M, size_t N, size_t K)
+{
+    static const bool off = getenv("NCHIP_BF16_SHADOWS") && atoi(getenv("NCHIP_BF16_SHADOWS")) == 0;
+    return !off && m->matmul_bf16 && K % 64 == 0 && K >= 64 && M >= 64 && N >= 16 && (ta || M % 64 == 0) && (!tb || N % 64 == 0);
+}
+
 // The product through the operands' bf16 shadows (bf16 mode, plain unbatched products whose
 // shape the unguarded loaders take): no operand is converted inside the product, and none is
 // cast more than once however many products read it.  want_c16: also leave the result's own
@@ -643,10 +649,8 @@ static bool dev_gemm_bf16_operands(NCContext *m, bool ta, bool tb, size_t M, siz
                                    const NCTensor *a, const NCTensor *b, NCTensor *c, const float *bias, int act,
                                    float *pre, const float *addend, bool want_c16, const Bf16Extra *ex = nullptr)
 {
-    static const bool off = getenv("NCHIP_BF16_SHADOWS") && atoi(getenv("NCHIP_BF16_SHADOWS")) == 0;
-    if (off || !m->matmul_bf16 || K % 64 || K < 64 || M < 64 || N < 16) return false;
+    if (!fits_bf16_operands(m, ta, tb, M, N, K)) return false;
     const size_t lda = ta ? K : M, ldb = tb ? N : K;
-    if (lda % 8 || ldb % 8 || (!ta && M % 64) || (tb && N % 64)) return false;
     const uint16_t *a16 = nc_shadow_of(m, a), *b16 = a16 ? nc_shadow_of(m, b) : nullptr;
     if (!a16 || !b16) return false;
     NchipGemmBf16Args g;
@@ -764,10 +768,10 @@ static void matmul_bw(NCNode *nd, NCTensor *g, NCTensor **ga, int ia, int ib)
         // or twice (K/V of the segment and of the memory): postponed to the
         // grouped launch at the end of nc_backward; the second use joins the
         // first as a second k range of the same problem where that one is a multiple
-        // of 64 columns.  With other counts the gradient stays the sum of two products, of the
-        // same sums as ever: the second, in the class of its shape, follows the launch and
-        // takes the first as its addend.  (One chain over both is no faster - 5 layers of 352, a pass:
-        // 3.12 ms against 3.08 - and its rms error is 1.6 times theirs: 352 x 352 over 585 and 481 columns.)
+        // of 64 columns.  With other counts the gradient stays the sum of two products with the sums of
+        // their shapes' classes (one chain over both has 1.6 times their rms error: 352 x 352 over 585 and
+        // 481 columns): the second ones of the 64x64 class go in a grouped launch of their own
+        // that adds to the first's results, any other follows alone with the first's as its addend.
         DeferredGemm *open_entry = nullptr;
         for (DeferredGemm &e : m->deferred)
             if (e.param == pa) open_entry = &e;
@@ -775,7 +779,7 @@ static void matmul_bw(NCNode *nd, NCTensor *g, NCTensor **ga, int ia, int ib)
         if (plain && !open_entry && pa->consumers <= 2) {
             DeferredGemm d;
             d.a = nc_contig(nc_dup_tensor(g)); d.b = nc_dup_tensor(b); d.c = nc_dup_tensor(da);
-            d.a2 = d.b2 = d.part = nullptr; d.k2 = 0;
+            d.a2 = d.b2 = d.part = nullptr; d.k2 = 0; d.own = false;
             d.m = (int)s.m; d.n = (int)s.k; d.k = (int)s.n; d.alpha = alpha;
             d.param = pa;
             m->deferred.push_back(d);
@@ -786,8 +790,13 @@ static void matmul_bw(NCNode *nd, NCTensor *g, NCTensor **ga, int ia, int ib)
             open_entry->b2 = nc_dup_tensor(b);
             open_entry->k2 = (int)s.n;
             // the first use's tensor receives the whole gradient
-            if (open_entry->k % 64 == 0) nc_free_tensor(da);
-            else open_entry->part = da;
+            open_entry->own = open_entry->k % 64 != 0;
+            if (open_entry->own && !(alpha == 1.0f && !fits_bf16_operands(m, false, true, s.m, s.k, s.n) &&
+                                     nchip_gemm_pick_ksplit((int)s.m, (int)s.k, (int)s.n, 1) == 1 &&
+                                     nchip_gemm_two_chains((int)s.m, (int)s.k, (int)s.n, m->matmul_bf16)))
+                open_entry->part = da;
+            else
+                nc_free_tensor(da);
         } else {
             const float *prev = nc_bw_addend(m, ia, nc_numel(da));
             if (!ta) dev_gemm(m, false, !tb, s.m, s.k, s.n, alpha, g, b, 0.0f, da, s.batch, nullptr, 0, nullptr, prev);
@@ -1621,10 +1630,10 @@ extern "C" float nc_exp_det(float x)
 static void flush_deferred_gemms(NCContext *m)
 {
     if (m->deferred.empty()) return;
-    std::vector<NchipGemmProblem> tab;
-    int tiles = 0;
-    double flops = 0.0;
-    auto joined_k = [](const DeferredGemm &d) { return d.a2 && !d.part ? d.k2 : 0; };
+    std::vector<NchipGemmProblem> tab, tab2; // (tab2: second uses that are added to the first one's results)
+    int tiles = 0, tiles2 = 0;
+    double flops = 0.0, flops2 = 0.0;
+    auto joined_k = [](const DeferredGemm &d) { return d.a2 && !d.own ? d.k2 : 0; };
     // longest reductions first: their tiles run longest and would otherwise
     // form the tail of the launch
     std::stable_sort(m->deferred.begin(), m->deferred.end(), [&](const DeferredGemm &x, const DeferredGemm &y) {
@@ -1639,7 +1648,7 @@ static void flush_deferred_gemms(NCContext *m)
     std::vector<const uint16_t *> sh;
     if (from_shadows) {
         for (const DeferredGemm &d : m->deferred) {
-            const NCTensor *ops[4] = { d.a, d.b, d.part ? nullptr : d.a2, d.part ? nullptr : d.b2 };
+            const NCTensor *ops[4] = { d.a, d.b, d.own ? nullptr : d.a2, d.own ? nullptr : d.b2 };
             for (const NCTensor *t : ops) {
                 const uint16_t *q = t ? nc_shadow_of(m, t) : nullptr;
                 if (t && !q) from_shadows = false;
@@ -1658,7 +1667,7 @@ static void flush_deferred_gemms(NCContext *m)
     bool units = !from_shadows && !m->matmul_bf16;
     for (const DeferredGemm &d : m->deferred) {
         if (d.k < 32 || d.k % 32 || joined_k(d) % 32 || d.m % 4 || d.n % 4 || d.m >= 1 << 22 || d.n >= 1 << 22) units = false;
-        for (const NCTensor *t : { d.a, d.b, d.part ? nullptr : d.a2, d.part ? nullptr : d.b2 })
+        for (const NCTensor *t : { d.a, d.b, d.own ? nullptr : d.a2, d.own ? nullptr : d.b2 })
             if (t && ((uintptr_t)nc_f32(t) & 15)) units = false;
     }
     size_t di = 0;
@@ -1680,16 +1689,32 @@ static void flush_deferred_gemms(NCContext *m)
         p.tile_start = tiles; p.alpha = d.alpha;
         tiles += wide ? nchip_gemm_grouped_tiles256(d.m, d.n) : nchip_gemm_grouped_tiles(d.m, d.n);
         tab.push_back(p);
+        if (d.own && !d.part) {
+            p.A = nc_f32(d.a2); p.B = nc_f32(d.b2); p.A2 = p.B2 = nullptr;
+            p.k = d.k2; p.k2 = 0;
+            flops2 += 2.0 * d.m * d.n * (double)d.k2;
+            p.tile_start = tiles2;
+            tiles2 += nchip_gemm_grouped_tiles64(d.m, d.n);
+            tab2.push_back(p);
+        }
     }
+    const size_t n_first = tab.size();
+    tab.insert(tab.end(), tab2.begin(), tab2.end());
     size_t bytes = tab.size() * sizeof(NchipGemmProblem), hcap, dcap;
     void *host = m->host_pool.get(bytes, &hcap);
     void *dev = m->dev_pool.get(bytes, &dcap);
     memcpy(host, tab.data(), bytes);
     hip_check(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, m->stream), "hipMemcpyAsync gemm table");
-    if (nchip_gemm_grouped(m->stream, 0, 1, (const NchipGemmProblem *)dev, (int)tab.size(), tiles,
+    if (nchip_gemm_grouped(m->stream, 0, 1, (const NchipGemmProblem *)dev, (int)n_first, tiles,
                            wide ? 3 : (from_shadows ? 2 : (units ? 4 : m->matmul_bf16)), flops))
         nc_fatal("grouped weight-gradient GEMM failed");
     m->launches++;
+    if (tiles2) {
+        if (nchip_gemm_grouped(m->stream, 0, 1, (const NchipGemmProblem *)dev + n_first, (int)tab2.size(), tiles2,
+                               m->matmul_bf16 ? 6 : 5, flops2))
+            nc_fatal("grouped weight-gradient GEMM failed");
+        m->launches++;
+    }
     // pinned staging is recycled one flush later, after a wait for the stream
     nc_staging_retire(m, m->grp_staging, m->grp_staging_cap, m->grp_staging_stamp);
     m->grp_staging = host; m->grp_staging_cap = hcap; m->grp_staging_stamp = m->sync_count;

@@ -517,7 +517,7 @@ def test_postponed_gradient_of_a_weight_used_over_two_widths(hip, pkg, m, k, fir
     assert np.all(np.abs(got - want) <= 2.0 ** -24 * (first + second + 2) * size)
 
 
-@pytest.mark.parametrize("m,k,later,earlier", [(37, 21, 5, 3), (130, 70, 33, 31), (352, 352, 585, 481), (128, 128, 64, 100), (128, 256, 448, 33)])
+@pytest.mark.parametrize("m,k,later,earlier", [(37, 21, 5, 3), (130, 70, 33, 31), (352, 352, 585, 481), (128, 128, 64, 100), (128, 256, 448, 33), (128, 128, 33, 64), (64, 96, 33, 1100)])
 @pytest.mark.parametrize("bf16", [0, 1])
 def test_postponed_gradient_over_two_widths_is_the_sum_of_two_products(hip, pkg, m, k, later, earlier, bf16):
     """A weight whose use that is reached first (the later term of the loss) has a number of columns that is no
