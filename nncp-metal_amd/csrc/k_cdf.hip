@@ -341,6 +341,7 @@ __global__ __launch_bounds__(TPB) void cdf_lookup_kernel(const uint16_t *cdf, co
 // 256 MB: 64.7 -> 48.0 us; one column of 10^6: 33.6 -> 9.6 us.
 typedef unsigned short ushortx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int INV_NT = 1024, INV_ROWS = 65536 / (8 * INV_NT); // a row: 8 entries of every thread
 __device__ __forceinline__ uint32_t max2(uint32_t a, uint32_t b)
 {
@@ -412,13 +413,13 @@ __global__ __launch_bounds__(INV_NT) void cdf_lookup_table_kernel(const uint16_t
     __syncthreads();
     const uint16_t *tp = target + (int64_t)blockIdx.y * m;
     uint16_t *sp = sym + (int64_t)blockIdx.y * m;
-    // units of 8 targets from the first 16-byte boundary of the column on (vec: its symbols have theirs
-    // at the same place), this workgroup's share of them; the first workgroup takes what is left
+    // units of 8 targets from the first 16-byte boundary of the column on (vec: its symbols are at least
+    // 4-byte aligned there), this workgroup's share of them; the first workgroup takes what is left
     const int64_t head0 = vec ? ((16 - ((uintptr_t)tp & 15)) & 15) >> 1 : m, head = head0 < m ? head0 : m;
     const int64_t units = (m - head) >> 3, per = (units + gridDim.x - 1) / gridDim.x;
     const int64_t u0 = per * blockIdx.x, u1 = u0 + per < units ? u0 + per : units;
     const u32x4 *t4 = reinterpret_cast<const u32x4 *>(tp + head);
-    u32x4 *s4 = reinterpret_cast<u32x4 *>(sp + head);
+    u32x4_u *s4 = reinterpret_cast<u32x4_u *>(sp + head);
     // two units a lane in flight while the two before them are looked up (index clamped, store guarded)
     u32x4 cur[2], nxt[2];
     if (u0 < u1) {
@@ -450,7 +451,7 @@ __global__ __launch_bounds__(INV_NT) void cdf_lookup_table_kernel(const uint16_t
             const int64_t rest = head + 8 * units + t;
             if (t < 8 && rest < m) sp[rest] = inv[tp[rest]];
         }
-    } else { // targets and symbols aligned differently: one at a time
+    } else { // an odd number of elements between their alignments: one at a time
         const int64_t share = (m + gridDim.x - 1) / gridDim.x, i1 = share * (blockIdx.x + 1);
         for (int64_t i = share * blockIdx.x + t; i < (i1 < m ? i1 : m); i += INV_NT) sp[i] = inv[tp[i]];
     }
@@ -621,8 +622,9 @@ extern "C" int nchip_cdf_lookup(void *stream, const uint16_t *cdf, const uint16_
             const int64_t cost = (s * n + 255) / 256 * (CDF_TABLE_COST + (m + s - 1) / s);
             if (cost < best) { best = cost; split = s; }
         }
-        // 16-byte accesses from each column's first boundary on: the same place in targets and symbols
-        const int vec = (((uintptr_t)target ^ (uintptr_t)sym) & 15) == 0;
+        // 16-byte accesses from each column's first boundary in the targets on; stores need 4-byte
+        // alignment (us, 256 x 64 and 16384 x 64, 10^6 lookups each: 43 and 49, one value at a time 84 and 96)
+        const int vec = (((uintptr_t)target ^ (uintptr_t)sym) & 3) == 0;
         hipLaunchKernelGGL(cdf_lookup_table_kernel, dim3((unsigned)split, (unsigned)n), dim3(INV_NT), 65536 * 2,
                            (hipStream_t)stream, cdf, target, sym, v, m, vec);
     } else {
