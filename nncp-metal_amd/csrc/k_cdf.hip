@@ -612,9 +612,14 @@ extern "C" int nchip_cdf_lookup(void *stream, const uint16_t *cdf, const uint16_
     // Table or search, both measured (us; v x columns, lookups a column): 256 x 64, 32768 6.5 search,
     // 7.3 table; 65536 9.1, 8.2; 10^6 99, 43; 1000 x 40, 65536 8.8, 7.7; 2048 x 8, 2000 5.1, 7.0, 4001
     // 8.2, 7.0; 16384 x 1, 1000 5.2, 9.3, 4001 13.2, 9.3; 16384 x 64, 10^6 576, 48.  A search is
-    // log2 v dependent LDS reads behind the staging of its column, a table two passes over LDS.
+    // log2 v dependent LDS reads behind the staging of its column, a table two passes over LDS.  More columns
+    // than CUs take their tables in turns, which short columns do not pay for: 2048 x 300, 4001 12.6, 13.2, 5000
+    // 14.1, 13.1; x 4096, 4001 83, 106, 5000 101, 103, 6000 121, 103; 4096 x 1000, 4001 29.3, 27.8, x 4096 106, 115;
+    // 16384 x 4096, 4001 165, 173, 5000 205, 169; above 16384 symbols, where the search reads global memory,
+    // they do (32768 x 4096, 4001 615, 352).
     static const bool table_ok = allow_table_lds();
-    if (table_ok && (v >= 2048 ? m >= 4000 : m >= 32768 && m * n >= 4 << 20)) {
+    const bool turns = v <= 16384 && n > (v < 4096 ? 256 : 1024);
+    if (table_ok && (v >= 2048 ? m >= (turns ? 5120 : 4000) : m >= 32768 && m * n >= 4 << 20)) {
         // one workgroup a CU (the table fills its LDS): the split of a column whose rounds of
         // workgroups, each a table and a share of at least 4096 lookups, take the least time
         int64_t split = 1, best = INT64_MAX;

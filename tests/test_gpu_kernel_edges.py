@@ -362,7 +362,8 @@ def test_gradients_of_a_parameter_used_three_times(hip, m, k, cols, ta):
 
 
 @pytest.mark.parametrize("v,n,m,to,so", [(2048, 2, 4000, 0, 0), (2049, 3, 4007, 3, 3), (16385, 1, 8195, 1, 0),
-                                         (65535, 1, 4001, 7, 7), (300, 33, 131073, 0, 0), (2048, 3, 4003, 4, 0), (2048, 3, 4009, 1, 3)])
+                                         (65535, 1, 4001, 7, 7), (300, 33, 131073, 0, 0), (2048, 3, 4003, 4, 0), (2048, 3, 4009, 1, 3),
+                                         (2048, 257, 5119, 0, 0), (2048, 257, 5120, 0, 0)])
 def test_lookup_table_inverts_an_ascending_cdf(hip, v, n, m, to, so):
     """The inverse table of nchip_cdf_lookup, with columns that start `to` / `so` elements off a 16-byte
     boundary: runs of one target and of thousands, entries that share a value (the last one's
