@@ -2125,12 +2125,16 @@ static bool gemm_is_small(int m, int n, int k, int batch, int ksplit)
 
 // Whether an fp32 product of class 7, 4 or 10 is issued by gemm_dma_kernel (the same sums; this is about
 // time only): whole stages of 32 k, 16-byte units, 32-bit offsets inside a stage.  The single-chain
-// classes gain everywhere; of the 64x64 class, tiles that the other kernel would guard, more tiles than CUs
-// and operands that need no reads across rows (both K-contiguous reads of a step hit two banks twice),
-// us 64x64 class -> this:
-//   352 x 1066 x 352 16.0 -> 10.3   704 x 1066 x 352 15.9 -> 10.9   512 x 2048 x 512 16.7 -> 14.5
-//   512 x 2048 x 2048 42.5 -> 43.9 (kept out), A transposed 45.9 -> 48.1, x 1024 24.0 -> 26.2 (out), B transposed 43.4 -> 41.5
-//   256 of 64 x 320 x 128, A transposed 36.0 -> 28.6
+// classes gain everywhere; of the 64x64 class, more tiles than CUs and operands that need no reads across
+// rows (both K-contiguous reads of a step hit two banks twice); partial tiles, whose rows this kernel
+// repeats and the other moves to the edge, and short reductions make up for one such operand.  Speed against
+// the 64x64 class, K = 128 / 352 / 512 / 1024 / 2048 / 4096:
+//   512 x 2112 (264 tiles)   1.23 / 1.22 / 1.12 / 1.11 / 1.11 / 1.10   A transposed 1.15 / 1.15 / 1.08 / 1.07 / 1.05 / 1.04
+//   1028 x 1028 (289)        1.35 / 1.27 / 1.22 / 1.18 / 1.14 / 1.11   A transposed 1.23 / 1.19 / 1.11 / 1.08 / 1.06 / 1.04
+//   512 x 2048 (256)         1.08 / 1.08 / 1.01 / 1.01; 43.9 us against 42.5 at 2048 (kept out), B transposed 1.11 / 1.12 / 1.06 / 1.08 / 1.10 / 1.10
+//   1000 x 1000 (256)        1.16 / 1.13 / 1.16 / 1.10 / 1.08 / 1.05   A transposed 1.10 / 1.04 / 0.95 / 0.95 / 0.93 / 0.92
+//   352 x 1068 (102)         K = 352 1.16, A transposed 1.05, B transposed 1.22; 512 1.17, 0.98, 1.23
+//   128 of 100 x 100 (512)   B transposed 1.41 / 1.26 / 1.23 / 1.09 / 0.97 / 0.95, the others 1.07 and up
 // class 4: 2048 x 2048 x 512 48.5 -> 42.0, 1024 x 2048 x 512 24.9 -> 23.7, 256 of 320 x 64 x 128 31.0 -> 24.8
 // class 7: 4096 x 4096 x 1024 300 -> 261, A transposed 291 -> 267, B transposed (4096 x 1024 x 4096) 303 -> 249
 static bool dma_fits_f32(const GemmArgs &g, int ta, int tb)
@@ -2143,7 +2147,8 @@ static bool dma_gains_f32(const GemmArgs &g, int cfg, int ta, int tb)
 {
     if (cfg != 10) return cfg == 7 || cfg == 4;
     const int64_t tiles = (int64_t)((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch * g.ksplit;
-    return g.M % 64 || g.N % 64 || tiles > 256 || tb || (!ta && g.K <= 1024);
+    const bool partial = g.M % 64 || g.N % 64;
+    return tiles > 256 || tb || (ta ? partial && g.K <= 384 : partial || g.K <= 1024);
 }
 
 extern "C" int nchip_gemm_is_small(int m, int n, int k, int batch)
