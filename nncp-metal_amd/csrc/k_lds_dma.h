@@ -29,7 +29,7 @@ __device__ __forceinline__ void lds_dma16(uint16_t NCHIP_LDS *lds, const void *b
     // (the base is copied by the scalar unit: a vector instruction's scalar result may not be read by
     // a memory instruction right behind it; the copy is also the slot that the load needs after m0)
     asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %3, %0"
-                 : "=&s"(from) : "s"(at), "s"((uint64_t)lo | (uint64_t)up << 32), "v"(off) : "memory");
+                 : "=&s"(from) : "s"(at), "s"((uint64_t)lo | (uint64_t)up << 32), "v"(off) : "memory", "m0");
 #else
     memcpy(lds + 8 * (threadIdx.x & 63), (const char *)base + off, 16);
 #endif
