@@ -1919,8 +1919,9 @@ void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int 
 #undef LAUNCH
 }
 
+// (0, or -2 with a message where the stages' LDS is refused)
 template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int NACC = 1>
-void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int grouped_tiles = 0)
+int launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int grouped_tiles = 0)
 {
     g.tiles_m = (g.M + BM - 1) / BM;
     g.tiles_n = (g.N + BN - 1) / BN;
@@ -1933,7 +1934,7 @@ void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int g
         static const bool ok = hipFuncSetAttribute(                                                        \
             reinterpret_cast<const void *>(gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>),                    \
             hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn) == hipSuccess;                           \
-        if (!ok) { fprintf(stderr, "nchip_gemm: cannot reserve %zu bytes of LDS\n", dyn); abort(); }      \
+        if (!ok) { fprintf(stderr, "nchip_gemm: cannot reserve %zu bytes of LDS\n", dyn); return -2; }    \
         if (rec) hipExtLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>), grid, block, dyn, st, rec->start, rec->stop, 0, g); \
         else hipLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>), grid, block, dyn, st, g);   \
     } while (0)
@@ -1942,6 +1943,7 @@ void launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int g
     else if (!ta && tb) LAUNCH(0, 1);
     else LAUNCH(1, 1);
 #undef LAUNCH
+    return 0;
 }
 
 // Tile class of a product of bf16 operands, from the tile counts.  One 256 x 256 tile fills a CU
@@ -1967,19 +1969,18 @@ static int dma_class(int m, int n, bool two_chains)
     return tiles(128, 64) >= 224 && m >= 128 ? 2 : 3;
 }
 
-static void launch_dma_class(hipStream_t st, int cls, bool two_chains, int ta, int tb, GemmArgs &g, ProfRec *rec)
+static int launch_dma_class(hipStream_t st, int cls, bool two_chains, int ta, int tb, GemmArgs &g, ProfRec *rec)
 {
     if (two_chains) {
-        if (cls == 1 || cls == 5) launch_dma<0, 128, 128, 2, 4, 1, 4, 2>(st, ta, tb, g, rec);
-        else if (cls == 2) launch_dma<0, 128, 64, 2, 2, 1, 3, 2>(st, ta, tb, g, rec);
-        else launch_dma<0, 64, 64, 2, 2, 1, 4, 2>(st, ta, tb, g, rec);
-        return;
+        if (cls == 1 || cls == 5) return launch_dma<0, 128, 128, 2, 4, 1, 4, 2>(st, ta, tb, g, rec);
+        if (cls == 2) return launch_dma<0, 128, 64, 2, 2, 1, 3, 2>(st, ta, tb, g, rec);
+        return launch_dma<0, 64, 64, 2, 2, 1, 4, 2>(st, ta, tb, g, rec);
     }
-    if (cls == 4) launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, rec);
-    else if (cls == 1) launch_dma<0, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, rec);
-    else if (cls == 5) launch_dma<0, 128, 128, 2, 4, 1, 4>(st, ta, tb, g, rec);
-    else if (cls == 2) launch_dma<0, 128, 64, 2, 2, 1, 3>(st, ta, tb, g, rec);
-    else launch_dma<0, 64, 64, 2, 2, 1, 4>(st, ta, tb, g, rec);
+    if (cls == 4) return launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, rec);
+    if (cls == 1) return launch_dma<0, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, rec);
+    if (cls == 5) return launch_dma<0, 128, 128, 2, 4, 1, 4>(st, ta, tb, g, rec);
+    if (cls == 2) return launch_dma<0, 128, 64, 2, 2, 1, 3>(st, ta, tb, g, rec);
+    return launch_dma<0, 64, 64, 2, 2, 1, 4>(st, ta, tb, g, rec);
 }
 
 template <int NW, int PF, int SPLIT>
@@ -2270,16 +2271,17 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     }
     if (from_bf16) {
         const bool two_chains = bf16_two_chains(m, n, k);
-        launch_dma_class(st, dma_class(m, n, two_chains), two_chains, ta, tb, g, pr);
+        if (launch_dma_class(st, dma_class(m, n, two_chains), two_chains, ta, tb, g, pr)) return -2;
     } else if (precision == 1) {
         if (cfg == 7) launch_tile<128, 128, 32, 4, 2, 1>(st, ta, tb, g, pr);
         else if (cfg == 4) launch_tile<128, 64, 32, 4, 2, 1>(st, ta, tb, g, pr);
         else if (cfg == 9) launch_tile<64, 64, 64, 2, 2, 1, 2>(st, ta, tb, g, pr);
         else launch_tile<64, 64, 32, 2, 2, 1, 2>(st, ta, tb, g, pr);
     } else if (dma) {
-        if (cfg == 10) launch_dma<1, 64, 64, 2, 2, 2, 4>(st, ta, tb, g, pr);
-        else if (cfg == 7 && !tb) launch_dma<1, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, pr);
-        else launch_dma<1, 128, 64, 4, 2, 1, 3>(st, ta, tb, g, pr);
+        if (cfg == 10 ? launch_dma<1, 64, 64, 2, 2, 2, 4>(st, ta, tb, g, pr)
+            : cfg == 7 && !tb ? launch_dma<1, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, pr)
+                              : launch_dma<1, 128, 64, 4, 2, 1, 3>(st, ta, tb, g, pr))
+            return -2;
     } else if (cfg == 40) {
         // (wavefronts: the two chains, or as many of the 2 ksplit; blocks in flight: one round trip's)
         if (ksplit > 4) launch_small<16, 8, 1>(st, ta, tb, g, pr);
@@ -2573,7 +2575,7 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
         rec.variant = 64 + cls * 4 + ta * 2 + tb; // the bf16-operand classes
     }
     ProfRec *pr = g_prof_on ? &rec : nullptr;
-    launch_dma_class(st, cls, two_chains, ta, tb, g, pr);
+    if (launch_dma_class(st, cls, two_chains, ta, tb, g, pr)) return -2;
     if (g_prof_on) g_prof.push_back(rec);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
@@ -2696,11 +2698,11 @@ extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmP
     } else if (precision == 5) {
         launch_tile<64, 64, 32, 2, 2, 0, 2, 4>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
     } else if (precision == 4) {
-        launch_dma<1, 128, 128, 4, 2, 1, 4>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+        if (launch_dma<1, 128, 128, 4, 2, 1, 4>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles)) return -2;
     } else if (precision == 3) {
-        launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+        if (launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles)) return -2;
     } else if (precision == 2) {
-        launch_dma<0, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles);
+        if (launch_dma<0, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, g_prof_on ? &rec : nullptr, total_tiles)) return -2;
     } else if (precision == 1) {
         if (!ta && !tb) GRP(0, 0, 1); else if (ta && !tb) GRP(1, 0, 1); else if (!ta && tb) GRP(0, 1, 1); else GRP(1, 1, 1);
     } else {

@@ -121,7 +121,8 @@ static inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 static inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 static inline hipError_t hipEventSynchronize(hipEvent_t) { hipcpu_flush_copies(); return hipSuccess; }
 static inline hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 1e-3f; return hipSuccess; }
-static inline hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+// (HIPCPU_REFUSE_LDS: no launch gets more dynamic LDS than the default)
+static inline hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return getenv("HIPCPU_REFUSE_LDS") ? hipErrorInvalidValue : hipSuccess; }
 
 /* ---- launches ---------------------------------------------------------------------- */
 template <typename F, typename Tuple, size_t... I>

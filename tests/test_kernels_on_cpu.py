@@ -112,6 +112,19 @@ def test_host_tensor_compute_is_refused(emulated):
     assert r.returncode != 0 and "GPU only" in r.stderr
 
 
+def test_products_report_lds_that_they_do_not_get(emulated):
+    """Where the runtime refuses the LDS of the staged products, the raw entry points return -2 (nothing
+    launched) and the process goes on."""
+    code = ("import os, ctypes as C; lib = C.CDLL(os.environ['NNCP_TEST_HIP_LIB']);"
+            "lib.nchip_gemm_grouped.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_double];"
+            "print([lib.nchip_gemm_grouped(None, 0, 1, 4096, 1, 1, p, 0.0) for p in (2, 3, 4)]);"
+            "p, i, j, f = C.c_void_p, C.c_int, C.c_int64, C.c_float;"
+            "lib.nchip_gemm.argtypes = [p, i, i, i, i, i, f, p, j, j, p, j, j, f, p, j, j, i, p, i, p, i, i, p];"
+            "print(lib.nchip_gemm(None, 0, 0, 4096, 4096, 64, 1.0, 4096, 4096, 0, 4096, 64, 0, 0.0, 4096, 4096, 0, 1, None, 0, None, 0, 1, None))")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=dict(emulated, HIPCPU_REFUSE_LDS="1"))
+    assert r.returncode == 0 and r.stdout.split("\n")[:2] == ["[-2, -2, -2]", "-2"] and "cannot reserve" in r.stderr, (r.stdout, r.stderr)
+
+
 def test_malformed_parameter_files_end_with_a_message(emulated, tmp_path):
     """The product's own reader of parameter files (csrc/nc_params_io.cpp) against the malformed
     records of tests/test_host_model.py: each ends in nc_fatal's message, none in a fault."""
