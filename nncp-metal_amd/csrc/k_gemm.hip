@@ -2096,7 +2096,7 @@ static bool rounds_in_memory(int m, int n, int k)
 static bool bf16_two_chains(int m, int n, int k)
 {
     if (!rounds_in_memory(m, n, k)) return gemm_class(m, n, 1) == 10;
-    if (g_force_cfg == 11 || g_force_cfg == 13) return g_force_cfg == 11; // tuning aid
+    if (g_force_cfg == 7 || g_force_cfg == 11 || g_force_cfg == 13) return g_force_cfg == 11; // tuning aid
     return (int64_t)((m + 127) / 128) * ((n + 127) / 128) < 512;
 }
 
