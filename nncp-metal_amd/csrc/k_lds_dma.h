@@ -26,10 +26,11 @@ __device__ __forceinline__ void lds_dma16(uint16_t NCHIP_LDS *lds, const void *b
     const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)base);
     const uint32_t up = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uintptr_t)base >> 32));
     uint64_t from;
+    uint32_t m0; // (an output, for the compiler to know: it warns of a clobber, the register being reserved)
     // (the base is copied by the scalar unit: a vector instruction's scalar result may not be read by
     // a memory instruction right behind it; the copy is also the slot that the load needs after m0)
-    asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %3, %0"
-                 : "=&s"(from) : "s"(at), "s"((uint64_t)lo | (uint64_t)up << 32), "v"(off) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %4, %0"
+                 : "=&s"(from), "={m0}"(m0) : "s"(at), "s"((uint64_t)lo | (uint64_t)up << 32), "v"(off) : "memory");
 #else
     memcpy(lds + 8 * (threadIdx.x & 63), (const char *)base + off, 16);
 #endif
