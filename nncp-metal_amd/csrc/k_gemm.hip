@@ -874,7 +874,7 @@ __device__ __forceinline__ void each_constant(F f, std::integer_sequence<int, I.
 // us before -> now, 512 x 2048 x 512 16.7 -> 14.5, 2048 x 2048 x 512 48.5 -> 42.0, the grouped weight
 // gradients of 12 layers of 512 over 2048 tokens 1571 -> 1361 (133 TFLOP/s).
 constexpr int BOX_LD = 36; // words between the columns of an accumulator tile in LDS
-template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int TA, int TB, int NACC = 1>
+template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int TA, int TB, int NACC = 1, int FAR = 0>
 __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0)
 {
     GemmArgs g = g0;
@@ -921,8 +921,9 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
     }
     const int nk = (kend - kbeg) / BK, it2 = k1 / BK;
 
-    // this lane's byte offsets inside a stage's panel of an operand; rows and units past the edge
-    // repeat the last one (their results are not stored)
+    // this lane's byte offsets inside a stage's panel of an operand (64 bits with FAR, for rows that far apart);
+    // rows and units past the edge repeat the last one (their results are not stored)
+    using Off = std::conditional_t<FAR != 0, uint64_t, uint32_t>;
     auto offsets = [&](auto &off, auto kcontig, auto extent, int64_t ld, int i0, int imax) {
         constexpr int BT = decltype(extent)::value, NV = BT * 8 / NT;
 #pragma unroll
@@ -930,16 +931,16 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
             const int p = t + v * NT;
             if constexpr (decltype(kcontig)::value) {
                 const int i = p / 8, row = i0 + i < imax ? i : imax - 1 - i0;
-                off[v] = (uint32_t)(E * (row * ld + ((p ^ i >> 1) & 7) * V));
+                off[v] = (Off)(E * (row * ld + ((p ^ i >> 1) & 7) * V));
             } else {
                 constexpr int U = BT / V, SH = BT >= 128 ? 1 : 0;
                 const int k = p / U, u = p % U;
                 const int i = F32 ? (u ^ (k & 1) << 3) * V : (((u >> 1) ^ ((k & 3) << SH)) * 2 + (u & 1)) * V;
-                off[v] = (uint32_t)(E * (k * ld + (i0 + i + V <= imax ? i : imax - V - i0)));
+                off[v] = (Off)(E * (k * ld + (i0 + i + V <= imax ? i : imax - V - i0)));
             }
         }
     };
-    uint32_t oa[NVA], ob[NVB];
+    Off oa[NVA], ob[NVB];
     // (a long axis that is no multiple of V lies in a copy whose columns are padded to one)
     offsets(oa, std::integral_constant<bool, TA != 0>(), std::integral_constant<int, BM>(), g.lda, m0, TA ? g.M : (g.M + V - 1) & ~(V - 1));
     offsets(ob, std::integral_constant<bool, TB == 0>(), std::integral_constant<int, BN>(), g.ldb, n0, TB ? (g.N + V - 1) & ~(V - 1) : g.N);
@@ -1920,7 +1921,7 @@ void launch_tile(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int 
 }
 
 // (0, or -2 with a message where the stages' LDS is refused)
-template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int NACC = 1>
+template <int F32, int BM, int BN, int WM, int WN, int KW, int ST, int NACC = 1, int FAR = 0>
 int launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int grouped_tiles = 0)
 {
     g.tiles_m = (g.M + BM - 1) / BM;
@@ -1932,11 +1933,11 @@ int launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int gr
 #define LAUNCH(TA, TB)                                                                                     \
     do {                                                                                                   \
         static const bool ok = hipFuncSetAttribute(                                                        \
-            reinterpret_cast<const void *>(gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>),                    \
+            reinterpret_cast<const void *>(gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC, FAR>),                    \
             hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn) == hipSuccess;                           \
         if (!ok) { fprintf(stderr, "nchip_gemm: cannot reserve %zu bytes of LDS\n", dyn); return -2; }    \
-        if (rec) hipExtLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>), grid, block, dyn, st, rec->start, rec->stop, 0, g); \
-        else hipLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC>), grid, block, dyn, st, g);   \
+        if (rec) hipExtLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC, FAR>), grid, block, dyn, st, rec->start, rec->stop, 0, g); \
+        else hipLaunchKernelGGL((gemm_dma_kernel<F32, BM, BN, WM, WN, KW, ST, TA, TB, NACC, FAR>), grid, block, dyn, st, g);   \
     } while (0)
     if (!ta && !tb) LAUNCH(0, 0);
     else if (ta && !tb) LAUNCH(1, 0);
@@ -1945,6 +1946,9 @@ int launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int gr
 #undef LAUNCH
     return 0;
 }
+
+// The widest leading dimension of bf16 operands whose 256 rows or 64 k of a stage are within 32 bits.
+constexpr int64_t DMA_LD = 1 << 23;
 
 // Tile class of a product of bf16 operands, from the tile counts.  One 256 x 256 tile fills a CU
 // (128 KB of stages, 256 registers): it is taken when its rounds of 256 workgroups are at least
@@ -1958,9 +1962,11 @@ int launch_dma(hipStream_t st, int ta, int tb, GemmArgs &g, ProfRec *rec, int gr
 //   1024 x 4096 x 4096     96 /  59 /  43 /  53 /  64   before  52
 //   1024 x 2048 x 3072     71 /  39 /  30 /  24 /  28   before  33
 //   512 x 2048 x 2048      47 /  21 /  19 /  13 /  10   before  13
-// (two chains: no room for the second accumulators in 256 x 256 tiles, nor twice a CU in classes of 64 x 64 a wavefront)
-static int dma_class(int m, int n, bool two_chains)
+// (class 6: rows too far apart for 32-bit offsets; two chains: no room for the second accumulators in 256 x 256 tiles, nor twice a CU in classes of 64 x 64 a wavefront)
+static int dma_class(const GemmArgs &g, bool two_chains)
 {
+    const int m = g.M, n = g.N;
+    if (g.lda > DMA_LD || g.ldb > DMA_LD) return 6;
     auto tiles = [&](int bm, int bn) { return (int64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn); };
     const int64_t t256 = tiles(256, 256), t128 = tiles(128, 128);
     if (!two_chains && 8 * t256 >= 7 * 256 * ((t256 + 255) / 256)) return 4;
@@ -1972,10 +1978,12 @@ static int dma_class(int m, int n, bool two_chains)
 static int launch_dma_class(hipStream_t st, int cls, bool two_chains, int ta, int tb, GemmArgs &g, ProfRec *rec)
 {
     if (two_chains) {
+        if (cls == 6) return launch_dma<0, 64, 64, 2, 2, 1, 4, 2, 1>(st, ta, tb, g, rec);
         if (cls == 1 || cls == 5) return launch_dma<0, 128, 128, 2, 4, 1, 4, 2>(st, ta, tb, g, rec);
         if (cls == 2) return launch_dma<0, 128, 64, 2, 2, 1, 3, 2>(st, ta, tb, g, rec);
         return launch_dma<0, 64, 64, 2, 2, 1, 4, 2>(st, ta, tb, g, rec);
     }
+    if (cls == 6) return launch_dma<0, 64, 64, 2, 2, 1, 4, 1, 1>(st, ta, tb, g, rec);
     if (cls == 4) return launch_dma<0, 256, 256, 2, 4, 1, 2>(st, ta, tb, g, rec);
     if (cls == 1) return launch_dma<0, 128, 128, 2, 2, 1, 2>(st, ta, tb, g, rec);
     if (cls == 5) return launch_dma<0, 128, 128, 2, 4, 1, 4>(st, ta, tb, g, rec);
@@ -2245,8 +2253,7 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     // the ones the conversion inside the tile loader would produce, so the
     // result is the same either way.
     bool from_bf16 = false;
-    if (precision == 1 && batch == 1 && ksplit == 1 && !invariant && m < 1 << 21 && n < 1 << 21 && k < 1 << 21 && // (32-bit offsets)
-        rounds_in_memory(m, n, k)) {
+    if (precision == 1 && batch == 1 && ksplit == 1 && !invariant && rounds_in_memory(m, n, k)) {
         const int kpad = (k + 63) / 64 * 64;
         const size_t ea = cast_elems(ta ? k : m, ta ? m : k, ta != 0, kpad);
         const size_t eb = cast_elems(tb ? n : k, tb ? k : n, tb == 0, kpad);
@@ -2271,7 +2278,9 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     }
     if (from_bf16) {
         const bool two_chains = bf16_two_chains(m, n, k);
-        if (launch_dma_class(st, dma_class(m, n, two_chains), two_chains, ta, tb, g, pr)) return -2;
+        const int cls = dma_class(g, two_chains);
+        rec.variant = (two_chains ? 92 : 64) + cls * 4 + (ta ? 2 : 0) + (tb ? 1 : 0);
+        if (launch_dma_class(st, cls, two_chains, ta, tb, g, pr)) return -2;
     } else if (precision == 1) {
         if (cfg == 7) launch_tile<128, 128, 32, 4, 2, 1>(st, ta, tb, g, pr);
         else if (cfg == 4) launch_tile<128, 64, 32, 4, 2, 1>(st, ta, tb, g, pr);
@@ -2317,8 +2326,8 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
     }
     if (g_prof_on) {
         int tile = cfg == 40 ? 6 : cfg == 7 ? 2 : (cfg == 4 ? 1 : ((cfg == 8 || cfg == 10 || cfg == 30) ? 3 : 0));
-        rec.variant = tile * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 1 ? 1 : 0);
-        if (dma) rec.variant = 88 + (cfg == 10 ? 12 : (cfg == 7 && !tb ? 4 : 8)) + (ta ? 2 : 0) + (tb ? 1 : 0);
+        if (!from_bf16) rec.variant = tile * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 1 ? 1 : 0);
+        if (dma) rec.variant = 120 + (cfg == 10 ? 12 : (cfg == 7 && !tb ? 4 : 8)) + (ta ? 2 : 0) + (tb ? 1 : 0);
         g_prof.push_back(rec);
     }
     if (ksplit > 1 && cfg != 40) {
@@ -2545,7 +2554,7 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
         fprintf(stderr, "nchip_gemm_bf16_operands: bad arguments (m=%d n=%d k=%d)\n", m, n, k);
         return -1;
     }
-    if (k % 64 || a->lda % 8 || a->ldb % 8 || a->lda >= 1 << 22 || a->ldb >= 1 << 22 || (!ta && m % 64) || (tb && n % 64) || (((uintptr_t)a->A16 | (uintptr_t)a->B16) & 15) != 0)
+    if (k % 64 || a->lda % 8 || a->ldb % 8 || (!ta && m % 64) || (tb && n % 64) || (((uintptr_t)a->A16 | (uintptr_t)a->B16) & 15) != 0)
         return 1;
     GemmArgs g;
     memset(&g, 0, sizeof(g));
@@ -2561,7 +2570,8 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
     const int64_t t128 = (int64_t)((m + 127) / 128) * ((n + 127) / 128), t128x64 = (int64_t)((m + 127) / 128) * ((n + 63) / 64);
     const int bm = t128 >= 224 || (t128x64 >= 224 && m >= 128) ? 128 : 64, bn = t128 >= 224 ? 128 : 64;
     const bool whole = (ta || m % bm == 0) && (!tb || n % bn == 0), two_chains = !whole && bf16_two_chains(m, n, k);
-    const int cls = g_bf16ops_cls >= 1 && g_bf16ops_cls <= 5 && !(two_chains && g_bf16ops_cls == 4) ? g_bf16ops_cls : dma_class(m, n, two_chains);
+    int cls = dma_class(g, two_chains);
+    if (cls != 6 && g_bf16ops_cls >= 1 && g_bf16ops_cls <= 5 && !(two_chains && g_bf16ops_cls == 4)) cls = g_bf16ops_cls;
     if (a->rowsum && a->rows_written && a->dpre) {
         const int bn = cls == 4 ? 256 : (cls == 1 || cls == 5 ? 128 : 64);
         g.rowsum = a->rowsum;
@@ -2572,7 +2582,7 @@ extern "C" int nchip_gemm_bf16_operands(void *stream, const NchipGemmBf16Args *a
         (void)hipEventCreate(&rec.start);
         (void)hipEventCreate(&rec.stop);
         rec.flops = 2.0 * m * n * (double)k;
-        rec.variant = 64 + cls * 4 + ta * 2 + tb; // the bf16-operand classes
+        rec.variant = (two_chains ? 92 : 64) + cls * 4 + ta * 2 + tb;
     }
     ProfRec *pr = g_prof_on ? &rec : nullptr;
     if (launch_dma_class(st, cls, two_chains, ta, tb, g, pr)) return -2;
@@ -2598,7 +2608,7 @@ extern "C" void nchip_gemm_profile_enable(int on)
 extern "C" int nchip_gemm_profile_read(int max_variants, char (*names)[48], int64_t *launches,
                                        double *flops, double *seconds)
 {
-    constexpr int NVAR = 104;
+    constexpr int NVAR = 136;
     double fl[NVAR] = { 0 }, sec[NVAR] = { 0 };
     int64_t cnt[NVAR] = { 0 };
     for (ProfRec &r : g_prof) {
@@ -2616,13 +2626,15 @@ extern "C" int nchip_gemm_profile_read(int max_variants, char (*names)[48], int6
     g_prof.clear();
     static const char *tiles_f32[4] = { "64,64,16,2,2", "128,64,32,4,2", "128,128,32,4,2", "64,64,32,2,2" };
     static const char *tiles_bf16[4] = { "64,64,32,2,2", "128,64,32,4,2", "128,128,32,4,2", "64,64,32,2,2" };
-    static const char *tiles_ops[6] = { "256,256,2,4,1,2", "128,128,2,2,1,2", "128,64,2,2,1,3", "64,64,2,2,1,4", "256,256,2,4,1,2", "128,128,2,4,1,4" }; // 0: grouped
+    static const char *tiles_ops[7] = { "256,256,2,4,1,2", "128,128,2,2,1,2", "128,64,2,2,1,3", "64,64,2,2,1,4", "256,256,2,4,1,2", "128,128,2,4,1,4", "64,64,2,2,1,4" }; // 0: grouped; 6: 64-bit offsets
     static const char *tiles_f32_dma[4] = { "128,128,4,2,1,4", "128,128,2,2,1,2", "128,64,4,2,1,3", "64,64,2,2,2,4" }; // 0: grouped
     int n = 0;
     for (int v = 0; v < NVAR && n < max_variants; v++) {
         if (!cnt[v]) continue;
-        if (v >= 88) { // fp32 operands staged by DMA
-            snprintf(names[n], 48, "gemm_dma_kernel<1,%s,%d,%d%s>", tiles_f32_dma[(v - 88) / 4], (v >> 1) & 1, v & 1, v < 92 ? ",grouped" : "");
+        if (v >= 120) { // fp32 operands staged by DMA
+            snprintf(names[n], 48, "gemm_dma_kernel<1,%s,%d,%d%s>", tiles_f32_dma[(v - 120) / 4], (v >> 1) & 1, v & 1, v < 124 ? ",grouped" : "");
+        } else if (v >= 92) { // bf16, two chains
+            snprintf(names[n], 48, "gemm_dma_kernel<0,%s,%d,%d,2>", tiles_ops[(v - 92) / 4], (v >> 1) & 1, v & 1);
         } else if (v >= 64) { // operands read as bf16: gemm_dma_kernel<tile, wavefronts, stages, ta, tb>
             snprintf(names[n], 48, "gemm_dma_kernel<0,%s,%d,%d%s>", tiles_ops[(v - 64) / 4], (v >> 1) & 1, v & 1,
                      v < 68 ? ",grouped" : "");
@@ -2677,7 +2689,7 @@ extern "C" int nchip_gemm_grouped(void *stream, int ta, int tb, const NchipGemmP
         (void)hipEventCreate(&rec.start);
         (void)hipEventCreate(&rec.stop);
         rec.variant = precision >= 5 ? 3 * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 6 ? 1 : 0)
-                    : precision >= 2 ? (precision == 4 ? 88 : precision == 3 ? 64 : 32) + (ta ? 2 : 0) + (tb ? 1 : 0)
+                    : precision >= 2 ? (precision == 4 ? 120 : precision == 3 ? 64 : 32) + (ta ? 2 : 0) + (tb ? 1 : 0)
                                      : 2 * 8 + (ta ? 4 : 0) + (tb ? 2 : 0) + (precision == 1 ? 1 : 0);
         rec.flops = total_flops;
     }

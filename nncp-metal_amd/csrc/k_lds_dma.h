@@ -36,6 +36,20 @@ __device__ __forceinline__ void lds_dma16(uint16_t NCHIP_LDS *lds, const void *b
 #endif
 }
 
+// The same from 64-bit offsets, for rows more than 4 GiB apart.
+__device__ __forceinline__ void lds_dma16(uint16_t NCHIP_LDS *lds, const void *base, uint64_t off)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)lds);
+    uint32_t m0;
+    // (the wait is the slot that the load needs after m0)
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off"
+                 : "={m0}"(m0) : "s"(at), "v"((uint64_t)(uintptr_t)base + off) : "memory");
+#else
+    memcpy(lds + 8 * (threadIdx.x & 63), (const char *)base + off, 16);
+#endif
+}
+
 // Waits until at most LEFT of this wavefront's vector-memory instructions are in flight (they
 // complete in order) and its LDS reads are done, then for the other wavefronts of the workgroup.
 template <int LEFT>

@@ -420,3 +420,30 @@ def test_bf16_operands_that_do_not_fill_their_tiles_have_the_sums_of_the_general
     assert lib.nchip_gemm_bf16_operands(st, C.byref(g)) == 0
     assert np.array_equal(hip.numpy(c_t), hip.numpy(d_t))
     hip.free(a_t, b_t, c_t, d_t, a16, b16)
+
+
+@pytest.mark.parametrize("far,m,n,k,ld", [("a", 3, 70, 128, (1 << 30) + 8), ("b", 66, 64, 64, (1 << 25) + (1 << 21))])
+def test_bf16_operands_with_rows_gigabytes_apart(hip, raw, rng, far, m, n, k, ld):
+    """Rows whose offsets inside a stage pass 32 bits (k contiguous, and n contiguous): the bits of the compact
+    operands.  One operand lies in a buffer of 4.3 GB, of which only its rows are written."""
+    lib, st, ptr = raw
+    tb = far == "b"
+    rows = {"a": rng.standard_normal((m, k)).astype(np.float32), "b": rng.standard_normal((k, n) if tb else (n, k)).astype(np.float32)}
+    one = {"a": k, "b": n if tb else k}
+    n_big = (len(rows[far]) - 1) * ld + one[far]
+    big = hip.lib.nc_new_tensor_nz(hip.dev, 0, 1, (C.c_size_t * 1)((n_big + 1) // 2))  # (f32: two values each)
+    d = {x: hip.tensor(r) for x, r in rows.items()}
+    d16 = {x: hip.tensor(np.zeros(r.shape, np.uint16)) for x, r in rows.items()}
+    for x, r in rows.items():
+        assert lib.nchip_cast_bf16(st, ptr(d[x]), ptr(d16[x]), r.size) == 0
+    for i in range(len(rows[far])):
+        assert lib.nchip_cast_bf16(st, C.c_void_p(ptr(d[far]).value + 4 * i * one[far]), C.c_void_p(ptr(big).value + 2 * i * ld), one[far]) == 0
+    got = []
+    for a16, lda, b16, ldb in ((d16["a"], one["a"], d16["b"], one["b"]), (big if far == "a" else d16["a"], ld if far == "a" else one["a"],
+                                                                          big if far == "b" else d16["b"], ld if far == "b" else one["b"])):
+        c_t = hip.tensor(np.full((n, m), 7.0, np.float32))
+        g = Args(ta=1, tb=int(tb), m=m, n=n, k=k, alpha=1.0, A16=ptr(a16), B16=ptr(b16), lda=lda, ldb=ldb, C=ptr(c_t), ldc=m)
+        assert lib.nchip_gemm_bf16_operands(st, C.byref(g)) == 0
+        got.append(hip.numpy(c_t, free=True))
+    hip.free(big, *d.values(), *d16.values())
+    assert np.array_equal(*got)
