@@ -82,17 +82,18 @@ int nchip_gemm2(void *stream, int ta, int tb, int m, int n, int k, float alpha,
                 int ksplit, float *workspace);
 
 /* Many independent GEMMs C_p = alpha_p * op(A_p) * op(B_p) in ONE launch (same
-   transposition flags, 128x128 tiles, no bias/activation, beta = 0).  The
+   transposition flags, no bias/activation, beta = 0 but for precisions 5 and 6).  The
    weight-gradient GEMMs dW = dY X^T of a whole backward pass are issued this
    way: each is too small to fill 256 CUs on its own.  dev_table lives in
    device memory; tile_start is the running sum of
-   nchip_gemm_grouped_tiles(m, n) over the preceding problems.  total_flops
+   nchip_gemm_grouped_tiles(m, n) over the preceding problems (128x128 tiles; other
+   precisions count others, see below).  total_flops
    (sum of 2*m*n*k) is only recorded by the optional launch timing. */
 typedef struct {
     const float *A, *B;
     float *C;
     const float *A2, *B2; /* optional second k range: C = alpha*(op(A)op(B) + op(A2)op(B2)) */
-    int m, n, k, k2;      /* k2 = 0 without A2/B2; with them k must be a multiple of 64 */
+    int m, n, k, k2;      /* k2 = 0 without A2/B2; what k and k2 may be depends on the precision */
     int lda, ldb, ldc;    /* A2 / B2 use lda / ldb too */
     int tile_start;
     float alpha;
@@ -103,7 +104,7 @@ int nchip_gemm_grouped_tiles64(int m, int n);  /* and for precisions 5 and 6 */
 /* whether nchip_gemm (precision 0 or 1, ksplit 1, no forced class) sums an element of this product in two
    chains over k, k % 32 below 16 and from 16 on, rather than in one */
 int nchip_gemm_two_chains(int m, int n, int k, int precision);
-/* precision 0: fp32; 1: fp32 operands rounded to bf16 in the tile loader; 2: the operand
+/* precision 0: fp32; 1: fp32 operands rounded to bf16 in the tile loader (any k and k2 both); 2: the operand
    pointers of the table address bf16 copies (2 bytes per element, same layout and leading
    dimensions as the fp32 matrices they were rounded from), read with unguarded 16-byte
    loads - every k and k2 a multiple of 64, every row-contiguous operand extent (m with
@@ -168,13 +169,10 @@ void nchip_gemm_force_config(int cfg);
 
 /* nchip_gemm_dact that also leaves partial row sums of C (the bias gradient of the layer whose
    pre-activation gradient C is): `rowsum` holds nchip_gemm_rowsum_rows(n) rows of m floats;
-   *rows_written of them are written.  Row p is the sum over 16 columns of C, the 16 that one lane
-   of the epilogue holds: of the 32-column block p / 2, the columns c with c mod 8 in
-   [4 (p mod 2), 4 (p mod 2) + 4) - four runs of 4 consecutive columns, 8 apart - added in
-   increasing column order (columns past n count as zero).  Rows 2j and 2j + 1 together cover
-   block j, so the sum of all rows in row order is the row sum of C.  *rows_written is 0
-   when the kernel chosen for this product does not write them (split-K, bf16 operand copies):
-   the caller then sums C itself. */
+   *rows_written of them are written.  Each is the sum over 8 or 16 columns of C, in an order of the
+   kernel's (columns past n count as zero); together they cover every column once, so the sum of
+   all rows is the row sum of C.  *rows_written is 0 when the kernel chosen for this product does not
+   write them (split-K, operands rounded to copies by the call): the caller then sums C itself. */
 int nchip_gemm_rowsum_rows(int n);
 int nchip_gemm_dact_rowsum(void *stream, int ta, int tb, int m, int n, int k, float alpha,
                            const float *A, int64_t lda, const float *B, int64_t ldb,

@@ -63,7 +63,7 @@ struct GemmArgs {
     int dact;
     float *pre;
     float *ws;
-    uint16_t *c16; // the result once more, rounded to bf16, laid out like C (may be NULL)
+    uint16_t *c16; // the result once more, rounded to bf16, laid out like C (may be NULL; gemm_dma_kernel only)
     int64_t lda, ldb, ldc, sa, sb, sc;   // outer batch strides
     int64_t sa_in, sb_in, sc_in;         // inner batch strides
     int batch_in;                        // batch index z -> (z / batch_in, z % batch_in)
@@ -280,17 +280,15 @@ struct TileLoaderBf16 {
 // holds the lane's (lane/32)*4).  The 16 values go to 16 columns of C.  Everything read here
 // (addend, beta*C) is fetched for all 16 first, so the loads are in flight together, and the
 // uniform option tests sit outside the element loops: a branch per element with a load
-// behind it costs one memory round trip each.  Every product kernel ends in this function,
-// so kernels that feed it the same accumulators write the same bits.
+// behind it costs one memory round trip each.  Kernels that end here, and gemm_dma_kernel with the
+// same steps in its own layout, write the same bits for the same accumulators.
 __device__ __forceinline__ void epilogue_tile(const GemmArgs &g, const floatx16 &acc, int m, int nb,
                                               float NCHIP_GLOBAL *C, float NCHIP_GLOBAL *P,
                                               const float NCHIP_GLOBAL *Radd, const float NCHIP_GLOBAL *Dp,
-                                              bool full, bool plain, float NCHIP_GLOBAL *rowsum = nullptr,
-                                              uint16_t NCHIP_GLOBAL *H = nullptr)
+                                              bool full, bool plain, float NCHIP_GLOBAL *rowsum = nullptr)
 {
     if (!full && m >= g.M) return;
     float NCHIP_GLOBAL *Cp = C + (int64_t)nb * g.ldc + m; // element r lives at Cp + nofs(r)*ldc
-    uint16_t NCHIP_GLOBAL *Hp = H ? H + (int64_t)nb * g.ldc + m : nullptr; // bf16 copy of the same elements
     auto nofs = [](int r) { return (r >> 2) * 8 + (r & 3); };
     if (plain && full) {
 #pragma unroll
@@ -348,11 +346,6 @@ __device__ __forceinline__ void epilogue_tile(const GemmArgs &g, const floatx16 
 #pragma unroll
         for (int r = 0; r < 16; r++)
             if (ok[r]) Cp[(int64_t)nofs(r) * g.ldc] = v[r];
-        if (Hp) {
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-                if (ok[r]) Hp[(int64_t)nofs(r) * g.ldc] = f32_to_bf16_rne(v[r]);
-        }
         if (rowsum) { // this lane's 16 columns of row m, in column order: one entry of a partial row
             float sum = 0.0f;
 #pragma unroll
@@ -366,11 +359,6 @@ __device__ __forceinline__ void epilogue_tile(const GemmArgs &g, const floatx16 
 #pragma unroll
     for (int r = 0; r < 16; r++)
         if (ok[r]) Cp[(int64_t)nofs(r) * g.ldc] = v[r];
-    if (Hp) {
-#pragma unroll
-        for (int r = 0; r < 16; r++)
-            if (ok[r]) Hp[(int64_t)nofs(r) * g.ldc] = f32_to_bf16_rne(v[r]);
-    }
 }
 
 // Product with a few token columns for the width-invariant class: C (M x N, 32 columns per
@@ -886,7 +874,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
     static_assert(KW == 1 || (F32 && KW == 2 && TM * TN == 1), "k groups: fp32, one accumulator tile a wavefront");
     static_assert(NACC == 1 || (!F32 && NACC == 2), "two accumulator sets: bf16");
     static_assert(NVA * NT == BM * 8 && NVB * NT == BN * 8, "whole loads");
-    static_assert(ST >= 2 && (ST - 1) * NL <= 63, "the memory counter has six bits");
+    static_assert(ST >= 2 && ST <= 4 && (ST - 1) * NL <= 63, "arrive()'s counts; the memory counter has six bits");
     static_assert(NG * KW * 32 * BOX_LD * 4 <= ST * STAGE * 2, "the epilogue's corners fit where the stages were");
     extern __shared__ __attribute__((aligned(16))) uint16_t stages_lds[];
     uint16_t NCHIP_LDS *const stages = (uint16_t NCHIP_LDS *)stages_lds;
@@ -1047,8 +1035,6 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_dma_kernel(GemmArgs g0
     auto arrive = [&](int younger) {
         if (ST > 2 && younger >= ST - 2) { lds_dma_barrier<(ST - 2) * NL>(); return; }
         if (ST > 3 && younger == 1) { lds_dma_barrier<NL>(); return; }
-        if (ST > 4 && younger == 2) { lds_dma_barrier<2 * NL>(); return; }
-        if (ST > 5 && younger == 3) { lds_dma_barrier<3 * NL>(); return; }
         lds_dma_barrier<0>(); // (from here on: everything)
     };
 
@@ -1312,8 +1298,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
     // results that are not stored).  With the long axis contiguous such a load runs past the edge by up
     // to 3 values, into the next k: the stage with the range's last k is then left to the guarded loads.
     // Guarding every value of partial or unaligned tiles made a stage a serial chain of memory round trips
-    // (3.8 us); us: 777 x 352 over 481 and 585 k, five layers' gradients in one launch instead of ten
-    // 573 -> 126, 777 x 481 x 352 in the 64x64 class 19.8 -> 16.1.
+    // (3.8 us); 777 x 481 x 352 in the 64x64 class 19.8 -> 16.1 us.
     const bool two = g.grp && A2; // uniform
     const int end1 = two ? k1 : kend, end2 = kend - k1; // where the ranges end (the second counts from 0)
     const int nk1 = (end1 - kbeg + BK - 1) / BK, nk = nk1 + (two ? (end2 + BK - 1) / BK : 0);
@@ -1597,8 +1582,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
     const float NCHIP_GLOBAL *Radd = g.add ? as_global(g.add + coff) : nullptr;
     const bool full = (m0 + BM <= g.M) && (n0 + BN <= g.N); // uniform
     const float NCHIP_GLOBAL *Dp = g.dpre ? as_global(g.dpre + coff) : nullptr;
-    uint16_t NCHIP_GLOBAL *H16 = g.c16 ? as_global(g.c16 + coff) : nullptr;
-    const bool plain = !g.bias && !P && !Radd && !Dp && !H16 && g.beta == 0.0f && g.act == NCHIP_ACT_NONE;
+    const bool plain = !g.bias && !P && !Radd && !Dp && g.beta == 0.0f && g.act == NCHIP_ACT_NONE;
 #pragma unroll
     for (int i = 0; i < TN; i++)
 #pragma unroll
@@ -1606,7 +1590,7 @@ __global__ __launch_bounds__(64 * WM * WN * KW) void gemm_kernel(GemmArgs g0)
             float NCHIP_GLOBAL *rs = nullptr;
             if (g.rowsum) // partial row of this (tile column, wavefront column, accumulator column, lane half)
                 rs = as_global(g.rowsum) + (int64_t)((((tile_n * WN + wn) * TN + i) * 2) + (lane >> 5)) * g.M;
-            epilogue_tile(g, acc[i][j], mm_base + j * 32, nn_base + i * 32, C, P, Radd, Dp, full, plain, rs, H16);
+            epilogue_tile(g, acc[i][j], mm_base + j * 32, nn_base + i * 32, C, P, Radd, Dp, full, plain, rs);
         }
 #ifdef NCHIP_GEMM_CLOCKS
     if (g_gemm_clk && blockIdx.y == 0 && t == 0) g_gemm_clk[6 + 3 * blockIdx.x] = wall_clock64(); // stores issued
@@ -2037,8 +2021,6 @@ uint16_t *cast_scratch(hipStream_t st, size_t elems)
     return c.ptr;
 }
 
-constexpr int CAST_SLACK = 512; // elements past a copy that a partial edge tile may read
-
 // copy of a column-major rows x cols operand; k_is_rows says which extent is k
 // (padded to kpad); returns the leading dimension of the copy
 int64_t cast_operand(hipStream_t st, const float *src, int rows, int cols, int64_t ld, bool k_is_rows,
@@ -2057,7 +2039,7 @@ size_t cast_elems(int rows, int cols, bool k_is_rows, int kpad)
 {
     const size_t rows_pad = k_is_rows ? kpad : (rows + 7) / 8 * 8;
     const size_t cols_pad = k_is_rows ? cols : kpad;
-    return (rows_pad * cols_pad + CAST_SLACK + 127) / 128 * 128;
+    return (rows_pad * cols_pad + 127) / 128 * 128;
 }
 
 } // namespace
@@ -2268,8 +2250,8 @@ static int gemm2_impl(void *stream, int ta, int tb, int m, int n, int k, float a
         }
     }
     const bool dma = precision == 0 && !g_force_cfg && dma_fits_f32(g, ta, tb) && dma_gains_f32(g, cfg, ta, tb);
-    // partial row sums of the result (activation-gradient epilogue): one row per 16 columns of
-    // the padded column range; only the plain tile classes write them
+    // partial row sums of the result (activation-gradient epilogue): one row per 16 columns of the
+    // padded column range, 8 in two k groups staged by DMA; only the plain tile classes write them
     if (rowsum && rowsum_rows && dpre && ksplit == 1 && batch == 1 && !from_bf16 &&
         (cfg == 7 || cfg == 4 || cfg == 10 || cfg == 30)) {
         const int bn = cfg == 7 && !(dma && tb) ? 128 : 64;
@@ -2379,8 +2361,8 @@ extern "C" int nchip_gemm_dact(void *stream, int ta, int tb, int m, int n, int k
 }
 
 // nchip_gemm_dact that also leaves partial row sums of C: rowsum holds nchip_gemm_rowsum_rows(n)
-// rows of m floats, of which *rows_written are written (row p = the sum over 16 columns of C;
-// 0 when this product's kernel does not write them: the caller then sums C itself)
+// rows of m floats, of which *rows_written are written, each over 8 or 16 columns of C (0 when this
+// product's kernel does not write them: the caller then sums C itself)
 extern "C" int nchip_gemm_rowsum_rows(int n) { return (n + 255) / 256 * 32; } // (the widest tile's, two k groups)
 
 extern "C" int nchip_gemm_dact_rowsum(void *stream, int ta, int tb, int m, int n, int k, float alpha,
