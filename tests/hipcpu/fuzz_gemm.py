@@ -35,12 +35,15 @@ for case in range(n_cases):
     ta, tb = int(rng.integers(2)), int(rng.integers(2))
     m, n, k = (int(rng.choice([1, 3, 8, 31, 64, 65, 100, 128, 129, 200, 257, 300, 513])) for _ in range(3))
     k = int(rng.choice([0, 1, 5, 16, 31, 32, 33, 64, 70, 96, 130, 257, 400]))
-    lib.nchip_gemm_force_config(int(rng.choice([0, 0, 0, 4, 7, 8, 9, 5, 1, 2, 3, 6, 10, 11, 13])))
+    forced = int(rng.choice([0, 0, 0, 0, 0, 4, 7, 8, 9, 5, 1, 2, 3, 6, 10, 11, 13]))
+    lib.nchip_gemm_force_config(forced)
     batch = int(rng.choice([1, 1, 1, 2, 3]))
+    if forced == 0 and rng.integers(4) == 0:  # enough tiles for the products staged by DMA, whole units of theirs
+        m, n, k, batch = 4 * int(rng.integers(25, 45)), 4 * int(rng.integers(10, 40)), 32 * int(rng.integers(1, 6)), int(rng.integers(50, 70))
     prec = int(rng.choice([0, 0, 1]))
     mode = int(rng.choice([0, 1, 2]))
     inv = int(rng.integers(4) == 0)
-    ksplit = int(rng.choice([1, 1, 1, 2, 3])) if (not inv and k >= 32) else 1
+    ksplit = int(rng.choice([1, 1, 1, 2, 3, 5, 12])) if (not inv and k >= 32) else 1
     pad_a, pad_b, pad_c = (int(rng.choice([0, 0, 1, 4])) for _ in range(3))
     ra, ca = (k, m) if ta else (m, k)       # stored rows (contiguous), cols
     rb, cb = (n, k) if tb else (k, n)

@@ -447,3 +447,54 @@ def test_bf16_operands_with_rows_gigabytes_apart(hip, raw, rng, far, m, n, k, ld
         got.append(hip.numpy(c_t, free=True))
     hip.free(big, *d.values(), *d16.values())
     assert np.array_equal(*got)
+
+
+def _grouped_products(hip, raw, problems, precision, tiles_of, ta, tb, start=0.0):
+    """C of each (a, b, a2, b2) - stored (columns, rows), a2 / b2 or None - through one grouped launch."""
+    lib, st, ptr = raw
+    keep, outs, table, tiles = [], [], b"", 0
+    for a, b, a2, b2 in problems:
+        (k, m), (n, kb) = (a.shape if not ta else a.shape[::-1]), (b.shape if not tb else b.shape[::-1])
+        assert k == kb
+        d = [None if x is None else hip.tensor(x) for x in (a, b, a2, b2)]
+        out = hip.tensor(np.full((n, m), start, np.float32))
+        k2 = 0 if a2 is None else a2.shape[1 if ta else 0]
+        table += bytes(Problem(A=ptr(d[0]), B=ptr(d[1]), C=ptr(out), A2=ptr(d[2]) if k2 else None, B2=ptr(d[3]) if k2 else None,
+                               m=m, n=n, k=k, k2=k2, lda=k if ta else m, ldb=n if tb else k, ldc=m, tile_start=tiles, alpha=0.5))
+        tiles += tiles_of(m, n)
+        keep += [x for x in d if x]
+        outs.append(out)
+    t = hip.tensor(np.frombuffer(table, dtype=np.uint8))
+    assert lib.nchip_gemm_grouped(st, ta, tb, ptr(t), len(problems), tiles, precision, 1.0) == 0
+    got = [hip.numpy(x, free=True) for x in outs]
+    hip.free(t, *keep)
+    return got
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 0), (0, 1), (1, 1)])
+def test_grouped_fp32_launch_by_whole_units(hip, raw, rng, ta, tb):
+    """nchip_gemm_grouped with precision 4: partial tiles, ranges of one stage and of several, a second range (with k
+    contiguous in neither operand: the two share their leading dimensions), no k at all: the bits of precision 0."""
+    def operands(m, n, k):
+        return (rng.standard_normal((m, k) if ta else (k, m)).astype(np.float32), rng.standard_normal((k, n) if tb else (n, k)).astype(np.float32))
+    problems = []
+    for m, n, k, k2 in [(4, 132, 32, 32), (260, 64, 160, 32), (128, 128, 96, 288), (68, 4, 256, 0), (32, 36, 0, 0)]:
+        second = operands(m, n, k2) if k2 and not ta and tb else (None, None)
+        problems.append(operands(m, n, k) + second if k else (np.zeros((m, 0) if ta else (0, m), np.float32), np.zeros((0, n) if tb else (n, 0), np.float32), None, None))
+    lib = raw[0]
+    zero, four = (_grouped_products(hip, raw, problems, p, lib.nchip_gemm_grouped_tiles, ta, tb, 5.0) for p in (0, 4))
+    assert all(np.array_equal(x, y) for x, y in zip(zero, four)) and not four[-1].any()
+
+
+@pytest.mark.parametrize("precision", [0, 1, 5, 6])
+def test_grouped_launch_of_any_k(hip, raw, rng, precision):
+    """Ranges that end inside a stage, and the launch that adds to what C holds: float64 of the same operands (bf16
+    values, so that both precisions form the same products) within a rounding per addition."""
+    bf = lambda *s: bf16_round(rng.standard_normal(s).astype(np.float32))[0]
+    shapes = [(37, 70, 5, 33), (130, 64, 131, 97), (129, 257, 64, 1), (5, 3, 1, 0)]
+    problems = [(bf(k, m), bf(k, n), bf(k2, m) if k2 and precision < 5 else None, bf(k2, n) if k2 and precision < 5 else None) for m, n, k, k2 in shapes]
+    lib, start = raw[0], 3.0 if precision >= 5 else 0.0
+    got = _grouped_products(hip, raw, problems, precision, lib.nchip_gemm_grouped_tiles64 if precision >= 5 else lib.nchip_gemm_grouped_tiles, 0, 1, 3.0)
+    for (a, b, a2, b2), c in zip(problems, got):
+        a, b = (np.concatenate([x] if y is None else [x, y]).astype(np.float64) for x, y in ((a, a2), (b, b2)))
+        assert np.all(np.abs(c - (0.5 * b.T @ a + start)) <= 2.0 ** -24 * (len(a) + 2) * (np.abs(b).T @ np.abs(a) + start))
