@@ -231,8 +231,10 @@ void nchip_gemm_force_band(int gm);
    products first write bf16 copies of both operands to a scratch buffer (one
    streaming pass each) and the tiles load those, half the bytes; 2 = every
    unbatched bf16 product takes that route (testing aid).  The rounded values
-   and the accumulation order are the same on both routes.  The environment
-   variable NCHIP_GEMM_BF16SRC sets the initial value. */
+   are the same on both routes; an element is one chain over k or two (see
+   nchip_gemm_two_chains): two from copies below 512 tiles of 128x128, in the tile
+   loader in the 64x64 class.  The environment variable NCHIP_GEMM_BF16SRC sets
+   the initial value. */
 void nchip_gemm_bf16_source(int mode);
 
 /* Chooses ksplit for nchip_gemm from the shape alone (never from data). */

@@ -490,8 +490,9 @@ def test_tile_products_at_any_alignment(hip, cfg, precision, ta, tb, m, n, k):
 @pytest.mark.parametrize("m,k,first,second", [(37, 21, 5, 3), (130, 70, 33, 31), (129, 131, 257, 65), (64, 128, 100, 320), (132, 36, 32, 1)])
 @pytest.mark.parametrize("bf16", [0, 1])
 def test_postponed_gradient_of_a_weight_used_over_two_widths(hip, pkg, m, k, first, second, bf16):
-    """One problem of the grouped launch with two ranges of columns, neither a multiple of a stage.  Inputs
-    are bf16 values; bound: a rounding per addition."""
+    """A weight used over two ranges of columns: one problem of the grouped launch where the range reached first
+    (the later term's) is a multiple of 64, else two products.  Inputs are bf16 values; bound: a rounding per
+    addition."""
     B, rng = pkg.binding, np.random.default_rng(m + first)
     bf = lambda *s: (rng.standard_normal(s).astype(np.float32).view(np.uint32) & 0xffff0000).view(np.float32)
     xs, gs = [bf(c, k) for c in (first, second)], [bf(c, m) for c in (first, second)]
