@@ -101,9 +101,9 @@ typedef struct {
 int nchip_gemm_grouped_tiles(int m, int n);
 int nchip_gemm_grouped_tiles256(int m, int n); /* the same for precision 3 */
 int nchip_gemm_grouped_tiles64(int m, int n);  /* and for precisions 5 and 6 */
-/* whether nchip_gemm (precision 0 or 1, ksplit 1, no forced class) sums an element of this product in two
-   chains over k, k % 32 below 16 and from 16 on, rather than in one */
-int nchip_gemm_two_chains(int m, int n, int k, int precision);
+/* whether nchip_gemm (precision 0 or 1, ksplit 1, no forced class) forms this product in the 64x64 class, whose
+   elements are two chains over k, k % 32 below 16 and from 16 on, from its fp32 operands */
+int nchip_gemm_is_64x64(int m, int n, int k, int precision);
 /* precision 0: fp32; 1: fp32 operands rounded to bf16 in the tile loader (any k and k2 both); 2: the operand
    pointers of the table address bf16 copies (2 bytes per element, same layout and leading
    dimensions as the fp32 matrices they were rounded from), read with unguarded 16-byte
@@ -231,9 +231,8 @@ void nchip_gemm_force_band(int gm);
    products first write bf16 copies of both operands to a scratch buffer (one
    streaming pass each) and the tiles load those, half the bytes; 2 = every
    unbatched bf16 product takes that route (testing aid).  The rounded values
-   are the same on both routes; an element is one chain over k or two (see
-   nchip_gemm_two_chains): two from copies below 512 tiles of 128x128, in the tile
-   loader in the 64x64 class.  The environment variable NCHIP_GEMM_BF16SRC sets
+   are the same on both routes; an element is one chain over k or two, two from
+   copies below 512 tiles of 128x128 and, in the tile loader, in the 64x64 class.  The environment variable NCHIP_GEMM_BF16SRC sets
    the initial value. */
 void nchip_gemm_bf16_source(int mode);
 

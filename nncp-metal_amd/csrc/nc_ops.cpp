@@ -793,7 +793,7 @@ static void matmul_bw(NCNode *nd, NCTensor *g, NCTensor **ga, int ia, int ib)
             open_entry->own = open_entry->k % 64 != 0;
             if (open_entry->own && !(alpha == 1.0f && !fits_bf16_operands(m, false, true, s.m, s.k, s.n) &&
                                      nchip_gemm_pick_ksplit((int)s.m, (int)s.k, (int)s.n, 1) == 1 &&
-                                     nchip_gemm_two_chains((int)s.m, (int)s.k, (int)s.n, m->matmul_bf16)))
+                                     nchip_gemm_is_64x64((int)s.m, (int)s.k, (int)s.n, m->matmul_bf16)))
                 open_entry->part = da;
             else
                 nc_free_tensor(da);
