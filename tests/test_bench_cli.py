@@ -58,3 +58,6 @@ def test_traffic_is_read_from_the_committed_counter_summary(tmp_path, monkeypatc
     # the summary the repository holds covers the kernel the bench line names
     monkeypatch.undo()
     assert bench.measured_traffic("gemm_kernel<128,128,32,4,2,0,1,0>", "fp32")[0] > 1e9
+    # (fp32 and bf16: the dominant kernels of the default line, and the grouped launch in its other tiles above)
+    assert bench.measured_traffic("gemm_dma_kernel<1,128,128,4,2,1,4,0,1,grouped>", "fp32")[0] > 1e9
+    assert bench.measured_traffic("gemm_dma_kernel<0,64,64,2,2,1,4,1,0>", "bf16")[0] > 1e7
